@@ -49,7 +49,7 @@ __device__ __forceinline__ float div_y(float x, float d, float y)
 // every step equals, scaled by a power of two, the same step on the
 // operands' significands.  The device check covers the reciprocal's scaling
 // over d's exponents FDIV_E_LO..FDIV_E_HI.
-constexpr int FDIV_E_LO = -60, FDIV_E_HI = 40;
+constexpr int FDIV_E_LO = -60, FDIV_E_HI = 60;
 constexpr float FDIV_D_LO = 0x1p-60f, FDIV_D_HI = 0x1p40f;
 constexpr float FDIV_X_LO = 0x1p-78f, FDIV_X_HI = 0x1p64f;
 

@@ -86,19 +86,8 @@ __device__ __forceinline__ uint32_t ld_raw(const void *p, size_t i, int kind)
     return ((gcu32 *)p)[kind == ICAR_ADV_STORE_F32 ? i : (i >> 1)];
 }
 
-// the value of element i from the word ld_raw returned for it, with a branch
-// on the kind: fewer live registers where the kind is the same for the block
-__device__ __forceinline__ float cvt_q_uniform(uint32_t w, size_t i, int kind, float scale)
-{
-    if (kind == ICAR_ADV_STORE_F32) return __uint_as_float(w);
-    const uint32_t raw = (i & 1) ? (w >> 16) : (w & 0xFFFFu);
-    const float v = is_bf16(kind) ? __uint_as_float(raw << 16)
-                                  : __half2float(__ushort_as_half((uint16_t)raw));
-    return v * scale;
-}
-
-// the same without a branch: both 16-bit forms are decoded and the kind
-// selects, so that no conversion waits on a branch while loads are in flight
+// the value of element i from the word ld_raw returned for it, without a
+// branch: both 16-bit forms are decoded and the kind selects, so that no conversion waits on a branch while loads are in flight
 __device__ __forceinline__ float cvt_q(uint32_t w, size_t i, int kind, float scale)
 {
     const uint32_t raw = (i & 1) ? (w >> 16) : (w & 0xFFFFu);
@@ -211,15 +200,6 @@ __device__ __forceinline__ float cv_w(uint32_t w, size_t i, int kind, float scal
     return cvt_q(w, i, kind, scale);
 }
 
-// the same where the kind is uniform for the block (any kind: a branch, not a
-// select)
-template <int QK>
-__device__ __forceinline__ float cv_w_uniform(uint32_t w, size_t i, int kind, float scale)
-{
-    if (QK == QK_ANY) return cvt_q_uniform(w, i, kind, scale);
-    return cv_w<QK>(w, i, kind, scale);
-}
-
 template <int QK>
 __device__ __forceinline__ void st_w(void *p, size_t i, int kind, float inv_scale, float v,
                                      uint32_t rnd)
@@ -236,8 +216,14 @@ __device__ __forceinline__ void st_w(void *p, size_t i, int kind, float inv_scal
     }
 }
 
-__device__ __forceinline__ float max3(float a, float b, float c) { return fmaxf(fmaxf(a, b), c); }
-__device__ __forceinline__ float min3(float a, float b, float c) { return fminf(fminf(a, b), c); }
+// the stored bits of a value at a 16-bit kind of the class
+template <int QK>
+__device__ __forceinline__ uint16_t q16_of(float v, int kind, float inv_scale, uint32_t rnd)
+{
+    if (QK == QK_BF16) return bf16_of(v * inv_scale, kind == ICAR_ADV_STORE_BF16_SR, rnd);
+    return to16(v, kind, inv_scale, rnd);
+}
+
 
 // One pass of one species: where to read q0 (and q1) and where to write.
 struct SpecPass {
@@ -264,7 +250,8 @@ struct DomDesc {
     DomainFields f;       // raw inputs
     StepFields sf;        // Courant numbers and products (written by k_courant_b)
     float *coef;          // face coefficients (float4 groups)
-    unsigned *step;       // steps taken (drives the stochastic rounding)
+    unsigned *step;       // [0] steps taken (drives the stochastic rounding); [1] a coefficient
+                          // is out of the bounds of the fast quotients (k_coef)
     const SpecPass *pass[MAXP];  // species table of pass p at index p-1
 };
 
@@ -312,6 +299,7 @@ __global__ void __launch_bounds__(256) k_courant_b(const DomDesc *__restrict__ D
     int i, k, j;
     cell_of(D, blockIdx.x, i, k, j);
     const Dims d = D.d;
+    if (blockIdx.x == D.cb0 && threadIdx.x + threadIdx.y == 0) D.step[1] = 0u;
     if (i >= d.nx || j >= d.ny) return;
     gcfloat *__restrict__ den = gp(D.f.density), *__restrict__ fu = gp(D.f.u);
     gcfloat *__restrict__ fv = gp(D.f.v), *__restrict__ fw = gp(D.f.w);
@@ -413,6 +401,17 @@ __global__ void __launch_bounds__(256) k_coef(const DomDesc *__restrict__ DD, in
         if (j >= 1 && j <= ny - 2)
             v[CZV] = 0.5f * Wc * ((1.0f / 4.0f) * (V[c] + V[c + sk] + V[c + sj] + V[c + sk + sj]));
     }
+    // outside the bounds the corrective kernel's quotients are proven for
+    // (k_corr), it takes the IEEE division for the whole domain
+    auto within = [](float c0, float c1, float c2, float sg) {
+        return fabsf(c0) <= 16.0f && sg >= 0x1p-30f && sg <= 0x1p30f && fabsf(c1) <= 16.0f * sg &&
+               fabsf(c2) <= 16.0f * sg;
+    };
+    bool ok = true;
+    if (i >= 1) ok = ok && within(v[CUX], v[CXV], v[CXW], v[SGX]);
+    if (j >= 1) ok = ok && within(v[CUY], v[CYU], v[CYW], v[SGY]);
+    if (k <= nz - 2) ok = ok && within(v[CUZ], v[CZU], v[CZV], v[SGZ]) && fabsf(gp(D.f.dz)[c]) <= 0x1p14f;
+    if (!ok) D.step[1] = 1u;
 #pragma unroll
     for (int g = 0; g < 3; g++)
 #pragma unroll
@@ -589,21 +588,19 @@ __global__ void __launch_bounds__(FBX *FBY) k_first(const DomDesc *__restrict__ 
 constexpr int CX = 64;            // staged tile width (one wavefront per row)
 constexpr int CH = 2;             // halo
 constexpr int CTI = CX - 2 * CH;  // 60 output columns
-constexpr int OWN = 2;            // output rows per wave: ly + NW*(rb + t), t = 0, 1
 
-// A corrective tile of TJ output rows (16 or 32): CY = TJ + 4 staged rows,
-// NW = TJ / 2 wavefronts (wave ly stages rows ly, ly + NW, ... and owns two
-// output rows), SR staged-row slots per wave.  Taller tiles recompute fewer
-// halo rows (y faces on CY - 1 rows, y betas on CY - 2) per output row but
-// take twice the LDS (one block of 16 waves per CU instead of two of 8).
+// A corrective tile of TJ output rows (16 or 8): CY = TJ + 4 staged rows, one
+// wave per pair of output rows.  16 rows recompute fewer halo faces (19 y
+// faces per 16 rows against 11 per 8), 8 rows give twice the blocks on a
+// small grid; the autotuner times both.  Wave w stages and owns rows 2 + 2w and 3 + 2w; the
+// four halo rows are staged by waves 0..3, one each (row_extra).
 template <int TJ>
 struct Tile {
     static constexpr int CY = TJ + 2 * CH;
     static constexpr int NW = TJ / 2;
     static constexpr int CNT = 64 * NW;
-    static constexpr int SR = (CY + NW - 1) / NW;
+    static_assert(NW >= 4, "four waves stage the halo rows");
 };
-
 
 // s = RN(a + b) and its rounding error e, a + b = s + e exactly (Knuth's
 // TwoSum; the unit is compiled without contraction)
@@ -639,54 +636,157 @@ __device__ __forceinline__ float divergence_compensated(float q1, float fl, floa
     return u + ((e1 + e2) - (ch + cz));
 }
 
+// Maxima and minima of values that come from memory.  fmaxf on such a value
+// first quiets a possible signalling NaN with an instruction of its own; the
+// hardware's max and min ignore quiet NaNs as fmaxf does.
+__device__ __forceinline__ float vmax(float a, float b)
+{
+    float r;
+    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float vmin(float a, float b)
+{
+    float r;
+    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float vmax3(float a, float b, float c)
+{
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+__device__ __forceinline__ float vmin3(float a, float b, float c)
+{
+    float r;
+    asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+// max(0, a), min(0, a), and min(1, a, b)
+__device__ __forceinline__ float vpos(float a)
+{
+    float r;
+    asm("v_max_f32 %0, 0, %1" : "=v"(r) : "v"(a));
+    return r;
+}
+__device__ __forceinline__ float vneg(float a)
+{
+    float r;
+    asm("v_min_f32 %0, 0, %1" : "=v"(r) : "v"(a));
+    return r;
+}
+__device__ __forceinline__ float vmin1(float a, float b)
+{
+    float r;
+    asm("v_min3_f32 %0, 1.0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
+// the value of the next lane (lane 63: its own) and of the previous lane
+// (lane 0: its own): one move within the wave, no LDS
+__device__ __forceinline__ float lane_next(float v)
+{
+    const int b = __float_as_int(v);
+    return __int_as_float(__builtin_amdgcn_update_dpp(b, b, 0x130, 0xf, 0xf, false));  // wave_shl:1
+}
+__device__ __forceinline__ float lane_prev(float v)
+{
+    const int b = __float_as_int(v);
+    return __int_as_float(__builtin_amdgcn_update_dpp(b, b, 0x138, 0xf, 0xf, false));  // wave_shr:1
+}
+
 // x/d: the IEEE division, or (F) the three-operation quotient of fdiv.hpp
-// with the operands added to the guard g
 template <bool F>
-__device__ __forceinline__ float fdiv(float x, float d, DivGuard &g)
+__device__ __forceinline__ float fdiv(float x, float d)
 {
-    if constexpr (F) {
-        guard_div(g, x, d);
-        return div_y(x, d, recip_nr(d));
-    } else {
-        return x / d;
-    }
+    if constexpr (F) return div_y(x, d, recip_nr(d));
+    else return x / d;
 }
 
-// the same with y = recip_of(d, g) computed once for several numerators
+// the same with y = recip_nr(d) computed once for several numerators
 template <bool F>
-__device__ __forceinline__ float fdiv_y(float x, float d, float y, DivGuard &g)
+__device__ __forceinline__ float fdiv_y(float x, float d, float y)
 {
-    if constexpr (F) {
-        guard_num(g, x);
-        return div_y(x, d, y);
-    } else {
-        return x / d;
-    }
+    if constexpr (F) return div_y(x, d, y);
+    else return x / d;
 }
 
-__device__ __forceinline__ float recip_of(float d, DivGuard &g)
+// A face velocity u limited by the betas of the cells on its positive (p)
+// and negative (m) side (adv_mpdata_FCT_core.f90:103-115): u times the
+// smallest of 1, the receiving cell's beta_in and the giving cell's beta_out.
+// A zero u stays zero whichever pair is taken.
+__device__ __forceinline__ float limit_u(float u, bool up, float bi_p, float bo_p, float bi_m,
+                                         float bo_m)
 {
-    guard_den(g, d);
-    return recip_nr(d);
+    return vmin1(up ? bi_p : bi_m, up ? bo_m : bo_p) * u;
 }
 
-// WPE: waves per SIMD the register allocation targets (2 blocks of 8 waves
-// per CU need 4); PF: load this iteration's coefficients before the first
-// barrier (latency hidden by the barrier) or at their use; FD: the
-// three-operation quotient where its operands are in range (fdiv.hpp).
-template <bool FCT, int WPE, bool PF, int QK, bool FD, int TJ>
+// Where the corrective kernel takes the three-operation quotient.
+//
+// Every float is a multiple of the last place of the smallest non-zero float
+// around it, so values that are +0 or in [2^lo, 2^hi] have sums and
+// differences that are 0 or at least 2^(lo-23) (rounding only coarsens the
+// multiples), and the bounds on the numerators and divisors of every quotient
+// of a level follow from the range of the staged q1 and q0 alone, once the
+// coefficients are bounded (k_coef): each staged level is checked as it is
+// staged (two integer extrema per value), and a level's quotients take the
+// fast form if the four levels they read are in one of two ranges of 80
+// binades.  Then, with eps and 1e-15 in the divisors,
+//   - numerators that are sums or differences are 0 or >= 2^-99 (exact
+//     remainders need 2^-101), divisors lie in [2^-50, 2^56], quotients are 0
+//     or >= 2^(lo-23-hi-20) = 2^-123, normal;
+//   - the products in the pseudo-velocities (coefficient times difference or
+//     ratio) may be smaller: their smallest non-zero magnitude is tracked
+//     (1.5 operations per product) and a wave that meets one below 2^-88
+//     computes the phase again with the IEEE division.
+// The two ranges: mixing ratios (8e-24 .. 16 per unit) and temperatures or
+// number concentrations (1e-14 .. 1.7e10).
+struct QRange {
+    uint32_t lo, hi;  // bit patterns
+};
+constexpr QRange QR_SMALL = {(127u - 76u) << 23, (127u + 4u) << 23};
+constexpr QRange QR_LARGE = {(127u - 46u) << 23, (127u + 34u) << 23};
+constexpr uint32_t KEY_MIN = ((127u - 88u) << 24) - 1u;  // nz_key(2^-88)
+
+// WPE: waves per SIMD the register allocation targets; PF: the coefficients
+// of a level are loaded during the previous level's divergence phase, or at
+// the start of the phase that uses them.
+//
+// One block marches a (tile, species) column upwards.  Iteration m holds q1
+// of levels m-3 .. m in LDS and computes
+//   B  the z faces on top of level m-1 and the x/y faces of level m-2
+//   -- barrier
+//   C  the betas: x within the wave's rows (the neighbours' values come by
+//      lane moves, so the x direction is finished here), z within the
+//      thread's column, y to LDS; level m+1 is staged and m+2 prefetched
+//   -- barrier
+//   D  the y fluxes and the divergence of level m-2
+// What bounds it is VALU issue, so the phases do the reference's operations
+// and little else: quotients take 6 operations instead of 11 (3 where the
+// divisor is shared), each limited x and y face is computed once per wave,
+// the bounds use max(q0,q1) and min(q0,q1) staged once per value,
+// out-of-domain rows and lanes hold clamped copies and are computed like the
+// others (their values reach no output, so no phase masks lanes), and every
+// global load is a scalar base plus one 32-bit lane offset.  Two barriers per
+// level: the y velocities are double buffered and the planes a phase writes
+// are those no wave reads before the next barrier.  Measured per launch on
+// 1024 x 1024 x 30, 10 FP32 species: 4.19 ms against 5.80 ms with IEEE
+// quotients, three barriers and the faces limited once per cell; 256 x 64 x
+// 20, one species: 20 against 40 us (half of that from the 60 x 8 tiles).
+template <bool FCT, int WPE, bool PF, int QK, int TJ>
 __global__ void __launch_bounds__(Tile<TJ>::CNT) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
-    k_corr(const DomDesc *__restrict__ DD, int nd, int pass, unsigned nwork)
+    k_corr(const DomDesc *__restrict__ DD, int nd, int pass, unsigned nwork, int fast)
 {
-    constexpr int CY = Tile<TJ>::CY, NW = Tile<TJ>::NW, SR = Tile<TJ>::SR;
+    constexpr int CY = Tile<TJ>::CY;
     // XCD-aware mapping: consecutive work items (the species of one tile)
     // land on the same XCD (blocks are dealt round-robin over 8 XCDs) and
     // share the tile's coefficients in its L2.
     const unsigned nb = gridDim.x;
-    const unsigned w = (blockIdx.x & 7) * (nb >> 3) + (blockIdx.x >> 3);
-    if (w >= nwork) return;
-    const DomDesc &D = DD[find_dom_w(DD, nd, w)];
-    const unsigned lw = w - D.w0;
+    const unsigned wi = (blockIdx.x & 7) * (nb >> 3) + (blockIdx.x >> 3);
+    if (wi >= nwork) return;
+    const DomDesc &D = DD[find_dom_w(DD, nd, wi)];
+    const unsigned lw = wi - D.w0;
     const int s = (int)(lw % (unsigned)D.nspec);
     const unsigned tk = lw / (unsigned)D.nspec;
     const int kc = (int)(tk % (unsigned)D.nks);  // column chunk
@@ -694,500 +794,474 @@ __global__ void __launch_bounds__(Tile<TJ>::CNT) __attribute__((amdgpu_waves_per
     const int tx = tile % D.tiles_x, ty = tile / D.tiles_x;
     const int nx = D.d.nx, ny = D.d.ny, nz = D.d.nz;
     // Levels [k0, k1) of the column are written by this block.  The march
-    // starts three levels below k0 so that the vertical pipeline (q0 of
-    // three levels, the two z faces below, the betas and flux of the level
-    // below) holds the values a march from the ground would hold when it
-    // reaches k0; the warm-up levels are computed but not stored.
+    // starts two levels below k0: the flux through the face under k0 needs
+    // the betas of level k0-1, and these the face under it, so with levels
+    // k0-2 and up the pipeline holds what a march from the ground would hold
+    // when it reaches k0.  The x/y faces below k0 are not computed.
     const int k0 = kc * D.kch;
     const int k1 = min(nz, k0 + D.kch);
-    const int m0 = max(0, k0 - 3);
-    // 32-bit element offsets (the host checks nx*ny*nz < 2^32) so that the
-    // loads use a scalar base and one VGPR offset
-    const unsigned sk = (unsigned)nx, sj = (unsigned)nx * (unsigned)nz;
-    const size_t N = (size_t)nx * ny * nz;
-    // ly is the same for the whole wave: as a scalar, every row offset below
-    // is one too, which keeps the LDS addresses out of the vector registers
-    const int lx = threadIdx.x & 63, ly = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int m0 = max(0, k0 - 2);
+    const size_t sk = (size_t)nx, sj = (size_t)nx * nz;
+    const size_t N = sj * ny;
+    const int lx = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int gi = tx * CTI - CH + lx;
     const int j0 = ty * TJ - CH;  // global row of staged row 0
+    const int r0 = 2 + 2 * w;     // first owned staged row; the second is r0 + 1
+    const bool has_x = w < 4;     // this wave stages a halo row as well
+    const int rx = w < 2 ? w : TJ + w;  // rows 0, 1, TJ+2, TJ+3
+
     SpecPass p = D.pass[pass - 1][s];
     if (QK == QK_F32) p.kind0 = p.kindo = ICAR_ADV_STORE_F32;  // an FP32-only batch: no 16-bit code
     p.kind0 = __builtin_amdgcn_readfirstlane(p.kind0);  // uniform: branches on the kinds are scalar
     p.kindo = __builtin_amdgcn_readfirstlane(p.kindo);
     const bool same = p.q1 == nullptr;
     const unsigned tstep = is_sr(p.kindo) ? *D.step : 0u;
+    const bool dom_ok = fast && D.step[1] == 0u;  // coefficients in range (k_coef)
     const float eps = 1e-10f, eps15 = 1e-15f;
-    gcfloat *__restrict__ Gp = gp(D.sf.G), *__restrict__ Gzp = gp(D.sf.Gz), *__restrict__ dzp = gp(D.f.dz);
-    gcfloat *__restrict__ q1p = gp(p.q1);
-    // three groups of four coefficients per cell (x, y, z faces), one
-    // 128-bit load each
-    gcfloat *__restrict__ gx = gp(D.coef);
-    gcfloat *__restrict__ gy = gx + 4 * N;
-    gcfloat *__restrict__ gz = gx + 8 * N;
 
-    __shared__ float sq1[4][CY][CX];  // q1 at levels m-3..m (ring by level & 3)
-    __shared__ float sq0[3][CY][CX];  // q0 at levels m-2..m (ring by level % 3)
-    __shared__ float sxu[CY][CX], sxf[CY][CX];  // x face left of a column: U2, flux1(U2)
-    __shared__ float syu[CY][CX], syf[CY][CX];  // y face south of a row
-    __shared__ float sbxi[CY][CX], sbxo[CY][CX], sbyi[CY][CX], sbyo[CY][CX];  // FCT betas
+    // Global addresses: the row (clamped to the domain), the level and the
+    // tile's first column are scalar, the lane's clamped column is one offset
+    const int x0 = max(0, tx * CTI - CH);
+    const unsigned lo = (unsigned)(min(max(gi, 0), nx - 1) - x0);
+    auto row_at = [&](int r) -> size_t {  // cell (x0, 0, row r)
+        return (size_t)x0 + sj * (size_t)min(max(j0 + r, 0), ny - 1);
+    };
+    const size_t ra[2] = {row_at(r0), row_at(r0 + 1)};
+    const size_t rax = row_at(has_x ? rx : r0);
+    typedef __attribute__((address_space(1))) const char gcchar;
+    typedef __attribute__((address_space(1))) char gchar;
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(1))) const f4 gcf4;
+    auto ld1 = [&](const float *b, size_t c) -> float {
+        return *(gcfloat *)((gcchar *)(gcfloat *)(b + c) + lo * 4u);
+    };
+    auto ld4 = [&](const float *b, size_t c) -> f4 {
+        return *(gcf4 *)((gcchar *)(gcfloat *)(b + 4 * c) + lo * 16u);
+    };
+    auto ldq = [&](size_t c) -> uint32_t {  // raw bits of q0
+        if (QK == QK_F32 || p.kind0 == ICAR_ADV_STORE_F32)
+            return *(gcu32 *)((gcchar *)(gcfloat *)((const float *)p.q0 + c) + lo * 4u);
+        return *(gcu16 *)((gcchar *)(gcu16 *)((const uint16_t *)p.q0 + c) + lo * 2u);
+    };
+    auto cvq = [&](uint32_t b) -> float {
+        if (QK == QK_F32 || p.kind0 == ICAR_ADV_STORE_F32) return __uint_as_float(b);
+        if (QK == QK_BF16 || is_bf16(p.kind0)) return __uint_as_float(b << 16) * p.scale0;
+        return __half2float(__ushort_as_half((uint16_t)b)) * p.scale0;
+    };
 
-    const bool lane_in = gi >= 0 && gi < nx;
-    const bool lane_out = lx >= CH && lx < CX - CH && lane_in;
-    const int rb = (ly < 2) ? 1 : 0;
-    const int nsr = (ly + NW * (SR - 1) < CY) ? SR : SR - 1;  // staged rows of this wave
+    // LDS planes of CY rows of 64 floats (a wave reads one row, lane i at
+    // word i, so no bank conflicts)
+    constexpr int PL = CY * CX;
+    __shared__ float lds[CX + 4 * PL + 6 * PL + 2 * PL + PL + 2 * PL];
+    __shared__ int out_of[4][2];  // level & 3: a value outside QR_SMALL / QR_LARGE
+    float *const Q = lds + CX;    // q1, ring by level & 3 (CX floats below it: lane -1 of row 0)
+    float *const MX = Q + 4 * PL;   // max(q0, q1), ring by level % 3
+    float *const MN = MX + 3 * PL;  // min(q0, q1)
+    float *const VU = MN + 3 * PL;  // y face south of a row: its velocity, double buffered
+    float *const VF = VU + 2 * PL;  //   and its donor flux
+    float *const BI = VF + PL, *const BO = BI + PL;  // y betas
 
-    bool row_in[SR];
-    unsigned rowbase[SR];  // gi + sj*gj (the level offset is added per use)
+    const int own = r0 * CX + lx, ext = rx * CX + lx;
+    const bool lane_out = lx >= CH && lx < CX - CH && gi < nx;  // gi >= 0 there
+    const int gj0 = j0 + r0;
+    const bool edge_x = tx == 0 || tx == D.tiles_x - 1 || tx * CTI + CTI + 1 >= nx - 1;
+    const bool at_w = gi == 0, at_e = gi == nx - 1;
+
+    // z pipeline of the two owned columns
+    float wu2[2], wu1[2], fz2[2], fz1[2];  // unlimited w and its flux on faces m-2, m-1
+    float bzi[2], bzo[2];                  // betas of the cell below the current one
+    float Fzp[2];                          // flux on the face below the output level
 #pragma unroll
-    for (int r = 0; r < SR; r++) {
-        const int gj = j0 + ly + NW * r;
-        row_in[r] = r < nsr && lane_in && gj >= 0 && gj < ny;
-        rowbase[r] = row_in[r] ? (unsigned)gi + sj * (unsigned)gj : 0u;
-    }
-    // the owned rows rb, rb+1 with static indices (rb is 0 or 1), so that no
-    // per-lane array is indexed at run time
-    bool own_in[OWN];
-    unsigned own_base[OWN];
-#pragma unroll
-    for (int t = 0; t < OWN; t++) {
-        own_in[t] = rb ? row_in[t + 1] : row_in[t];
-        own_base[t] = rb ? rowbase[t + 1] : rowbase[t];
-    }
-
-    // per owned column: z pipeline state
-    float z0a[OWN], z0b[OWN], z0c[OWN];          // q0 at levels m-2, m-1, m
-    float wu2[OWN], wu1[OWN], fz2[OWN], fz1[OWN];  // unlimited w / its flux1 on faces m-2, m-1
-    float bzi[OWN], bzo[OWN];                    // betas of the cell below the current one
-    float Fzp[OWN];                              // flux on the face below the output level
-#pragma unroll
-    for (int t = 0; t < OWN; t++) {
-        z0a[t] = z0b[t] = z0c[t] = 0.0f;
+    for (int t = 0; t < 2; t++) {
         wu2[t] = wu1[t] = fz2[t] = fz1[t] = 0.0f;
         bzi[t] = bzo[t] = 1.0f;
         Fzp[t] = 0.0f;
     }
 
-    // register prefetch of the next staged level: raw bits of q0 and the
-    // FP32 q1 (unless it is q0), used only after the next barrier
-    uint32_t n0r[SR];
-    float n1[SR];
-#pragma unroll
-    for (int r = 0; r < SR; r++) {
-        n0r[r] = 0u;
-        n1[r] = 0.0f;
-        if (row_in[r]) {
-            const unsigned c = rowbase[r] + sk * (unsigned)m0;
-            n0r[r] = ld_w<QK>(p.q0, c, p.kind0);
-            if (!same) n1[r] = q1p[c];
+    uint32_t n0[3];  // the next level to stage: raw q0 and q1
+    float n1[3];
+    float nmx[3], nmn[3];
+    auto prefetch = [&](int m) {
+        if (m < nz) {
+            const size_t c = sk * (size_t)m;
+            n0[0] = ldq(ra[0] + c);
+            n0[1] = ldq(ra[1] + c);
+            if (has_x) n0[2] = ldq(rax + c);
+            if (!same) {
+                n1[0] = ld1(p.q1, ra[0] + c);
+                n1[1] = ld1(p.q1, ra[1] + c);
+                if (has_x) n1[2] = ld1(p.q1, rax + c);
+            }
         }
-    }
+    };
+    // level m into its q1 plane; the bounds' maxima and minima are kept for
+    // stage_bounds, which runs after the barrier that frees their planes
+    auto stage = [&](int m) {
+        if (m >= nz) return;
+        float *const q = Q + (m & 3) * PL;
+        uint32_t klo = 0xffffffffu, khi = 0u;
+#pragma unroll
+        for (int r = 0; r < 3; r++) {
+            if (r == 2 && !has_x) continue;
+            const float a = cvq(n0[r]), b = same ? a : n1[r];
+            q[r < 2 ? own + CX * r : ext] = b;
+            if (FCT) {
+                nmx[r] = vmax(a, b);
+                nmn[r] = vmin(a, b);
+            }
+            // the extremes of both fields, as unsigned bit patterns: -0 and
+            // negative values, infinities and NaN compare above every range,
+            // and +0 (minus 1) never counts as small
+            klo = min(klo, min(__float_as_uint(a) - 1u, __float_as_uint(b) - 1u));
+            khi = max(khi, max(__float_as_uint(a), __float_as_uint(b)));
+        }
+        const bool os = klo < QR_SMALL.lo - 1u || khi > QR_SMALL.hi;
+        const bool ol = klo < QR_LARGE.lo - 1u || khi > QR_LARGE.hi;
+        if (__any(os)) out_of[m & 3][0] = 1;
+        if (__any(ol)) out_of[m & 3][1] = 1;
+    };
+    auto stage_bounds = [&](int m) {
+        if (!FCT || m >= nz) return;
+        const int o = (m % 3) * PL;
+#pragma unroll
+        for (int r = 0; r < 3; r++) {
+            if (r == 2 && !has_x) continue;
+            const int c = o + (r < 2 ? own + CX * r : ext);
+            MX[c] = nmx[r];
+            MN[c] = nmn[r];
+        }
+    };
 
+    f4 kx[2], kz[2], ky[3];
+    float kd[2];
+    // The coefficients of iteration m; a level out of range reads the nearest
+    // one (its values are not used)
+    auto load_coef = [&](int m) {
+        const size_t c2 = sk * (size_t)min(max(m - 2, 0), nz - 1);
+        const size_t c1 = sk * (size_t)max(0, min(m - 1, nz - 2));
+        const float *gx = D.coef, *gy = gx + 4 * N, *gz = gx + 8 * N;
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            kz[t] = ld4(gz, ra[t] + c1);
+            kd[t] = ld1(D.f.dz, ra[t] + c1);
+        }
+#pragma unroll
+        for (int t = 0; t < 2; t++) kx[t] = ld4(gx, ra[t] + c2);
+#pragma unroll
+        for (int t = 0; t < 2; t++) ky[t] = ld4(gy, ra[t] + c2);
+        if (has_x) ky[2] = ld4(gy, rax + c2);
+    };
+
+    if (threadIdx.x < CX) {
+        lds[threadIdx.x] = 0.0f;
+        if (threadIdx.x < 8) out_of[threadIdx.x >> 1][threadIdx.x & 1] = 0;
+    }
+    __syncthreads();
+    prefetch(m0);
+    stage(m0);
+    stage_bounds(m0);
+    prefetch(m0 + 1);
+    if (PF) load_coef(m0);
+    __syncthreads();
+
+    int hs = 0, hl = 0;  // out_of of levels m, m-1, m-2, m-3 in bits 0..3
     for (int m = m0; m <= k1 + 1; m++) {
         const int L1 = m - 1, L2 = m - 2;
-        // ---------------- (A) stage level m, prefetch level m+1 and the
-        //                  coefficients of this iteration
-        float n0[SR];
+        const bool xy = L2 >= k0;  // (L2 < k1 by the loop's end)
+        const bool zf = L1 >= m0 && L1 <= nz - 1;
+        const float *const qm = Q + (m & 3) * PL + own;         // level m
+        const float *const qu = Q + ((m + 3) & 3) * PL + own;   // level m-1 = L1 = L2+1
+        const float *const qc = Q + ((m + 2) & 3) * PL + own;   // level m-2 = L2
+        const float *const qd = Q + ((m + 1) & 3) * PL + own;   // level m-3 = L2-1
+        float *const vu = VU + (m & 1) * PL;
+        if (!PF) load_coef(m);
+        float kg[2], kgz[2];
+        if (xy) {
+            const size_t c2 = sk * (size_t)L2;
 #pragma unroll
-        for (int r = 0; r < SR; r++) {
-            const int row = ly + NW * r;
-            n0[r] = cv_w_uniform<QK>(n0r[r], rowbase[r] + sk * (unsigned)m, p.kind0, p.scale0);
-            if (m < nz && r < nsr) {
-                sq0[m % 3][row][lx] = n0[r];
-                sq1[m & 3][row][lx] = same ? n0[r] : n1[r];
+            for (int t = 0; t < 2; t++) {
+                kg[t] = ld1(D.sf.G, ra[t] + c2);
+                kgz[t] = ld1(D.sf.Gz, ra[t] + c2);
             }
         }
-#pragma unroll
-        for (int t = 0; t < OWN; t++) {  // own column: q0 at levels m-2, m-1, m
-            const float nv = rb ? n0[t + 1] : n0[t];
-            z0a[t] = z0b[t];
-            z0b[t] = z0c[t];
-            z0c[t] = (m < nz) ? nv : 0.0f;
+        hs = (hs << 1) & 15;
+        hl = (hl << 1) & 15;
+        if (m < nz) {
+            hs |= __builtin_amdgcn_readfirstlane(out_of[m & 3][0]);
+            hl |= __builtin_amdgcn_readfirstlane(out_of[m & 3][1]);
         }
-        if (m + 1 < nz) {
-#pragma unroll
-            for (int r = 0; r < SR; r++) {
-                if (row_in[r]) {
-                    const unsigned c = rowbase[r] + sk * (unsigned)(m + 1);
-                    n0r[r] = ld_w<QK>(p.q0, c, p.kind0);
-                    if (!same) n1[r] = q1p[c];
-                }
-            }
-        }
-        // x faces and divergence at L2 (own rows), y faces at L2 (staged
-        // rows), z faces at L1 (own rows)
-        float kx[OWN][4], kz[OWN][5], ky[SR][4], kg[OWN][2];
-        // The loads are unconditional, from a valid cell: a lane outside the
-        // domain reads cell 0 and a level out of range the nearest one.  The
-        // values are used only where the lane and level are in range (the
-        // guards of the phases below), and no defaults are kept per lane.
-        auto load_coef = [&]() {
-            const unsigned l2 = (unsigned)max(L2, 0), l1 = (unsigned)max(0, min(L1, nz - 2));
-#pragma unroll
-            for (int t = 0; t < OWN; t++) {
-                {
-                    const unsigned c = own_base[t] + sk * l2;
-                    gcfloat *v4 = gx + 4 * (size_t)c;
-                    const float4 v = make_float4(v4[0], v4[1], v4[2], v4[3]);
-                    kx[t][0] = v.x;
-                    kx[t][1] = v.y;
-                    kx[t][2] = v.z;
-                    kx[t][3] = v.w;
-                    kg[t][0] = Gp[c];
-                    kg[t][1] = Gzp[c];
-                }
-                {
-                    const unsigned c = own_base[t] + sk * l1;
-                    gcfloat *v4 = gz + 4 * (size_t)c;
-                    const float4 v = make_float4(v4[0], v4[1], v4[2], v4[3]);
-                    kz[t][0] = v.x;
-                    kz[t][1] = v.y;
-                    kz[t][2] = v.z;
-                    kz[t][3] = v.w;
-                    kz[t][4] = dzp[c];
-                }
-            }
-#pragma unroll
-            for (int r = 0; r < SR; r++) {
-                const unsigned c = rowbase[r] + sk * l2;
-                gcfloat *v4 = gy + 4 * (size_t)c;
-                const float4 v = make_float4(v4[0], v4[1], v4[2], v4[3]);
-                ky[r][0] = v.x;
-                ky[r][1] = v.y;
-                ky[r][2] = v.z;
-                ky[r][3] = v.w;
-            }
-        };
-        if (PF) load_coef();
-        __syncthreads();
-        if (!PF) load_coef();
-
-        // Phases B, C and D divide as the reference does, one IEEE quotient
-        // per division.  With FD each quotient is the three-operation one of
-        // fdiv.hpp, which is the same value wherever its operands are in
-        // range; a guard collects the operands of a wave's quotients, and a
-        // wave with an operand out of range computes the phase again with
-        // the IEEE division before anything is written.
-        using fast_t = std::integral_constant<bool, true>;
-        using ieee_t = std::integral_constant<bool, false>;
+        const bool ok = dom_ok && (hs == 0 || hl == 0);
 
         // ---------------- (B) unlimited pseudo-velocities (mpdata_fluxes)
-        // (the x and y faces go to LDS as they are computed: a phase computed
-        // again writes the same places; the z faces are kept until the phase
-        // is accepted, since they shift the column's pipeline)
-        float zw[OWN], zf[OWN];
-        auto phase_b = [&](auto fd_c) -> bool {
+        // A phase computed again writes the same places.
+        float zw[2], zq[2], xu[2], xf[2], yu[3], yf[3];
+        auto phase_b = [&](auto fd_c) -> uint32_t {
             constexpr bool F = decltype(fd_c)::value;
-            DivGuard g;
-            auto dv = [&](float x, float d) { return fdiv<F>(x, d, g); };
+            uint32_t key = 0xffffffffu;
+            // a face's value: its first term and two cross terms (the second
+            // where the face has levels on both sides)
+            auto face = [&](float l, float r, f4 k, float d1, float s1, bool two, float d2,
+                            float s2) -> float {
+                const float x = k.x * (r - l);
+                float val = fdiv<F>(x, r + l + eps);
+                const float y = F ? recip_nr(k.w) : 0.0f;
+                const float x1 = k.y * fdiv<F>(d1, s1 + eps);
+                val = val - fdiv_y<F>(x1, k.w, y);
+                if (F) key = min(key, min(nz_key(x), nz_key(x1)));
+                if (two) {
+                    const float x2 = k.z * fdiv<F>(d2, s2 + eps);
+                    val = val - fdiv_y<F>(x2, k.w, y);
+                    if (F) key = min(key, nz_key(x2));
+                }
+                return val;
+            };
             // z face on top of level L1 for the owned columns (:211-246, :380)
-            if (L1 >= 0 && L1 <= nz - 1) {
-                const bool kz_ok = L1 <= nz - 2;
+            if (zf) {
+                if (L1 <= nz - 2) {
 #pragma unroll
-                for (int t = 0; t < OWN; t++) {
-                    const int row = ly + NW * (rb + t);
-                    const int gj = j0 + row;
-                    float wv = 0.0f, fv = 0.0f;
-                    if (kz_ok && lane_out && own_in[t]) {
-                        const float(*qa)[CX] = sq1[L1 & 3];  // level k
-                        const float(*qb)[CX] = sq1[m & 3];   // level k+1
-                        const float l = qa[row][lx], r = qb[row][lx];
-                        float val = dv(kz[t][0] * (r - l), r + l + eps);
-                        const bool cu = gi >= 1 && gi <= nx - 2, cv = gj >= 1 && gj <= ny - 2;
-                        const float ys = (F && (cu || cv)) ? recip_of(kz[t][3], g) : 0.0f;
-                        if (cu) {  // WxU (:227-233)
-                            const float eq = dv(qb[row][lx + 1] - qa[row][lx - 1] + qa[row][lx + 1] - qb[row][lx - 1],
-                                                qa[row][lx + 1] + qb[row][lx + 1] + qa[row][lx - 1] + qb[row][lx - 1] + eps);
-                            val = val - fdiv_y<F>(kz[t][1] * eq, kz[t][3], ys, g);
-                        }
-                        if (cv) {  // WxV (:238-245)
-                            const float eq = dv(qb[row + 1][lx] - qa[row - 1][lx] + qa[row + 1][lx] - qb[row - 1][lx],
-                                                qa[row + 1][lx] + qb[row - 1][lx] + qb[row + 1][lx] + qa[row - 1][lx] + eps);
-                            val = val - fdiv_y<F>(kz[t][2] * eq, kz[t][3], ys, g);
-                        }
-                        wv = val * 0.5f * kz[t][4];
-                        fv = flux1(l, r, wv);
+                    for (int t = 0; t < 2; t++) {
+                        const float *a = qu + CX * t, *b = qm + CX * t;  // levels k and k+1
+                        const float l = a[0], r = b[0];
+                        // WxU (:227-233), WxV (:238-245)
+                        const float v = face(l, r, kz[t],
+                                             b[1] - a[-1] + a[1] - b[-1], a[1] + b[1] + a[-1] + b[-1], true,
+                                             b[CX] - a[-CX] + a[CX] - b[-CX],
+                                             a[CX] + b[-CX] + b[CX] + a[-CX]);
+                        zw[t] = v * 0.5f * kd[t];
+                        zq[t] = flux1(l, r, zw[t]);
                     }
-                    zw[t] = wv;
-                    zf[t] = fv;
+                } else {
+                    zw[0] = zw[1] = zq[0] = zq[1] = 0.0f;
                 }
             }
-            if (L2 >= 0) {
-                const float(*q1m)[CX] = sq1[L2 & 3];
-                const float(*q1u)[CX] = sq1[(L2 + 1) & 3];
-                const float(*q1d)[CX] = sq1[(L2 + 3) & 3];
+            if (xy) {
                 const bool kin = L2 >= 1 && L2 <= nz - 2;
-                // x faces (left of column gi) on the owned rows, lanes 1..63 (:131-165, :378)
+                // x faces left of the owned rows' cells (:131-165, :378)
 #pragma unroll
-                for (int t = 0; t < OWN; t++) {
-                    const int row = ly + NW * (rb + t);
-                    const int gj = j0 + row;
-                    float uv = 0.0f, fv = 0.0f;
-                    if (lx >= 1 && gi >= 1 && own_in[t]) {
-                        const float r = q1m[row][lx], l = q1m[row][lx - 1];
-                        float val = dv(kx[t][0] * (r - l), r + l + eps);
-                        const bool cv = gj >= 1 && gj <= ny - 2;
-                        const float ys = (F && (cv || kin)) ? recip_of(kx[t][3], g) : 0.0f;
-                        if (cv) {  // UxV (:145-152)
-                            const float eq = dv(q1m[row + 1][lx] - q1m[row - 1][lx] + q1m[row + 1][lx - 1] - q1m[row - 1][lx - 1],
-                                                q1m[row + 1][lx] + q1m[row - 1][lx] + q1m[row + 1][lx - 1] + q1m[row - 1][lx - 1] + eps);
-                            val = val - fdiv_y<F>(kx[t][1] * eq, kx[t][3], ys, g);
-                        }
-                        if (kin) {  // UxW (:157-164)
-                            const float eq = dv(q1u[row][lx] - q1d[row][lx] + q1u[row][lx - 1] - q1d[row][lx - 1],
-                                                q1u[row][lx] + q1d[row][lx] + q1u[row][lx - 1] + q1d[row][lx - 1] + eps);
-                            val = val - fdiv_y<F>(kx[t][2] * eq, kx[t][3], ys, g);
-                        }
-                        uv = val * 0.5f;
-                        fv = flux1(l, r, uv);
+                for (int t = 0; t < 2; t++) {
+                    const float *c = qc + CX * t, *u = qu + CX * t, *d = qd + CX * t;
+                    const float l = c[-1], r = c[0];
+                    // UxV (:145-152), UxW (:157-164)
+                    float d2 = 0.0f, s2 = 0.0f;
+                    if (kin) {
+                        d2 = u[0] - d[0] + u[-1] - d[-1];
+                        s2 = u[0] + d[0] + u[-1] + d[-1];
                     }
-                    sxu[row][lx] = uv;
-                    sxf[row][lx] = fv;
+                    const float v = face(l, r, kx[t],
+                                         c[CX] - c[-CX] + c[CX - 1] - c[-CX - 1],
+                                         c[CX] + c[-CX] + c[CX - 1] + c[-CX - 1], kin, d2, s2);
+                    xu[t] = v * 0.5f;
+                    xf[t] = flux1(l, r, xu[t]);
                 }
-                // y faces (south of row gj) on the staged rows 1..19, lanes 2..61 (:169-205, :379)
+                // y faces south of the owned rows and the halo rows 1, TJ+2
+                // and TJ+3 (:169-205, :379)
 #pragma unroll
-                for (int r4 = 0; r4 < SR; r4++) {
-                    const int row = ly + NW * r4;
-                    if (r4 >= nsr || row < 1) continue;
-                    const int gj = j0 + row;
-                    float vv = 0.0f, fv = 0.0f;
-                    if (lane_out && gj >= 1 && gj <= ny - 1) {
-                        const float r = q1m[row][lx], l = q1m[row - 1][lx];
-                        float val = dv(ky[r4][0] * (r - l), r + l + eps);
-                        const bool cu = gi >= 1 && gi <= nx - 2;
-                        const float ys = (F && (cu || kin)) ? recip_of(ky[r4][3], g) : 0.0f;
-                        if (cu) {  // VxU (:186-192)
-                            const float eq = dv(q1m[row - 1][lx + 1] - q1m[row][lx - 1] + q1m[row][lx + 1] - q1m[row - 1][lx - 1],
-                                                q1m[row][lx + 1] + q1m[row - 1][lx + 1] + q1m[row][lx - 1] + q1m[row - 1][lx - 1] + eps);
-                            val = val - fdiv_y<F>(ky[r4][1] * eq, ky[r4][3], ys, g);
-                        }
-                        if (kin) {  // VxW (:197-204)
-                            const float eq = dv(q1u[row - 1][lx] - q1d[row][lx] + q1u[row][lx] - q1d[row - 1][lx],
-                                                q1u[row - 1][lx] + q1d[row][lx] + q1u[row][lx] + q1d[row - 1][lx] + eps);
-                            val = val - fdiv_y<F>(ky[r4][2] * eq, ky[r4][3], ys, g);
-                        }
-                        vv = val * 0.5f;
-                        fv = flux1(l, r, vv);
+                for (int t = 0; t < 3; t++) {
+                    if (t == 2 && (!has_x || w == 0)) continue;
+                    const int o = t < 2 ? CX * t : ext - own;
+                    const float *c = qc + o, *u = qu + o, *d = qd + o;
+                    const float l = c[-CX], r = c[0];
+                    // VxU (:186-192), VxW (:197-204)
+                    float d2 = 0.0f, s2 = 0.0f;
+                    if (kin) {
+                        d2 = u[-CX] - d[0] + u[0] - d[-CX];
+                        s2 = u[-CX] + d[0] + u[0] + d[-CX];
                     }
-                    syu[row][lx] = vv;
-                    syf[row][lx] = fv;
+                    const float v = face(l, r, ky[t],
+                                         c[1 - CX] - c[-1] + c[1] - c[-CX - 1],
+                                         c[1] + c[1 - CX] + c[-1] + c[-CX - 1], kin, d2, s2);
+                    yu[t] = v * 0.5f;
+                    yf[t] = flux1(l, r, yu[t]);
+                    vu[own + o] = yu[t];
+                    VF[own + o] = yf[t];
                 }
             }
-            return guard_ok(g);
+            return key;
         };
-        if (!FD || __any(!phase_b(fast_t{}))) phase_b(ieee_t{});
-        if (L1 >= 0 && L1 <= nz - 1) {
+        {
+            bool ieee = true;
+            if (ok) ieee = __any(phase_b(std::integral_constant<bool, true>{}) < KEY_MIN);
+            if (ieee) phase_b(std::integral_constant<bool, false>{});
+        }
+        if (zf) {
 #pragma unroll
-            for (int t = 0; t < OWN; t++) {
+            for (int t = 0; t < 2; t++) {
                 wu2[t] = wu1[t];
                 fz2[t] = fz1[t];
                 wu1[t] = zw[t];
-                fz1[t] = zf[t];
+                fz1[t] = zq[t];
             }
         }
         __syncthreads();
 
         // ---------------- (C) FCT: per-cell betas (adv_mpdata_FCT_core.f90:47-116)
-        float Fzc[OWN];  // flux on top of level L2
-#pragma unroll
-        for (int t = 0; t < OWN; t++) Fzc[t] = 0.0f;
+        float Fzc[2] = {0.0f, 0.0f};  // flux on top of level L2
+        float Fxl[2], Fxr[2];  // limited fluxes of the x faces
+        const int o2 = ((L2 + 3) % 3) * PL, o1 = ((L1 + 3) % 3) * PL, om = (m % 3) * PL;
         if (FCT) {
-            float zbi[OWN], zbo[OWN], fzc[OWN];  // the x and y betas go to LDS directly
-            auto phase_c = [&](auto fd_c) -> bool {
+            auto phase_c = [&](auto fd_c) {
                 constexpr bool F = decltype(fd_c)::value;
-                DivGuard g;
-                auto dv = [&](float x, float d) { return fdiv<F>(x, d, g); };
-                if (L2 >= 0) {
-                    const float(*q1m)[CX] = sq1[L2 & 3];
-                    const float(*q0m)[CX] = sq0[L2 % 3];
-                    // x cells of the owned rows, lanes 1..62
+                // the betas of a cell from its bounds and the fluxes of its
+                // two faces in one direction
+                auto betas = [&](float q, float hi, float low, float fin, float fout, float &bi,
+                                 float &bo) {
+                    bi = fdiv<F>(hi - q, fin + eps15);
+                    bo = fdiv<F>(q - low, fout + eps15);
+                };
+                if (xy) {
 #pragma unroll
-                    for (int t = 0; t < OWN; t++) {
-                        const int row = ly + NW * (rb + t);
-                        if (lx >= 1 && lx <= CX - 2 && lane_in) {
-                            float qmax, qmin, fin = 0.0f, fout = 0.0f;
-                            const float qc1 = q1m[row][lx];
-                            if (gi == 0) {
-                                qmax = fmaxf(fmaxf(qc1, q1m[row][lx + 1]), fmaxf(q0m[row][lx], q0m[row][lx + 1]));
-                                qmin = fminf(fminf(qc1, q1m[row][lx + 1]), fminf(q0m[row][lx], q0m[row][lx + 1]));
-                            } else if (gi == nx - 1) {
-                                qmax = max3(q1m[row][lx - 1], qc1, q0m[row][lx - 1]);
-                                qmin = min3(q1m[row][lx - 1], qc1, q0m[row][lx - 1]);
-                            } else {
-                                qmax = fmaxf(max3(q1m[row][lx - 1], qc1, q1m[row][lx + 1]),
-                                             max3(q0m[row][lx - 1], q0m[row][lx], q0m[row][lx + 1]));
-                                qmin = fminf(min3(q1m[row][lx - 1], qc1, q1m[row][lx + 1]),
-                                             min3(q0m[row][lx - 1], q0m[row][lx], q0m[row][lx + 1]));
-                                const float fl = sxf[row][lx], fr = sxf[row][lx + 1];
-                                fin = fmaxf(0.0f, fl) - fminf(0.0f, fr);
-                                fout = fmaxf(0.0f, fr) - fminf(0.0f, fl);
-                            }
-                            sbxi[row][lx] = dv(qmax - qc1, fin + eps15);
-                            sbxo[row][lx] = dv(qc1 - qmin, fout + eps15);
+                    for (int t = 0; t < 2; t++) {
+                        const int c = o2 + own + CX * t;
+                        const float q = qc[CX * t], ql = qc[CX * t - 1];
+                        float xw = MX[c - 1], xc = MX[c], xe = MX[c + 1];
+                        float nw = MN[c - 1], nc = MN[c], ne = MN[c + 1];
+                        const float fl = xf[t], fr = lane_next(fl);
+                        float fin = vpos(fl) - vneg(fr), fout = vpos(fr) - vneg(fl);
+                        if (edge_x) {  // the row's end cells: :50-55, :62-68, :79-83, :95-99
+                            xw = at_w ? xc : xw;
+                            nw = at_w ? nc : nw;
+                            xc = at_e ? q : xc;
+                            nc = at_e ? q : nc;
+                            xe = at_e ? q : xe;
+                            ne = at_e ? q : ne;
+                            fin = at_w || at_e ? 0.0f : fin;
+                            fout = at_w || at_e ? 0.0f : fout;
                         }
+                        float bi, bo;
+                        betas(q, vmax3(xw, xc, xe), vmin3(nw, nc, ne), fin, fout, bi, bo);
+                        const float bil = lane_prev(bi), bol = lane_prev(bo);
+                        const float u = limit_u(xu[t], xu[t] > 0.0f, bi, bo, bil, bol);
+                        Fxl[t] = flux1(ql, q, u);
+                        Fxr[t] = lane_next(Fxl[t]);
                     }
-                    // y cells on the staged rows 1..18, lanes 2..61
+                    // y cells on the owned rows and the halo rows 1 and TJ+2
 #pragma unroll
-                    for (int r4 = 0; r4 < SR; r4++) {
-                        const int row = ly + NW * r4;
-                        if (r4 >= nsr || row < 1 || row > CY - 2) continue;
-                        const int gj = j0 + row;
-                        if (lane_out && gj >= 0 && gj < ny) {
-                            float qmax, qmin, fin = 0.0f, fout = 0.0f;
-                            const float qc1 = q1m[row][lx];
-                            if (gj == 0) {
-                                qmax = fmaxf(fmaxf(qc1, q1m[row + 1][lx]), fmaxf(q0m[row][lx], q0m[row + 1][lx]));
-                                qmin = fminf(fminf(qc1, q1m[row + 1][lx]), fminf(q0m[row][lx], q0m[row + 1][lx]));
-                            } else if (gj == ny - 1) {
-                                qmax = max3(q1m[row - 1][lx], qc1, q0m[row - 1][lx]);
-                                qmin = min3(q1m[row - 1][lx], qc1, q0m[row - 1][lx]);
-                            } else {
-                                qmax = fmaxf(max3(q1m[row - 1][lx], qc1, q1m[row + 1][lx]),
-                                             max3(q0m[row - 1][lx], q0m[row][lx], q0m[row + 1][lx]));
-                                qmin = fminf(min3(q1m[row - 1][lx], qc1, q1m[row + 1][lx]),
-                                             min3(q0m[row - 1][lx], q0m[row][lx], q0m[row + 1][lx]));
-                                const float fs = syf[row][lx], fn = syf[row + 1][lx];
-                                fin = fmaxf(0.0f, fs) - fminf(0.0f, fn);
-                                fout = fmaxf(0.0f, fn) - fminf(0.0f, fs);
-                            }
-                            sbyi[row][lx] = dv(qmax - qc1, fin + eps15);
-                            sbyo[row][lx] = dv(qc1 - qmin, fout + eps15);
+                    for (int t = 0; t < 3; t++) {
+                        if (t == 2 && !(w == 1 || w == 2)) continue;
+                        const int o = t < 2 ? CX * t : ext - own;
+                        const int c = o2 + own + o, gj = t < 2 ? gj0 + t : j0 + rx;
+                        const float q = qc[o];
+                        float hi, low, fin, fout;
+                        if (gj <= 0) {
+                            hi = vmax(MX[c], MX[c + CX]);
+                            low = vmin(MN[c], MN[c + CX]);
+                            fin = fout = 0.0f;
+                        } else if (gj >= ny - 1) {
+                            hi = vmax(MX[c - CX], q);
+                            low = vmin(MN[c - CX], q);
+                            fin = fout = 0.0f;
+                        } else {
+                            hi = vmax3(MX[c - CX], MX[c], MX[c + CX]);
+                            low = vmin3(MN[c - CX], MN[c], MN[c + CX]);
+                            const float fs = yf[t], fn = VF[own + o + CX];
+                            fin = vpos(fs) - vneg(fn);
+                            fout = vpos(fn) - vneg(fs);
                         }
+                        float bi, bo;
+                        betas(q, hi, low, fin, fout, bi, bo);
+                        BI[own + o] = bi;
+                        BO[own + o] = bo;
                     }
                 }
                 // z: betas of cell L1 of each owned column, then the limited
                 // velocity and flux on the face between L2 and L1 (flux_is_w ends)
-                if (L1 >= 0 && L1 <= nz - 1) {
+                if (zf) {
 #pragma unroll
-                    for (int t = 0; t < OWN; t++) {
-                        const int row = ly + NW * (rb + t);
-                        const float qc1 = sq1[L1 & 3][row][lx];
-                        float qmax, qmin, fin, fout;
+                    for (int t = 0; t < 2; t++) {
+                        const int c = own + CX * t;
+                        const float q = qu[CX * t];
+                        float hi, low, fin, fout;
                         if (L1 == 0) {
-                            const float qu1 = sq1[m & 3][row][lx];
-                            qmax = fmaxf(fmaxf(qc1, qu1), fmaxf(z0b[t], z0c[t]));
-                            qmin = fminf(fminf(qc1, qu1), fminf(z0b[t], z0c[t]));
-                            fin = 0.0f - fminf(0.0f, fz1[t]);
-                            fout = fmaxf(0.0f, fz1[t]);
+                            hi = vmax(MX[o1 + c], MX[om + c]);
+                            low = vmin(MN[o1 + c], MN[om + c]);
+                            fin = 0.0f - vneg(fz1[t]);
+                            fout = vpos(fz1[t]);
                         } else if (L1 == nz - 1) {
-                            const float qd1 = sq1[L2 & 3][row][lx];
-                            qmax = max3(qd1, qc1, z0a[t]);
-                            qmin = min3(qd1, qc1, z0a[t]);
-                            fin = fmaxf(0.0f, fz2[t]) - fminf(0.0f, fz2[t]);
-                            fout = fmaxf(0.0f, fz2[t]) - fminf(0.0f, fz2[t]);
+                            hi = vmax(MX[o2 + c], q);
+                            low = vmin(MN[o2 + c], q);
+                            fin = vpos(fz2[t]) - vneg(fz2[t]);
+                            fout = fin;
                         } else {
-                            const float qd1 = sq1[L2 & 3][row][lx], qu1 = sq1[m & 3][row][lx];
-                            qmax = fmaxf(max3(qd1, qc1, qu1), max3(z0a[t], z0b[t], z0c[t]));
-                            qmin = fminf(min3(qd1, qc1, qu1), min3(z0a[t], z0b[t], z0c[t]));
-                            fin = fmaxf(0.0f, fz2[t]) - fminf(0.0f, fz1[t]);
-                            fout = fmaxf(0.0f, fz1[t]) - fminf(0.0f, fz2[t]);
+                            hi = vmax3(MX[o2 + c], MX[o1 + c], MX[om + c]);
+                            low = vmin3(MN[o2 + c], MN[o1 + c], MN[om + c]);
+                            fin = vpos(fz2[t]) - vneg(fz1[t]);
+                            fout = vpos(fz1[t]) - vneg(fz2[t]);
                         }
-                        const float bi = dv(qmax - qc1, fin + eps15);
-                        const float bo = dv(qc1 - qmin, fout + eps15);
-                        fzc[t] = 0.0f;
-                        if (L2 >= 0 && L2 <= nz - 2) {
-                            float wl = wu2[t];
-                            if (wl > 0.0f)
-                                wl = fminf(fminf(1.0f, bi), bzo[t]) * wl;
-                            else if (wl < 0.0f)
-                                wl = fminf(fminf(1.0f, bzi[t]), bo) * wl;
-                            fzc[t] = flux1(sq1[L2 & 3][row][lx], qc1, wl);
+                        float bi, bo;
+                        betas(q, hi, low, fin, fout, bi, bo);
+                        if (L2 >= m0) {
+                            const float u = limit_u(wu2[t], wu2[t] > 0.0f, bi, bo, bzi[t], bzo[t]);
+                            Fzc[t] = flux1(qc[CX * t], q, u);
                         }
-                        zbi[t] = bi;
-                        zbo[t] = bo;
+                        bzi[t] = bi;
+                        bzo[t] = bo;
                     }
                 }
-                return guard_ok(g);
             };
-            if (!FD || __any(!phase_c(fast_t{}))) phase_c(ieee_t{});
-            if (L1 >= 0 && L1 <= nz - 1) {
-#pragma unroll
-                for (int t = 0; t < OWN; t++) {
-                    Fzc[t] = fzc[t];
-                    bzi[t] = zbi[t];
-                    bzo[t] = zbo[t];
-                }
-            }
+            if (ok) phase_c(std::integral_constant<bool, true>{});
+            else phase_c(std::integral_constant<bool, false>{});
         } else {
 #pragma unroll
-            for (int t = 0; t < OWN; t++) Fzc[t] = (L2 >= 0 && L2 <= nz - 2) ? fz2[t] : 0.0f;
+            for (int t = 0; t < 2; t++) {
+                if (L2 >= m0 && L2 <= nz - 2) Fzc[t] = fz2[t];
+                if (xy) {
+                    Fxl[t] = xf[t];
+                    Fxr[t] = lane_next(xf[t]);
+                }
+            }
         }
+        stage(m + 1);
+        prefetch(m + 2);
         __syncthreads();
 
         // ---------------- (D) flux divergence on level L2 (upwind_advection
-        // :86-97) with the limited velocities of the cell's four side faces;
-        // a face shared by two cells is limited identically by both
-        if (L2 >= 0) {
-            const float(*q1m)[CX] = sq1[L2 & 3];
-            float qn[OWN];
-            auto phase_d = [&](auto fd_c) -> bool {
-                constexpr bool F = decltype(fd_c)::value;
-                DivGuard g;
-                auto dv = [&](float x, float d) { return fdiv<F>(x, d, g); };
+        // :86-97) with the limited velocities of the cell's four side faces
+        if (threadIdx.x < 2) out_of[(m + 2) & 3][threadIdx.x] = 0;
+        stage_bounds(m + 1);
+        if (PF) load_coef(m + 1);
+        if (xy) {
+            // the y faces south of the owned rows and of the row north of them
+            float Fy[3];
+            if (FCT) {
 #pragma unroll
-                for (int t = 0; t < OWN; t++) {
-                    const int row = ly + NW * (rb + t);
-                    const int gj = j0 + row;
-                    qn[t] = 0.0f;
-                    if (lane_out && own_in[t] && L2 >= k0) {
-                        const float qc1 = q1m[row][lx];
-                        float q = qc1;
-                        if (!(gi == 0 || gi == nx - 1 || gj == 0 || gj == ny - 1)) {
-                            float fl, fr, fs, fn;
-                            if (FCT) {
-                                float u = sxu[row][lx];  // face between lx-1 and lx
-                                if (u > 0.0f)
-                                    u = fminf(fminf(1.0f, sbxi[row][lx]), sbxo[row][lx - 1]) * u;
-                                else if (u < 0.0f)
-                                    u = fminf(fminf(1.0f, sbxi[row][lx - 1]), sbxo[row][lx]) * u;
-                                fl = flux1(q1m[row][lx - 1], qc1, u);
-                                u = sxu[row][lx + 1];  // face between lx and lx+1
-                                if (u > 0.0f)
-                                    u = fminf(fminf(1.0f, sbxi[row][lx + 1]), sbxo[row][lx]) * u;
-                                else if (u < 0.0f)
-                                    u = fminf(fminf(1.0f, sbxi[row][lx]), sbxo[row][lx + 1]) * u;
-                                fr = flux1(qc1, q1m[row][lx + 1], u);
-                                float v = syu[row][lx];  // face between row-1 and row
-                                if (v > 0.0f)
-                                    v = fminf(fminf(1.0f, sbyi[row][lx]), sbyo[row - 1][lx]) * v;
-                                else if (v < 0.0f)
-                                    v = fminf(fminf(1.0f, sbyi[row - 1][lx]), sbyo[row][lx]) * v;
-                                fs = flux1(q1m[row - 1][lx], qc1, v);
-                                v = syu[row + 1][lx];  // face between row and row+1
-                                if (v > 0.0f)
-                                    v = fminf(fminf(1.0f, sbyi[row + 1][lx]), sbyo[row][lx]) * v;
-                                else if (v < 0.0f)
-                                    v = fminf(fminf(1.0f, sbyi[row][lx]), sbyo[row + 1][lx]) * v;
-                                fn = flux1(qc1, q1m[row + 1][lx], v);
-                            } else {
-                                fl = sxf[row][lx];
-                                fr = sxf[row][lx + 1];
-                                fs = syf[row][lx];
-                                fn = syf[row + 1][lx];
-                            }
-                            if (D.compensated)
-                                q = divergence_compensated(qc1, fl, fr, fs, fn, Fzc[t], Fzp[t],
-                                                           kg[t][0], kg[t][1]);
-                            else {
-                                q = q - dv((fr - fl) + (fn - fs), kg[t][0]);
-                                q = q - dv(Fzc[t] - Fzp[t], kg[t][1]);
-                            }
-                        }
-                        qn[t] = q;
+                for (int t = 0; t < 3; t++) {
+                    const int c = own + CX * t;
+                    const float v = t < 2 ? yu[t] : vu[c];
+                    const float u = limit_u(v, v > 0.0f, BI[c], BO[c], BI[c - CX], BO[c - CX]);
+                    Fy[t] = flux1(qc[CX * (t - 1)], qc[CX * t], u);
+                }
+            } else {
+                Fy[0] = yf[0];
+                Fy[1] = yf[1];
+                Fy[2] = VF[own + 2 * CX];
+            }
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                const int gj = gj0 + t;
+                float q = qc[CX * t];
+                if (gj > 0 && gj < ny - 1) {  // the ring keeps its values
+                    float v;
+                    if (D.compensated) {
+                        v = divergence_compensated(q, Fxl[t], Fxr[t], Fy[t], Fy[t + 1], Fzc[t], Fzp[t],
+                                                   kg[t], kgz[t]);
+                    } else {
+                        v = q - ((Fxr[t] - Fxl[t]) + (Fy[t + 1] - Fy[t])) / kg[t];
+                        v = v - (Fzc[t] - Fzp[t]) / kgz[t];
                     }
+                    q = at_w || at_e ? q : v;
                 }
-                return guard_ok(g);
-            };
-            if (!FD || __any(!phase_d(fast_t{}))) phase_d(ieee_t{});
-#pragma unroll
-            for (int t = 0; t < OWN; t++) {
-                if (lane_out && own_in[t] && L2 >= k0) {
-                    const unsigned c = own_base[t] + sk * (unsigned)L2;
-                    st_w<QK>(p.out, c, p.kindo, p.inv_scaleo, qn[t],
-                             is_sr(p.kindo) ? sr_bits(c, s, tstep) : 0u);
+                if (lane_out && gj < ny) {  // gj >= 0: owned rows start at the tile's first
+                    const size_t c = ra[t] + sk * (size_t)L2;
+                    const uint32_t rnd = is_sr(p.kindo) ? sr_bits((uint32_t)c + lo, s, tstep) : 0u;
+                    if (QK == QK_F32 || p.kindo == ICAR_ADV_STORE_F32)
+                        *(gfloat *)((gchar *)(gfloat *)((float *)p.out + c) + lo * 4u) = q;
+                    else
+                        *(gu16 *)((gchar *)(gu16 *)((uint16_t *)p.out + c) + lo * 2u) = q16_of<QK>(q, p.kindo, p.inv_scaleo, rnd);
                 }
-                Fzp[t] = Fzc[t];
             }
         }
+#pragma unroll
+        for (int t = 0; t < 2; t++) Fzp[t] = Fzc[t];
     }
 }
 
@@ -1269,7 +1343,7 @@ struct FastState {
     SpecPass *d_tab = nullptr;           // [2 parities][passes][nspec]
     int tab_order = -1;
     size_t tab_cap = 0;
-    unsigned *d_step = nullptr;          // steps taken (stochastic rounding counter)
+    unsigned *d_step = nullptr;          // DomDesc::step
 };
 
 struct FastBatch {
@@ -1390,8 +1464,8 @@ FastState *fast_create(Dims d)
     st->d = d;
     st->N = (size_t)d.nx * d.ny * d.nz;
     if (hipMalloc(&st->coef, (size_t)NCOEF * st->N * sizeof(float)) != hipSuccess ||
-        hipMalloc(&st->d_step, sizeof(unsigned)) != hipSuccess ||
-        hipMemset(st->d_step, 0, sizeof(unsigned)) != hipSuccess) {
+        hipMalloc(&st->d_step, 2 * sizeof(unsigned)) != hipSuccess ||
+        hipMemset(st->d_step, 0, 2 * sizeof(unsigned)) != hipSuccess) {
         fast_destroy(st);
         return nullptr;
     }
@@ -1504,21 +1578,18 @@ int upload_tables(FastBatch *b, std::string *err)
     return 0;
 }
 
-// corr_cfg: bit 0 -> 4 waves per SIMD (else 2), bit 1 -> no prefetch, bit 2 ->
-// 60x32 tiles of 16 waves (which need 4 waves per SIMD: bit 0 is implied)
-template <bool FCT, int QK, bool FD>
+// corr_cfg: bit 1 -> coefficients loaded where they are used, bit 2 -> 60x8
+// tiles of 4 waves (60x16 tiles of 8 waves otherwise)
+template <bool FCT, int QK>
 void launch_corr_t(unsigned nb, hipStream_t s, const DomDesc *D, int n, int pass, unsigned nw,
-                   int cfg)
+                   int cfg, int fast)
 {
-    constexpr unsigned T16 = Tile<16>::CNT, T32 = Tile<32>::CNT;
-    switch (cfg & 7) {
-    case 0: hipLaunchKernelGGL((k_corr<FCT, 2, true, QK, FD, 16>), dim3(nb), dim3(T16), 0, s, D, n, pass, nw); break;
-    case 1: hipLaunchKernelGGL((k_corr<FCT, 4, true, QK, FD, 16>), dim3(nb), dim3(T16), 0, s, D, n, pass, nw); break;
-    case 2: hipLaunchKernelGGL((k_corr<FCT, 2, false, QK, FD, 16>), dim3(nb), dim3(T16), 0, s, D, n, pass, nw); break;
-    case 3: hipLaunchKernelGGL((k_corr<FCT, 4, false, QK, FD, 16>), dim3(nb), dim3(T16), 0, s, D, n, pass, nw); break;
-    case 4:
-    case 5: hipLaunchKernelGGL((k_corr<FCT, 4, true, QK, FD, 32>), dim3(nb), dim3(T32), 0, s, D, n, pass, nw); break;
-    default: hipLaunchKernelGGL((k_corr<FCT, 4, false, QK, FD, 32>), dim3(nb), dim3(T32), 0, s, D, n, pass, nw); break;
+    constexpr unsigned T16 = Tile<16>::CNT, T8 = Tile<8>::CNT;
+    switch (cfg & 6) {
+    case 0: hipLaunchKernelGGL((k_corr<FCT, 4, true, QK, 16>), dim3(nb), dim3(T16), 0, s, D, n, pass, nw, fast); break;
+    case 2: hipLaunchKernelGGL((k_corr<FCT, 4, false, QK, 16>), dim3(nb), dim3(T16), 0, s, D, n, pass, nw, fast); break;
+    case 4: hipLaunchKernelGGL((k_corr<FCT, 4, true, QK, 8>), dim3(nb), dim3(T8), 0, s, D, n, pass, nw, fast); break;
+    default: hipLaunchKernelGGL((k_corr<FCT, 4, false, QK, 8>), dim3(nb), dim3(T8), 0, s, D, n, pass, nw, fast); break;
     }
 }
 
@@ -1528,18 +1599,18 @@ int storage_class(const FastBatch *b)
     return !b->q16 ? QK_F32 : b->f16 ? QK_ANY : QK_BF16;
 }
 
-template <bool FCT, bool FD>
+template <bool FCT>
 void launch_corr_q(const FastBatch *b, unsigned nb, hipStream_t s, const DomDesc *D, int n,
-                   int pass, unsigned nw, int cfg)
+                   int pass, unsigned nw, int cfg, int fast)
 {
     switch (storage_class(b)) {
-    case QK_F32: launch_corr_t<FCT, QK_F32, FD>(nb, s, D, n, pass, nw, cfg); break;
-    case QK_BF16: launch_corr_t<FCT, QK_BF16, FD>(nb, s, D, n, pass, nw, cfg); break;
-    default: launch_corr_t<FCT, QK_ANY, FD>(nb, s, D, n, pass, nw, cfg); break;
+    case QK_F32: launch_corr_t<FCT, QK_F32>(nb, s, D, n, pass, nw, cfg, fast); break;
+    case QK_BF16: launch_corr_t<FCT, QK_BF16>(nb, s, D, n, pass, nw, cfg, fast); break;
+    default: launch_corr_t<FCT, QK_ANY>(nb, s, D, n, pass, nw, cfg, fast); break;
     }
 }
 
-int tile_rows(int cfg) { return (cfg & 4) ? 32 : 16; }
+int tile_rows(int cfg) { return (cfg & 4) ? 8 : 16; }
 
 // ICAR_ADV_FAST_DIV=1 takes the guarded three-operation quotient of fdiv.hpp
 // in the corrective and donor-cell kernels (the same results).  Off by
@@ -1553,18 +1624,24 @@ bool fast_division()
     return on;
 }
 
+// ICAR_ADV_FAST_DIV=0 makes the corrective kernel divide by the IEEE sequence
+// throughout (the same results)
+int corr_fast_division()
+{
+    static const int on = [] {
+        const char *e = getenv("ICAR_ADV_FAST_DIV");
+        return e && *e ? atoi(e) != 0 : 1;
+    }();
+    return on;
+}
+
 void launch_corr(const FastBatch *b, hipStream_t s, const DomDesc *D, int n, int pass, int cfg)
 {
     const unsigned nw = b->total_work;
     const unsigned nb = (nw + 7) / 8 * 8;
-    const bool fd = fast_division();
-    if (b->fct) {
-        if (fd) launch_corr_q<true, true>(b, nb, s, D, n, pass, nw, cfg);
-        else launch_corr_q<true, false>(b, nb, s, D, n, pass, nw, cfg);
-    } else {
-        if (fd) launch_corr_q<false, true>(b, nb, s, D, n, pass, nw, cfg);
-        else launch_corr_q<false, false>(b, nb, s, D, n, pass, nw, cfg);
-    }
+    const int fast = corr_fast_division();
+    if (b->fct) launch_corr_q<true>(b, nb, s, D, n, pass, nw, cfg, fast);
+    else launch_corr_q<false>(b, nb, s, D, n, pass, nw, cfg, fast);
 }
 
 // Tuned configurations by batch shape, shared by every batch of the process.
@@ -1638,7 +1715,7 @@ int fast_batch_tune(FastBatch *b, hipStream_t s, std::string *err)
     // candidates: the tile heights and launch configurations, and column
     // chunks while one chunk per column leaves the GPU with few blocks
     std::vector<int> cfgs = fix_cfg ? std::vector<int>{b->corr_cfg}
-                                    : std::vector<int>{1, 0, 3, 2, 5, 7};
+                                    : std::vector<int>{1, 3, 5, 7};
     const int n = (int)b->doms.size();
     const int par = b->doms[0].st->cur;
     // The timed launches are pass 2, which writes only the FP32 pass buffer
@@ -1667,7 +1744,7 @@ int fast_batch_tune(FastBatch *b, hipStream_t s, std::string *err)
     }
     float best = 1e30f;
     int best_cfg = b->corr_cfg, best_ks = b->nks;
-    for (int tj : {16, 32}) {
+    for (int tj : {16, 8}) {
       std::vector<int> tcfgs;
       for (int cfg : cfgs)
           if (tile_rows(cfg) == tj) tcfgs.push_back(cfg);
