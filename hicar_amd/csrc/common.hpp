@@ -144,29 +144,30 @@ struct StdGeom {
     int its, ite, jts, jte;
     int horder, vorder;
     const float *Um, *Vm, *Wm, *Rj, *Rdj;
+    const unsigned *general;  // non-zero: a wind or divisor is out of the fast quotients' range
 };
 constexpr int STD_MAX_BATCH = 16;
 // Species of one launch: the state the fluxes come from (qin), the base
-// state (qold), the output, and the limiter's work arrays: dumb_q and the
-// (scale_in, scale_out) pair of each cell.
+// state (qold), the output, and the limiter's dumb_q.
 struct StdBatch {
     int n;
     const float *qin[STD_MAX_BATCH];
     const float *qold[STD_MAX_BATCH];
     float *out[STD_MAX_BATCH];
     float *dq[STD_MAX_BATCH];
-    float2 *sc[STD_MAX_BATCH];
 };
 void launch_std_wind(hipStream_t s, Dims d, float dx, float dt, int adv_den,
                      const DomainFields &f, float *Um, float *Vm, float *Wm, float *Rj,
-                     float *Rdj);
+                     float *Rdj, unsigned *general);
 // mode 0: stage; 1: stage and dumb_q; 2: dumb_q only
 void launch_std_stage(hipStream_t s, const StdGeom &g, float t_factor, int mode,
                       const StdBatch &b);
-void launch_std_scale(hipStream_t s, const StdGeom &g, const StdBatch &b);
-void launch_std_final(hipStream_t s, const StdGeom &g, const StdBatch &b);
+// the limiter and the last update
+void launch_std_limit(hipStream_t s, const StdGeom &g, const StdBatch &b);
 // the cells no stage writes: qold into out outside the tile and, with
-// with_dq, into dq outside the tile plus one ring
-void launch_std_ring(hipStream_t s, const StdGeom &g, const StdBatch &b, int with_dq);
+// with_dq, into dq outside the tile plus one ring; clears *reset (not null:
+// the flag a following launch_std_wind may set)
+void launch_std_ring(hipStream_t s, const StdGeom &g, const StdBatch &b, int with_dq,
+                     unsigned *reset);
 
 }  // namespace icaradv
