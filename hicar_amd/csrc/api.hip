@@ -30,6 +30,7 @@
 #include "fast.hpp"
 
 using namespace icaradv;
+static_assert(LIST_MAX == ICAR_ADV_MAX_SPECIES, "species list");
 
 namespace {
 
@@ -395,6 +396,19 @@ void *species_dev(Handle *h, int s)
     return h->sp[s].dev;
 }
 
+// The bound species' current buffers.
+SpeciesList species_list(Handle *h)
+{
+    SpeciesList l;
+    for (int s = 0; s < h->nspecies; s++) {
+        if (!h->sp[s].bound) continue;
+        l.q[l.n] = species_dev(h, s);
+        l.storage[l.n] = h->sp[s].storage;
+        l.esize[l.n++] = h->sp[s].storage == ICAR_ADV_STORE_F32 ? 4 : 2;
+    }
+    return l;
+}
+
 // One species through mpdata_advect3d with the exact kernels.
 int advect_species_exact(Handle *h, float *q)
 {
@@ -489,8 +503,8 @@ int divergence_check(Handle *h)
 }
 
 // adv=1: the standard scheme for every bound species, in batches of up to
-// STD_MAX_BATCH species per launch.
-int advect_std(Handle *h, float dt)
+// STD_MAX_BATCH species per launch.  winds: as do_advect.
+int advect_std(Handle *h, float dt, bool winds)
 {
     const DomainFields f = domain_fields(h);
     const double n = cells(h);
@@ -538,18 +552,16 @@ int advect_std(Handle *h, float dt)
         // output (qfluxes = qold, advect.f90:298), dumb_q outside its ring
         fill(0);
         outs(1);
+        for (int m = 0; m < b.n; m++) b.out2[m] = rk3 ? h->std_b[idx[b0 + m]] : nullptr;
         timed(h, K_STD_RING, 0.0, [&] {
-            launch_std_ring(h->stream, g, b, fc ? 1 : 0, b0 == 0 ? h->std_general : nullptr);
+            launch_std_ring(h->stream, g, b, fc ? 1 : 0,
+                            winds && b0 == 0 ? h->std_general : nullptr);
         });
-        if (b0 == 0)  // after the first ring copy, which clears the flag this may set
+        if (winds && b0 == 0)  // after the first ring copy, which clears the flag this may set
             timed(h, K_STD_WIND, 14.0 * 4 * n, [&] {  // 9 inputs, 5 outputs
                 launch_std_wind(h->stream, h->d, h->g.dx, dt, h->o.advect_density, f, h->Um, h->Vm,
                                 h->Wm, h->Rj, h->Rdj, h->std_general);
             });
-        if (rk3) {
-            outs(2);
-            timed(h, K_STD_RING, 0.0, [&] { launch_std_ring(h->stream, g, b, 0, nullptr); });
-        }
         if (rk3) {  // advection_driver.f90:103-110
             fill(0);
             outs(1);
@@ -613,13 +625,17 @@ void set_parity(Handle *h, int p)
     }
 }
 
-int do_advect(Handle *h, float dt)
+// One step.  winds: form the Courant numbers (mass fluxes) and what follows
+// from them.  They depend on dt, the winds, density and metric only, none of
+// which changes between the steps of one icar_adv_run, so its loop forms them
+// in its first step.
+int do_advect(Handle *h, float dt, bool winds = true)
 {
     int rc = require_bound(h);
     if (rc) return rc;
     h->last_dt = dt;
     h->have_dt = true;
-    if (h->is_std) return advect_std(h, dt);
+    if (h->is_std) return advect_std(h, dt, winds);
     const DomainFields f = domain_fields(h);
     const double n = cells(h);
     if (h->o.kernel_variant == 1 && !h->o.rk3 && h->nspecies > 0 && h->o.mpdata_order >= 1) {
@@ -628,16 +644,18 @@ int do_advect(Handle *h, float dt)
         rc = ensure_batch(h);
         if (rc) return rc;
         std::string e;
-        rc = fast_batch_advect(h->batch, h->stream, &dt, timed_fn(h), &e);
+        rc = fast_batch_advect(h->batch, h->stream, &dt, winds, timed_fn(h), &e);
         if (rc) return set_err(h, rc, "%s", e.c_str());
         HIPCHK(h, hipGetLastError());
         if (h->o.debug) return divergence_check(h);
         return 0;
     }
-    timed(h, K_COURANT, (9 + 6) * 4 * n, [&] {
-        launch_courant(h->stream, h->d, h->g.dx, dt, h->o.advect_density, f, h->sf);
-    });
-    HIPCHK(h, hipGetLastError());
+    if (winds) {
+        timed(h, K_COURANT, (9 + 6) * 4 * n, [&] {
+            launch_courant(h->stream, h->d, h->g.dx, dt, h->o.advect_density, f, h->sf);
+        });
+        HIPCHK(h, hipGetLastError());
+    }
     if (h->o.debug) {
         rc = divergence_check(h);
         if (rc) return rc;
@@ -679,16 +697,7 @@ int apply_bc_on(Handle *h, T *owner, hipStream_t stream, int bc_x, int bc_y)
     if (bc_x < 0 || bc_x > 2 || (bc_y != 0 && bc_y != 2))
         return set_err(h, ICAR_ADV_EINVAL, "bc_x must be 0/1/2 and bc_y 0/2");
     if (bc_x == 0 && bc_y == 0) return 0;
-    for (int s = 0; s < h->nspecies; s++) {
-        SpeciesSlot &sl = h->sp[s];
-        if (!sl.bound) continue;
-        timed(owner, K_BC, 0.0, [&] {
-            if (sl.storage == ICAR_ADV_STORE_F32)
-                launch_bc(stream, h->d, static_cast<float *>(species_dev(h, s)), bc_x, bc_y);
-            else
-                launch_bc16(stream, h->d, species_dev(h, s), bc_x, bc_y);
-        });
-    }
+    timed(owner, K_BC, 0.0, [&] { launch_ring(stream, h->d, species_list(h), bc_x, bc_y); });
     HIPCHK(h, hipGetLastError());
     return 0;
 }
@@ -1708,13 +1717,10 @@ int icar_adv_enforce_limits(void *handle)
     Handle *h;
     int rc = check_handle(handle, &h);
     if (rc) return rc;
-    for (int s = 0; s < h->nspecies; s++) {
-        SpeciesSlot &sl = h->sp[s];
-        if (!sl.bound) continue;
-        const double es = sl.storage == ICAR_ADV_STORE_F32 ? 4.0 : 2.0;
-        timed(h, K_CLAMP, 2.0 * es * cells(h),
-              [&] { launch_clamp(h->stream, h->N, species_dev(h, s), sl.storage); });
-    }
+    const SpeciesList l = species_list(h);
+    double bytes = 0.0;
+    for (int s = 0; s < l.n; s++) bytes += l.esize[s] * cells(h);
+    timed(h, K_CLAMP, bytes, [&] { launch_clamp(h->stream, h->N, l); });
     HIPCHK(h, hipGetLastError());
     return 0;
 }
@@ -1838,9 +1844,9 @@ int icar_adv_run(void *handle, float dt, int nsteps, int bc_x, int bc_y)
         return set_err(h, ICAR_ADV_EINVAL, "bc_x must be 0/1/2 and bc_y 0/2");
     auto steps = [&]() -> int {
         for (int s = 0; s < nsteps; s++) {
-            int r = do_advect(h, dt);
+            int r = do_advect(h, dt, s == 0);
             if (r) return r;
-            if (fused && h->batch) {  // every species' ring conditions in two launches
+            if (fused && h->batch) {  // every species' ring conditions in one launch
                 timed(h, K_BC, 0.0, [&] { r = fast_batch_bc(h->batch, h->stream, bc_x, bc_y); });
                 if (r) return set_err(h, r, "ring conditions: %s", hipGetErrorString((hipError_t)r));
             } else {
@@ -2014,13 +2020,13 @@ int ens_steps(Ensemble *e, const float *dt, int nsteps, int bc_x, int bc_y)
         return ens_err(e, ICAR_ADV_EINVAL, "bc_x must be 0/1/2 and bc_y 0/2");
     for (int st = 0; st < nsteps; st++) {
         std::string m;
-        int rc = fast_batch_advect(e->batch, e->stream, dt, timed_fn(e), &m);
+        int rc = fast_batch_advect(e->batch, e->stream, dt, st == 0, timed_fn(e), &m);
         if (rc) return ens_err(e, rc, "%s", m.c_str());
         for (size_t k = 0; k < e->hs.size(); k++) {
             e->hs[k]->last_dt = dt[k];
             e->hs[k]->have_dt = true;
         }
-        // the ring conditions of every member's species: two launches
+        // the ring conditions of every member's species: one launch
         timed(e, K_BC, 0.0, [&] { rc = fast_batch_bc(e->batch, e->stream, bc_x, bc_y); });
         if (rc) return ens_err(e, rc, "ring conditions: %s", hipGetErrorString((hipError_t)rc));
     }

@@ -89,7 +89,16 @@ void launch_pseudo(hipStream_t s, Dims d, const float *q1, const StepFields &sf,
                    float *u2, float *v2, float *w2);
 void launch_fct(hipStream_t s, Dims d, const float *q0, const float *q1, const float *u2,
                 const float *v2, const float *w2, float *u2l, float *v2l, float *w2l);
-void launch_bc(hipStream_t s, Dims d, float *q, int bc_x, int bc_y);
+// The current buffers of a handle's species and their bytes per element.
+constexpr int LIST_MAX = 48;  // ICAR_ADV_MAX_SPECIES
+struct SpeciesList {
+    int n = 0;
+    void *q[LIST_MAX];
+    int esize[LIST_MAX];
+    int storage[LIST_MAX];
+};
+// Ring conditions of every listed species, in one launch.
+void launch_ring(hipStream_t s, Dims d, const SpeciesList &l, int bc_x, int bc_y);
 // FP64 mass budget partial sums: writes nblocks doubles to partial.
 int mass_partials_blocks(Dims d);
 
@@ -130,8 +139,8 @@ struct HaloStrips {
 };
 // mode 0: a -> buffer; 1: buffer -> b; 2: a -> b
 void launch_strip(hipStream_t s, const HaloStrips &hs, int nz, int mode);
-// enforce_limits on n elements of one species at its storage kind
-void launch_clamp(hipStream_t s, size_t n, void *q, int storage);
+// enforce_limits on the n elements of every listed species, in one launch
+void launch_clamp(hipStream_t s, size_t n, const SpeciesList &l);
 
 // ---- standard scheme, adv=1 (kernels_std.hip) ----
 // Geometry of the flux-form update: the tile (0-based memory offsets), the
@@ -148,12 +157,13 @@ struct StdGeom {
 };
 constexpr int STD_MAX_BATCH = 16;
 // Species of one launch: the state the fluxes come from (qin), the base
-// state (qold), the output, and the limiter's dumb_q.
+// state (qold), the output, and the limiter's dumb_q.  out2: a second buffer
+// the ring copy fills, or null.
 struct StdBatch {
     int n;
     const float *qin[STD_MAX_BATCH];
     const float *qold[STD_MAX_BATCH];
-    float *out[STD_MAX_BATCH];
+    float *out[STD_MAX_BATCH], *out2[STD_MAX_BATCH];
     float *dq[STD_MAX_BATCH];
 };
 void launch_std_wind(hipStream_t s, Dims d, float dx, float dt, int adv_den,
@@ -164,7 +174,7 @@ void launch_std_stage(hipStream_t s, const StdGeom &g, float t_factor, int mode,
                       const StdBatch &b);
 // the limiter and the last update
 void launch_std_limit(hipStream_t s, const StdGeom &g, const StdBatch &b);
-// the cells no stage writes: qold into out outside the tile and, with
+// the cells no stage writes: qold into out (and out2) outside the tile and, with
 // with_dq, into dq outside the tile plus one ring; clears *reset (not null:
 // the flag a following launch_std_wind may set)
 void launch_std_ring(hipStream_t s, const StdGeom &g, const StdBatch &b, int with_dq,

@@ -15,7 +15,7 @@
 //   k_forcing     the boundary-forced branch of apply_forcing
 //                 (src/objects/domain_obj.f90:3493-3503) for one species.
 //   k_strip       the halo strips of the species for the halo exchange.
-//   k_clamp       enforce_limits (domain_obj.f90:3092-3150) for one species.
+//   k_clamp       enforce_limits (domain_obj.f90:3092-3150) for every species.
 // Every expression keeps the Fortran's evaluation order; this unit is
 // compiled with -ffp-contract=off.
 #include "../../include/icar_adv.h"
@@ -281,33 +281,61 @@ namespace {
 // enforce_limits (domain_obj.f90:3092-3150, the data_3d branch): where a
 // species is below zero it becomes zero.  -0.0 and NaN are not below zero
 // and stay.  16-bit storage is judged on its bits: a set sign bit with a
-// non-zero magnitude that is not a NaN.
-__global__ void __launch_bounds__(256)
-    k_clamp(size_t n, void *__restrict__ q, int storage)
+// non-zero magnitude that is not a NaN.  One launch for all species (a block
+// row each), 16 bytes per thread and load, written back only where a value
+// changed: 6 us for a read-only species of 8 M cells against 15 us for a
+// launch per species with 4-byte accesses.
+__device__ __forceinline__ uint32_t below32(uint32_t v)
 {
-    for (size_t p = (size_t)blockIdx.x * 256 + threadIdx.x; p < n; p += (size_t)gridDim.x * 256) {
-        if (storage == ICAR_ADV_STORE_F32) {
-            float *f = static_cast<float *>(q);
-            const float v = f[p];
-            if (v < 0.0f) f[p] = 0.0f;
-        } else {
-            uint16_t *h = static_cast<uint16_t *>(q);
-            const uint16_t v = h[p];
-            const bool bf = storage == ICAR_ADV_STORE_BF16 || storage == ICAR_ADV_STORE_BF16_SR;
-            const uint16_t expm = bf ? 0x7f80u : 0x7c00u, manm = bf ? 0x007fu : 0x03ffu;
-            const bool nan = (v & expm) == expm && (v & manm) != 0;
-            if ((v & 0x8000u) && (v & 0x7fffu) && !nan) h[p] = 0;
-        }
+    return __uint_as_float(v) < 0.0f ? 0u : v;
+}
+
+template <uint32_t EXPM, uint32_t MANM>
+__device__ __forceinline__ uint32_t below16(uint32_t v)
+{
+    const bool nan = (v & EXPM) == EXPM && (v & MANM) != 0;
+    return (v & 0x8000u) && (v & 0x7fffu) && !nan ? 0u : v;
+}
+
+__device__ __forceinline__ uint32_t below_word(uint32_t v, int storage)
+{
+    if (storage == ICAR_ADV_STORE_F32) return below32(v);
+    if (storage == ICAR_ADV_STORE_BF16 || storage == ICAR_ADV_STORE_BF16_SR)
+        return below16<0x7f80u, 0x007fu>(v & 0xffffu) | below16<0x7f80u, 0x007fu>(v >> 16) << 16;
+    return below16<0x7c00u, 0x03ffu>(v & 0xffffu) | below16<0x7c00u, 0x03ffu>(v >> 16) << 16;
+}
+
+__global__ void __launch_bounds__(256) k_clamp(size_t n, SpeciesList l)
+{
+    const int s = blockIdx.y, storage = l.storage[s];
+    uint32_t *q = static_cast<uint32_t *>(l.q[s]);
+    const size_t words = storage == ICAR_ADV_STORE_F32 ? n : n / 2, quads = words / 4;
+    const size_t t0 = (size_t)blockIdx.x * 256 + threadIdx.x, step = (size_t)gridDim.x * 256;
+    uint4 *q4 = reinterpret_cast<uint4 *>(q);  // device allocations are 256-byte aligned
+    for (size_t p = t0; p < quads; p += step) {
+        const uint4 v = q4[p];
+        const uint4 r = make_uint4(below_word(v.x, storage), below_word(v.y, storage),
+                                   below_word(v.z, storage), below_word(v.w, storage));
+        if ((r.x ^ v.x) | (r.y ^ v.y) | (r.z ^ v.z) | (r.w ^ v.w)) q4[p] = r;
+    }
+    for (size_t p = 4 * quads + t0; p < words; p += step) {
+        const uint32_t v = q[p], r = below_word(v, storage);
+        if (r != v) q[p] = r;
+    }
+    if (storage != ICAR_ADV_STORE_F32 && (n & 1) && t0 == 0) {  // the last 16-bit element
+        uint16_t *h = static_cast<uint16_t *>(l.q[s]);
+        h[n - 1] = (uint16_t)below_word(h[n - 1], storage);
     }
 }
 
 }  // namespace
 
-void launch_clamp(hipStream_t s, size_t n, void *q, int storage)
+void launch_clamp(hipStream_t s, size_t n, const SpeciesList &l)
 {
-    size_t blocks = (n + 255) / 256;
-    if (blocks > 65536) blocks = 65536;
-    hipLaunchKernelGGL(k_clamp, dim3((unsigned)blocks), dim3(256), 0, s, n, q, storage);
+    if (l.n == 0) return;
+    size_t blocks = (n / 4 + 255) / 256;
+    blocks = blocks < 1 ? 1 : blocks > 16384 ? 16384 : blocks;
+    hipLaunchKernelGGL(k_clamp, dim3((unsigned)blocks, l.n), dim3(256), 0, s, n, l);
 }
 
 }  // namespace icaradv

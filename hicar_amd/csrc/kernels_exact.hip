@@ -7,6 +7,7 @@
 //
 // Reference: src/physics/adv_mpdata.f90 and adv_mpdata_FCT_core.f90.
 #include "common.hpp"
+#include "ring.hpp"
 
 namespace icaradv {
 
@@ -347,27 +348,13 @@ __global__ void __launch_bounds__(BX *BY)
     }
 }
 
-// Ring boundary conditions (see icar_adv_apply_bc).
-__global__ void k_bc_x(Dims d, float *q, int bc_x)
+// Ring conditions of every species of one domain, a block row per species
+__global__ void __launch_bounds__(256) k_ring(Dims d, SpeciesList l, int bc_x, int bc_y)
 {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = blockIdx.y;
-    if (k >= d.nz || j >= d.ny) return;
-    if (bc_x == 1) {
-        q[ix(d, d.nx - 1, k, j)] = q[ix(d, d.nx - 2, k, j)];
-    } else if (bc_x == 2) {
-        q[ix(d, 0, k, j)] = q[ix(d, d.nx - 2, k, j)];
-        q[ix(d, d.nx - 1, k, j)] = q[ix(d, 1, k, j)];
-    }
-}
-
-__global__ void k_bc_y(Dims d, float *q)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int k = blockIdx.y;
-    if (i >= d.nx || k >= d.nz) return;
-    q[ix(d, i, k, 0)] = q[ix(d, i, k, d.ny - 2)];
-    q[ix(d, i, k, d.ny - 1)] = q[ix(d, i, k, 1)];
+    const unsigned t = blockIdx.x * 256u + threadIdx.x;
+    const int s = blockIdx.y;
+    if (l.esize[s] == 4) ring_cells(static_cast<uint32_t *>(l.q[s]), d, t, bc_x, bc_y);
+    else ring_cells(static_cast<uint16_t *>(l.q[s]), d, t, bc_x, bc_y);
 }
 
 constexpr int RED_THREADS = 256;
@@ -545,12 +532,11 @@ void launch_fct(hipStream_t s, Dims d, const float *q0, const float *q1, const f
                        w2l);
 }
 
-void launch_bc(hipStream_t s, Dims d, float *q, int bc_x, int bc_y)
+void launch_ring(hipStream_t s, Dims d, const SpeciesList &l, int bc_x, int bc_y)
 {
-    if (bc_x == 1 || bc_x == 2)
-        hipLaunchKernelGGL(k_bc_x, dim3((d.nz + 63) / 64, d.ny), dim3(64), 0, s, d, q, bc_x);
-    if (bc_y == 2)
-        hipLaunchKernelGGL(k_bc_y, dim3((d.nx + 255) / 256, d.nz), dim3(256), 0, s, d, q);
+    const unsigned n = ring_x_threads(d, bc_x) + ring_y_threads(d, bc_y);
+    if (n == 0 || l.n == 0) return;
+    hipLaunchKernelGGL(k_ring, dim3(n / 256, l.n), dim3(256), 0, s, d, l, bc_x, bc_y);
 }
 
 int mass_partials_blocks(Dims d) { return red_blocks(d); }

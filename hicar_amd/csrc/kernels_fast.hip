@@ -43,6 +43,7 @@
 #include "../../include/icar_adv.h"
 #include "fast.hpp"
 #include "fdiv.hpp"
+#include "ring.hpp"
 
 namespace icaradv {
 
@@ -1265,57 +1266,23 @@ __global__ void __launch_bounds__(Tile<TJ>::CNT) __attribute__((amdgpu_waves_per
     }
 }
 
-// The same ring conditions for every species of every domain of a batch: one
-// launch for the x sides and one for the y sides (the y sides copy the
-// corners the x sides have written), each over a table of (domain, species)
-// entries with the species' current buffer; a block row per entry.  The
-// conditions copy the stored bits, so one kernel serves every storage kind.
+// The same ring conditions for every species of every domain of a batch, one
+// launch over a table of (domain, species) entries with the species' current
+// buffer; a block row per entry.
 struct BcEntry {
     Dims d;
     void *q;
     int esz;  // bytes per element: 4 (FP32) or 2 (16-bit kinds)
 };
 
-template <typename E>
-__device__ __forceinline__ void bc_x_cells(E *q, const Dims &d, int k, int j, int bc_x)
-{
-    if (bc_x == 1) {
-        q[ix(d, d.nx - 1, k, j)] = q[ix(d, d.nx - 2, k, j)];
-    } else {
-        q[ix(d, 0, k, j)] = q[ix(d, d.nx - 2, k, j)];
-        q[ix(d, d.nx - 1, k, j)] = q[ix(d, 1, k, j)];
-    }
-}
-
-template <typename E>
-__device__ __forceinline__ void bc_y_cells(E *q, const Dims &d, int i, int k)
-{
-    q[ix(d, i, k, 0)] = q[ix(d, i, k, d.ny - 2)];
-    q[ix(d, i, k, d.ny - 1)] = q[ix(d, i, k, 1)];
-}
-
-__global__ void __launch_bounds__(256) k_bc_x_all(const BcEntry *__restrict__ tab, int bc_x)
+__global__ void __launch_bounds__(256)
+    k_bc_all(const BcEntry *__restrict__ tab, int bc_x, int bc_y)
 {
     const BcEntry e = tab[blockIdx.y];
     const unsigned t = blockIdx.x * 256u + threadIdx.x;
-    if (t >= (unsigned)e.d.ny * (unsigned)e.d.nz) return;
-    const int k = (int)(t % (unsigned)e.d.nz), j = (int)(t / (unsigned)e.d.nz);
-    if (e.esz == 4)
-        bc_x_cells(static_cast<uint32_t *>(e.q), e.d, k, j, bc_x);
-    else
-        bc_x_cells(static_cast<uint16_t *>(e.q), e.d, k, j, bc_x);
-}
-
-__global__ void __launch_bounds__(256) k_bc_y_all(const BcEntry *__restrict__ tab)
-{
-    const BcEntry e = tab[blockIdx.y];
-    const unsigned t = blockIdx.x * 256u + threadIdx.x;
-    if (t >= (unsigned)e.d.nx * (unsigned)e.d.nz) return;
-    const int i = (int)(t % (unsigned)e.d.nx), k = (int)(t / (unsigned)e.d.nx);
-    if (e.esz == 4)
-        bc_y_cells(static_cast<uint32_t *>(e.q), e.d, i, k);
-    else
-        bc_y_cells(static_cast<uint16_t *>(e.q), e.d, i, k);
+    if (t >= ring_x_threads(e.d, bc_x) + ring_y_threads(e.d, bc_y)) return;
+    if (e.esz == 4) ring_cells(static_cast<uint32_t *>(e.q), e.d, t, bc_x, bc_y);
+    else ring_cells(static_cast<uint16_t *>(e.q), e.d, t, bc_x, bc_y);
 }
 
 unsigned grid_for(size_t n)
@@ -1364,7 +1331,6 @@ struct FastBatch {
     bool has_sr = false; // a species is stored with stochastic rounding
     BcEntry *d_bc = nullptr;  // ring-condition table: [2 parities][n_bc] (fast_batch_bc)
     int n_bc = 0;
-    unsigned bc_gx = 0, bc_gy = 0;  // blocks per entry for the x and y sides
     bool q16 = false;    // a species is stored in 16 bits
     bool f16 = false;    // a species is stored in FP16 (kernels for any kind)
 };
@@ -1895,8 +1861,6 @@ FastBatch *fast_batch_create(const FastDomain *doms, int n, int order, int fct, 
     for (int k = 0; k < n; k++) {
         FastState *st = doms[k].st;
         const Dims &d = st->d;
-        b->bc_gx = std::max(b->bc_gx, ((unsigned)d.ny * (unsigned)d.nz + 255u) / 256u);
-        b->bc_gy = std::max(b->bc_gy, ((unsigned)d.nx * (unsigned)d.nz + 255u) / 256u);
         for (int s = 0; s < (int)st->sp.size(); s++)
             for (int par = 0; par < 2; par++)
                 bc[par].push_back({d, home(st, s, par), (int)kind_bytes(st->sp[s].storage)});
@@ -1919,9 +1883,10 @@ int fast_batch_bc(const FastBatch *b, hipStream_t s, int bc_x, int bc_y)
 {
     if (b->n_bc == 0 || (bc_x == 0 && bc_y != 2)) return 0;
     const BcEntry *tab = b->d_bc + (size_t)b->doms[0].st->cur * b->n_bc;
-    if (bc_x == 1 || bc_x == 2)
-        hipLaunchKernelGGL(k_bc_x_all, dim3(b->bc_gx, b->n_bc), dim3(256), 0, s, tab, bc_x);
-    if (bc_y == 2) hipLaunchKernelGGL(k_bc_y_all, dim3(b->bc_gy, b->n_bc), dim3(256), 0, s, tab);
+    unsigned n = 0;
+    for (const auto &dm : b->doms)
+        n = std::max(n, ring_x_threads(dm.st->d, bc_x) + ring_y_threads(dm.st->d, bc_y));
+    hipLaunchKernelGGL(k_bc_all, dim3(n / 256, b->n_bc), dim3(256), 0, s, tab, bc_x, bc_y);
     return (int)hipGetLastError();
 }
 
@@ -1958,8 +1923,8 @@ int fast_batch_ready(FastBatch *b, hipStream_t s, const float *dt, std::string *
     return fast_batch_prepare(b, dt, err);
 }
 
-int fast_batch_advect(FastBatch *b, hipStream_t s, const float *dt, const TimedFn &timed,
-                      std::string *err)
+int fast_batch_advect(FastBatch *b, hipStream_t s, const float *dt, bool winds,
+                      const TimedFn &timed, std::string *err)
 {
     int rc = fast_batch_ready(b, s, dt, err);
     if (rc) return rc;
@@ -1972,10 +1937,12 @@ int fast_batch_advect(FastBatch *b, hipStream_t s, const float *dt, const TimedF
         }
     const DomDesc *D = b->d_desc + (size_t)par * n;
     const double cells = b->cells, cs = b->cell_species;
-    // Courant numbers: reads u, v, w, density, jacobians, dz; writes 6 fields
-    timed(K_COURANT, (9.0 + 6.0) * 4 * cells, [&] { launch_courant_b(b, s, D, n); });
-    // species-invariant coefficients: reads U, V, Wd, G; writes NCOEF
-    timed(K_COEF, (4.0 + NCOEF) * 4 * cells, [&] { launch_coef(b, s, D, n); });
+    if (winds) {
+        // Courant numbers: reads u, v, w, density, jacobians, dz; writes 6 fields
+        timed(K_COURANT, (9.0 + 6.0) * 4 * cells, [&] { launch_courant_b(b, s, D, n); });
+        // species-invariant coefficients: reads U, V, Wd, G; writes NCOEF
+        timed(K_COEF, (4.0 + NCOEF) * 4 * cells, [&] { launch_coef(b, s, D, n); });
+    }
     // pass 1: donor cell for every species
     timed(K_FUSED_FIRST, 5.0 * 4 * cells + 2.0 * 4 * cs, [&] { launch_first(b, s, D, n); });
     for (int pass = 2; pass <= b->order; pass++) {
@@ -2014,29 +1981,6 @@ __global__ void k_unpack(size_t n, const uint16_t *__restrict__ src, float *__re
         dst[p] = ld_q(src, p, storage, scale);
 }
 
-__global__ void k_bc16_x(Dims d, uint16_t *q, int bc_x)
-{
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = blockIdx.y;
-    if (k >= d.nz || j >= d.ny) return;
-    if (bc_x == 1) {
-        q[ix(d, d.nx - 1, k, j)] = q[ix(d, d.nx - 2, k, j)];
-    } else if (bc_x == 2) {
-        q[ix(d, 0, k, j)] = q[ix(d, d.nx - 2, k, j)];
-        q[ix(d, d.nx - 1, k, j)] = q[ix(d, 1, k, j)];
-    }
-}
-
-__global__ void k_bc16_y(Dims d, uint16_t *q)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int k = blockIdx.y;
-    if (i >= d.nx || k >= d.nz) return;
-    q[ix(d, i, k, 0)] = q[ix(d, i, k, d.ny - 2)];
-    q[ix(d, i, k, d.ny - 1)] = q[ix(d, i, k, 1)];
-}
-
-
 }  // namespace
 
 void launch_pack(hipStream_t s, size_t n, const float *src, void *dst, int storage, int pow2)
@@ -2049,15 +1993,6 @@ void launch_unpack(hipStream_t s, size_t n, const void *src, float *dst, int sto
 {
     hipLaunchKernelGGL(k_unpack, dim3(grid_for(n)), dim3(256), 0, s, n,
                        static_cast<const uint16_t *>(src), dst, storage, ldexpf(1.0f, pow2));
-}
-
-void launch_bc16(hipStream_t s, Dims d, void *q, int bc_x, int bc_y)
-{
-    uint16_t *p = static_cast<uint16_t *>(q);
-    if (bc_x == 1 || bc_x == 2)
-        hipLaunchKernelGGL(k_bc16_x, dim3((d.nz + 63) / 64, d.ny), dim3(64), 0, s, d, p, bc_x);
-    if (bc_y == 2)
-        hipLaunchKernelGGL(k_bc16_y, dim3((d.nx + 255) / 256, d.nz), dim3(256), 0, s, d, p);
 }
 
 }  // namespace icaradv

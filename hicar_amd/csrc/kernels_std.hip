@@ -1039,6 +1039,7 @@ __global__ void __launch_bounds__(256)
     for (int s = 0; s < b.n; s++) {
         const float v = b.qold[s][c];
         b.out[s][c] = v;
+        if (b.out2[s]) b.out2[s][c] = v;
         if (with_dq && !ext) b.dq[s][c] = v;
     }
 }
