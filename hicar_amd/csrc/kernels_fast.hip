@@ -235,6 +235,33 @@ struct SpecPass {
     float scale0, inv_scaleo;
 };
 
+// The entry in scalar registers: it is the same for every lane of a wave, and
+// known to be it its addresses take no vector registers and branches on the
+// kinds are scalar.
+template <class T>
+__device__ __forceinline__ T uniform_word(T v)
+{
+    constexpr int W = sizeof(T) / 4;
+    static_assert(sizeof(T) == 4 * W, "whole words");
+    int b[W];
+    __builtin_memcpy(b, &v, sizeof(T));
+#pragma unroll
+    for (int e = 0; e < W; e++) b[e] = __builtin_amdgcn_readfirstlane(b[e]);
+    __builtin_memcpy(&v, b, sizeof(T));
+    return v;
+}
+__device__ __forceinline__ SpecPass uniform(SpecPass p)
+{
+    p.q0 = uniform_word(p.q0);
+    p.q1 = uniform_word(p.q1);
+    p.out = uniform_word(p.out);
+    p.kind0 = uniform_word(p.kind0);
+    p.kindo = uniform_word(p.kindo);
+    p.scale0 = uniform_word(p.scale0);
+    p.inv_scaleo = uniform_word(p.inv_scaleo);
+    return p;
+}
+
 // One domain of a batched launch (a single handle, or one member of an
 // ensemble of unevenly sized domains).  Cell kernels cover 64x4-thread
 // blocks of one level; the corrective kernel covers (tile, species) items.
@@ -590,16 +617,21 @@ constexpr int CX = 64;            // staged tile width (one wavefront per row)
 constexpr int CH = 2;             // halo
 constexpr int CTI = CX - 2 * CH;  // 60 output columns
 
-// A corrective tile of TJ output rows (16 or 8): CY = TJ + 4 staged rows, one
-// wave per pair of output rows.  16 rows recompute fewer halo faces (19 y
-// faces per 16 rows against 11 per 8), 8 rows give twice the blocks on a
-// small grid; the autotuner times both.  Wave w stages and owns rows 2 + 2w and 3 + 2w; the
-// four halo rows are staged by waves 0..3, one each (row_extra).
-template <int TJ>
+// A corrective tile of TJ output rows (16 or 8): CY = TJ + 4 staged rows, RW
+// output rows per wave.  16 rows recompute fewer halo faces (19 y faces per 16
+// rows against 11 per 8), 8 rows give twice the blocks on a small grid, and
+// one row per wave (74 registers, six waves per SIMD, against 114 and four)
+// the shortest serial work per level; the autotuner times them.  Measured,
+// 16 rows x 2 / 8 x 2 / 8 x 1: 1024 x 1024 x 30, 10 FP32 species 3.89 / 3.97 /
+// 4.03 ms; 517 x 389 x 40, 7 species 0.89 / 0.83 / 0.82 ms; 256 x 64 x 20, one
+// species 23.1 / 18.8 / 17.3 us.  Wave w stages and owns rows 2 + RW w and up;
+// the four halo rows are staged by waves 0..3, one each.
+template <int TJ, int RW>
 struct Tile {
     static constexpr int CY = TJ + 2 * CH;
-    static constexpr int NW = TJ / 2;
+    static constexpr int NW = TJ / RW;
     static constexpr int CNT = 64 * NW;
+    static constexpr int WPE = RW == 2 ? 4 : 6;
     static_assert(NW >= 4, "four waves stage the halo rows");
 };
 
@@ -684,17 +716,17 @@ __device__ __forceinline__ float vmin1(float a, float b)
     return r;
 }
 
-// the value of the next lane (lane 63: its own) and of the previous lane
-// (lane 0: its own): one move within the wave, no LDS
+// the value of the next lane (lane 63: 0) and of the previous lane (lane 0:
+// 0): one move within the wave, no LDS
 __device__ __forceinline__ float lane_next(float v)
 {
     const int b = __float_as_int(v);
-    return __int_as_float(__builtin_amdgcn_update_dpp(b, b, 0x130, 0xf, 0xf, false));  // wave_shl:1
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, b, 0x130, 0xf, 0xf, true));  // wave_shl:1
 }
 __device__ __forceinline__ float lane_prev(float v)
 {
     const int b = __float_as_int(v);
-    return __int_as_float(__builtin_amdgcn_update_dpp(b, b, 0x138, 0xf, 0xf, false));  // wave_shr:1
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, b, 0x138, 0xf, 0xf, true));  // wave_shr:1
 }
 
 // x/d: the IEEE division, or (F) the three-operation quotient of fdiv.hpp
@@ -750,36 +782,38 @@ constexpr QRange QR_SMALL = {(127u - 76u) << 23, (127u + 4u) << 23};
 constexpr QRange QR_LARGE = {(127u - 46u) << 23, (127u + 34u) << 23};
 constexpr uint32_t KEY_MIN = ((127u - 88u) << 24) - 1u;  // nz_key(2^-88)
 
-// WPE: waves per SIMD the register allocation targets; PF: the coefficients
-// of a level are loaded during the previous level's divergence phase, or at
-// the start of the phase that uses them.
-//
 // One block marches a (tile, species) column upwards.  Iteration m holds q1
 // of levels m-3 .. m in LDS and computes
 //   B  the z faces on top of level m-1 and the x/y faces of level m-2
 //   -- barrier
 //   C  the betas: x within the wave's rows (the neighbours' values come by
 //      lane moves, so the x direction is finished here), z within the
-//      thread's column, y to LDS; level m+1 is staged and m+2 prefetched
+//      thread's column, y to LDS; level m+1 is staged
 //   -- barrier
-//   D  the y fluxes and the divergence of level m-2
-// What bounds it is VALU issue, so the phases do the reference's operations
+//   D  the y fluxes and the divergence of level m-2; level m+2 is prefetched
+// What bounds it is VALU issue (a reciprocal takes four slots of a multiply,
+// maxima, selects and integer operations two), so the phases do the reference's operations
 // and little else: quotients take 6 operations instead of 11 (3 where the
 // divisor is shared), each limited x and y face is computed once per wave,
 // the bounds use max(q0,q1) and min(q0,q1) staged once per value,
 // out-of-domain rows and lanes hold clamped copies and are computed like the
-// others (their values reach no output, so no phase masks lanes), and every
-// global load is a scalar base plus one 32-bit lane offset.  Two barriers per
-// level: the y velocities are double buffered and the planes a phase writes
-// are those no wave reads before the next barrier.  Measured per launch on
-// 1024 x 1024 x 30, 10 FP32 species: 4.19 ms against 5.80 ms with IEEE
-// quotients, three barriers and the faces limited once per cell; 256 x 64 x
-// 20, one species: 20 against 40 us (half of that from the 60 x 8 tiles).
-template <bool FCT, int WPE, bool PF, int QK, int TJ>
-__global__ void __launch_bounds__(Tile<TJ>::CNT) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
+// others (their values reach no output, so no phase masks lanes), levels and
+// tiles away from the domain's edges take phases without their tests, and
+// every global load is a scalar base plus one 32-bit lane offset.  Two
+// barriers per level: the planes a phase writes are those no wave reads
+// before the next barrier.  What only its own thread reads stays out of LDS
+// (12 planes: four 60 x 8 blocks of four waves fit on a CU, with 15 three).
+// Measured per launch: 1024 x 1024 x 30, 10 FP32 species, 5.80 ms with IEEE
+// quotients, three barriers and the faces limited once per cell, 4.10 without
+// those, 3.89 with 12 planes, scalar bases and the phases without tests; 517
+// x 389 x 40, 7 species 1.38, 0.92 and 0.83 ms; 256 x 64 x 20, one species
+// 40, 20 and 17 us.
+template <bool FCT, int RW, int QK, int TJ>
+__global__ void __launch_bounds__((Tile<TJ, RW>::CNT))
+    __attribute__((amdgpu_waves_per_eu(Tile<TJ, RW>::WPE, Tile<TJ, RW>::WPE)))
     k_corr(const DomDesc *__restrict__ DD, int nd, int pass, unsigned nwork, int fast)
 {
-    constexpr int CY = Tile<TJ>::CY;
+    constexpr int CY = Tile<TJ, RW>::CY;
     // XCD-aware mapping: consecutive work items (the species of one tile)
     // land on the same XCD (blocks are dealt round-robin over 8 XCDs) and
     // share the tile's coefficients in its L2.
@@ -807,14 +841,12 @@ __global__ void __launch_bounds__(Tile<TJ>::CNT) __attribute__((amdgpu_waves_per
     const int lx = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int gi = tx * CTI - CH + lx;
     const int j0 = ty * TJ - CH;  // global row of staged row 0
-    const int r0 = 2 + 2 * w;     // first owned staged row; the second is r0 + 1
+    const int r0 = 2 + RW * w;    // first owned staged row
     const bool has_x = w < 4;     // this wave stages a halo row as well
     const int rx = w < 2 ? w : TJ + w;  // rows 0, 1, TJ+2, TJ+3
 
-    SpecPass p = D.pass[pass - 1][s];
+    SpecPass p = uniform(D.pass[pass - 1][s]);
     if (QK == QK_F32) p.kind0 = p.kindo = ICAR_ADV_STORE_F32;  // an FP32-only batch: no 16-bit code
-    p.kind0 = __builtin_amdgcn_readfirstlane(p.kind0);  // uniform: branches on the kinds are scalar
-    p.kindo = __builtin_amdgcn_readfirstlane(p.kindo);
     const bool same = p.q1 == nullptr;
     const unsigned tstep = is_sr(p.kindo) ? *D.step : 0u;
     const bool dom_ok = fast && D.step[1] == 0u;  // coefficients in range (k_coef)
@@ -823,12 +855,17 @@ __global__ void __launch_bounds__(Tile<TJ>::CNT) __attribute__((amdgpu_waves_per
     // Global addresses: the row (clamped to the domain), the level and the
     // tile's first column are scalar, the lane's clamped column is one offset
     const int x0 = max(0, tx * CTI - CH);
-    const unsigned lo = (unsigned)(min(max(gi, 0), nx - 1) - x0);
+    unsigned lo = (unsigned)(min(max(gi, 0), nx - 1) - x0);
+    // an offset of which nothing is known: its multiples are not kept in
+    // registers over the levels, and addresses stay scalar plus offset
+    auto fresh = [&] { asm("" : "+v"(lo)); };
     auto row_at = [&](int r) -> size_t {  // cell (x0, 0, row r)
         return (size_t)x0 + sj * (size_t)min(max(j0 + r, 0), ny - 1);
     };
-    const size_t ra[2] = {row_at(r0), row_at(r0 + 1)};
-    const size_t rax = row_at(has_x ? rx : r0);
+    size_t ra[RW];
+#pragma unroll
+    for (int t = 0; t < RW; t++) ra[t] = row_at(r0 + t);
+    size_t rax = uniform_word(row_at(has_x ? rx : r0));
     typedef __attribute__((address_space(1))) const char gcchar;
     typedef __attribute__((address_space(1))) char gchar;
     typedef float f4 __attribute__((ext_vector_type(4)));
@@ -853,13 +890,13 @@ __global__ void __launch_bounds__(Tile<TJ>::CNT) __attribute__((amdgpu_waves_per
     // LDS planes of CY rows of 64 floats (a wave reads one row, lane i at
     // word i, so no bank conflicts)
     constexpr int PL = CY * CX;
-    __shared__ float lds[CX + 4 * PL + 6 * PL + 2 * PL + PL + 2 * PL];
+    __shared__ float lds[CX + 12 * PL];
     __shared__ int out_of[4][2];  // level & 3: a value outside QR_SMALL / QR_LARGE
     float *const Q = lds + CX;    // q1, ring by level & 3 (CX floats below it: lane -1 of row 0)
-    float *const MX = Q + 4 * PL;   // max(q0, q1), ring by level % 3
-    float *const MN = MX + 3 * PL;  // min(q0, q1)
-    float *const VU = MN + 3 * PL;  // y face south of a row: its velocity, double buffered
-    float *const VF = VU + 2 * PL;  //   and its donor flux
+    float *const MX = Q + 4 * PL;   // max(q0, q1), ring by level & 1
+    float *const MN = MX + 2 * PL;  // min(q0, q1)
+    float *const VU = MN + 2 * PL;  // y face south of a row: its velocity
+    float *const VF = VU + PL;      //   and its donor flux
     float *const BI = VF + PL, *const BO = BI + PL;  // y betas
 
     const int own = r0 * CX + lx, ext = rx * CX + lx;
@@ -867,49 +904,54 @@ __global__ void __launch_bounds__(Tile<TJ>::CNT) __attribute__((amdgpu_waves_per
     const int gj0 = j0 + r0;
     const bool edge_x = tx == 0 || tx == D.tiles_x - 1 || tx * CTI + CTI + 1 >= nx - 1;
     const bool at_w = gi == 0, at_e = gi == nx - 1;
+    // no cell whose betas are used is in the domain's ring of rows or columns
+    const bool inner = !edge_x && j0 >= 0 && j0 + TJ + 2 < ny - 1;
 
     // z pipeline of the two owned columns
-    float wu2[2], wu1[2], fz2[2], fz1[2];  // unlimited w and its flux on faces m-2, m-1
-    float bzi[2], bzo[2];                  // betas of the cell below the current one
-    float Fzp[2];                          // flux on the face below the output level
+    float wu2[RW], wu1[RW], fz2[RW], fz1[RW];  // unlimited w and its flux on faces m-2, m-1
+    float bzi[RW], bzo[RW];                  // betas of the cell below the current one
+    float Fzp[RW];                          // flux on the face below the output level
 #pragma unroll
-    for (int t = 0; t < 2; t++) {
+    for (int t = 0; t < RW; t++) {
         wu2[t] = wu1[t] = fz2[t] = fz1[t] = 0.0f;
         bzi[t] = bzo[t] = 1.0f;
         Fzp[t] = 0.0f;
     }
 
-    uint32_t n0[3];  // the next level to stage: raw q0 and q1
-    float n1[3];
-    float nmx[3], nmn[3];
+    uint32_t n0[RW + 1];  // the next level to stage: raw q0 and q1
+    float n1[RW + 1];
+    float bx[RW + 1], bn[RW + 1];  // max(q0, q1) and min(q0, q1) of the level staged last
     auto prefetch = [&](int m) {
         if (m < nz) {
+            fresh();
             const size_t c = sk * (size_t)m;
-            n0[0] = ldq(ra[0] + c);
-            n0[1] = ldq(ra[1] + c);
-            if (has_x) n0[2] = ldq(rax + c);
+#pragma unroll
+            for (int t = 0; t < RW; t++) n0[t] = ldq(ra[t] + c);
+            if (has_x) {
+                fresh();
+                n0[RW] = ldq(rax + c);
+            }
             if (!same) {
-                n1[0] = ld1(p.q1, ra[0] + c);
-                n1[1] = ld1(p.q1, ra[1] + c);
-                if (has_x) n1[2] = ld1(p.q1, rax + c);
+                fresh();
+#pragma unroll
+                for (int t = 0; t < RW; t++) n1[t] = ld1(p.q1, ra[t] + c);
+                if (has_x) {
+                    fresh();
+                    n1[RW] = ld1(p.q1, rax + c);
+                }
             }
         }
     };
-    // level m into its q1 plane; the bounds' maxima and minima are kept for
-    // stage_bounds, which runs after the barrier that frees their planes
+    // level m into its q1 plane
     auto stage = [&](int m) {
         if (m >= nz) return;
         float *const q = Q + (m & 3) * PL;
         uint32_t klo = 0xffffffffu, khi = 0u;
 #pragma unroll
-        for (int r = 0; r < 3; r++) {
-            if (r == 2 && !has_x) continue;
+        for (int r = 0; r < RW + 1; r++) {
+            if (r == RW && !has_x) continue;
             const float a = cvq(n0[r]), b = same ? a : n1[r];
-            q[r < 2 ? own + CX * r : ext] = b;
-            if (FCT) {
-                nmx[r] = vmax(a, b);
-                nmn[r] = vmin(a, b);
-            }
+            q[r < RW ? own + CX * r : ext] = b;
             // the extremes of both fields, as unsigned bit patterns: -0 and
             // negative values, infinities and NaN compare above every range,
             // and +0 (minus 1) never counts as small
@@ -921,36 +963,53 @@ __global__ void __launch_bounds__(Tile<TJ>::CNT) __attribute__((amdgpu_waves_per
         if (__any(os)) out_of[m & 3][0] = 1;
         if (__any(ol)) out_of[m & 3][1] = 1;
     };
-    auto stage_bounds = [&](int m) {
+    // The maxima and minima of the bounds of the level staged last; they stay
+    // in registers for a level, where only this thread needs them (the z
+    // direction), and then go to their planes, which so hold two levels.
+    auto bounds = [&](int m) {
         if (!FCT || m >= nz) return;
-        const int o = (m % 3) * PL;
 #pragma unroll
-        for (int r = 0; r < 3; r++) {
-            if (r == 2 && !has_x) continue;
-            const int c = o + (r < 2 ? own + CX * r : ext);
-            MX[c] = nmx[r];
-            MN[c] = nmn[r];
+        for (int r = 0; r < RW + 1; r++) {
+            if (r == RW && !has_x) continue;
+            const float a = cvq(n0[r]), b = same ? a : n1[r];
+            bx[r] = vmax(a, b);
+            bn[r] = vmin(a, b);
+        }
+    };
+    auto put_bounds = [&](int m) {
+        if (!FCT || m >= nz) return;
+        const int o = (m & 1) * PL;
+#pragma unroll
+        for (int r = 0; r < RW + 1; r++) {
+            if (r == RW && !has_x) continue;
+            const int c = o + (r < RW ? own + CX * r : ext);
+            MX[c] = bx[r];
+            MN[c] = bn[r];
         }
     };
 
-    f4 kx[2], kz[2], ky[3];
-    float kd[2];
+    f4 kx[RW], kz[RW], ky[RW + 1];
+    float kd[RW];
     // The coefficients of iteration m; a level out of range reads the nearest
     // one (its values are not used)
     auto load_coef = [&](int m) {
+        fresh();
         const size_t c2 = sk * (size_t)min(max(m - 2, 0), nz - 1);
         const size_t c1 = sk * (size_t)max(0, min(m - 1, nz - 2));
         const float *gx = D.coef, *gy = gx + 4 * N, *gz = gx + 8 * N;
 #pragma unroll
-        for (int t = 0; t < 2; t++) {
+        for (int t = 0; t < RW; t++) {
             kz[t] = ld4(gz, ra[t] + c1);
             kd[t] = ld1(D.f.dz, ra[t] + c1);
         }
 #pragma unroll
-        for (int t = 0; t < 2; t++) kx[t] = ld4(gx, ra[t] + c2);
+        for (int t = 0; t < RW; t++) kx[t] = ld4(gx, ra[t] + c2);
 #pragma unroll
-        for (int t = 0; t < 2; t++) ky[t] = ld4(gy, ra[t] + c2);
-        if (has_x) ky[2] = ld4(gy, rax + c2);
+        for (int t = 0; t < RW; t++) ky[t] = ld4(gy, ra[t] + c2);
+        if (has_x) {
+            fresh();
+            ky[RW] = ld4(gy, rax + c2);
+        }
     };
 
     if (threadIdx.x < CX) {
@@ -960,27 +1019,32 @@ __global__ void __launch_bounds__(Tile<TJ>::CNT) __attribute__((amdgpu_waves_per
     __syncthreads();
     prefetch(m0);
     stage(m0);
-    stage_bounds(m0);
+    bounds(m0);
     prefetch(m0 + 1);
-    if (PF) load_coef(m0);
     __syncthreads();
 
+    constexpr std::integral_constant<bool, true> yes;
+    constexpr std::integral_constant<bool, false> no;
     int hs = 0, hl = 0;  // out_of of levels m, m-1, m-2, m-3 in bits 0..3
     for (int m = m0; m <= k1 + 1; m++) {
+#pragma unroll
+        for (int t = 0; t < RW; t++) asm("" : "+s"(ra[t]));
+        asm("" : "+s"(rax));
         const int L1 = m - 1, L2 = m - 2;
         const bool xy = L2 >= k0;  // (L2 < k1 by the loop's end)
         const bool zf = L1 >= m0 && L1 <= nz - 1;
+        const bool mid = L2 >= max(k0, 1) && m < nz;  // no phase meets the ground or the top
         const float *const qm = Q + (m & 3) * PL + own;         // level m
         const float *const qu = Q + ((m + 3) & 3) * PL + own;   // level m-1 = L1 = L2+1
         const float *const qc = Q + ((m + 2) & 3) * PL + own;   // level m-2 = L2
         const float *const qd = Q + ((m + 1) & 3) * PL + own;   // level m-3 = L2-1
-        float *const vu = VU + (m & 1) * PL;
-        if (!PF) load_coef(m);
-        float kg[2], kgz[2];
+        load_coef(m);
+        float kg[RW], kgz[RW];
         if (xy) {
             const size_t c2 = sk * (size_t)L2;
+            fresh();
 #pragma unroll
-            for (int t = 0; t < 2; t++) {
+            for (int t = 0; t < RW; t++) {
                 kg[t] = ld1(D.sf.G, ra[t] + c2);
                 kgz[t] = ld1(D.sf.Gz, ra[t] + c2);
             }
@@ -995,9 +1059,9 @@ __global__ void __launch_bounds__(Tile<TJ>::CNT) __attribute__((amdgpu_waves_per
 
         // ---------------- (B) unlimited pseudo-velocities (mpdata_fluxes)
         // A phase computed again writes the same places.
-        float zw[2], zq[2], xu[2], xf[2], yu[3], yf[3];
-        auto phase_b = [&](auto fd_c) -> uint32_t {
-            constexpr bool F = decltype(fd_c)::value;
+        float zw[RW] = {}, zq[RW] = {}, xu[RW], xf[RW], yu[RW + 1], yf[RW + 1];
+        auto phase_b = [&](auto fd_c, auto mid_c) -> uint32_t {
+            constexpr bool F = decltype(fd_c)::value, M = decltype(mid_c)::value;
             uint32_t key = 0xffffffffu;
             // a face's value: its first term and two cross terms (the second
             // where the face has levels on both sides)
@@ -1017,10 +1081,10 @@ __global__ void __launch_bounds__(Tile<TJ>::CNT) __attribute__((amdgpu_waves_per
                 return val;
             };
             // z face on top of level L1 for the owned columns (:211-246, :380)
-            if (zf) {
-                if (L1 <= nz - 2) {
+            if (M || zf) {
+                if (M || L1 <= nz - 2) {
 #pragma unroll
-                    for (int t = 0; t < 2; t++) {
+                    for (int t = 0; t < RW; t++) {
                         const float *a = qu + CX * t, *b = qm + CX * t;  // levels k and k+1
                         const float l = a[0], r = b[0];
                         // WxU (:227-233), WxV (:238-245)
@@ -1031,15 +1095,13 @@ __global__ void __launch_bounds__(Tile<TJ>::CNT) __attribute__((amdgpu_waves_per
                         zw[t] = v * 0.5f * kd[t];
                         zq[t] = flux1(l, r, zw[t]);
                     }
-                } else {
-                    zw[0] = zw[1] = zq[0] = zq[1] = 0.0f;
                 }
             }
-            if (xy) {
-                const bool kin = L2 >= 1 && L2 <= nz - 2;
+            if (M || xy) {
+                const bool kin = M || (L2 >= 1 && L2 <= nz - 2);
                 // x faces left of the owned rows' cells (:131-165, :378)
 #pragma unroll
-                for (int t = 0; t < 2; t++) {
+                for (int t = 0; t < RW; t++) {
                     const float *c = qc + CX * t, *u = qu + CX * t, *d = qd + CX * t;
                     const float l = c[-1], r = c[0];
                     // UxV (:145-152), UxW (:157-164)
@@ -1057,9 +1119,9 @@ __global__ void __launch_bounds__(Tile<TJ>::CNT) __attribute__((amdgpu_waves_per
                 // y faces south of the owned rows and the halo rows 1, TJ+2
                 // and TJ+3 (:169-205, :379)
 #pragma unroll
-                for (int t = 0; t < 3; t++) {
-                    if (t == 2 && (!has_x || w == 0)) continue;
-                    const int o = t < 2 ? CX * t : ext - own;
+                for (int t = 0; t < RW + 1; t++) {
+                    if (t == RW && (!has_x || w == 0)) continue;
+                    const int o = t < RW ? CX * t : ext - own;
                     const float *c = qc + o, *u = qu + o, *d = qd + o;
                     const float l = c[-CX], r = c[0];
                     // VxU (:186-192), VxW (:197-204)
@@ -1073,7 +1135,7 @@ __global__ void __launch_bounds__(Tile<TJ>::CNT) __attribute__((amdgpu_waves_per
                                          c[1] + c[1 - CX] + c[-1] + c[-CX - 1], kin, d2, s2);
                     yu[t] = v * 0.5f;
                     yf[t] = flux1(l, r, yu[t]);
-                    vu[own + o] = yu[t];
+                    VU[own + o] = yu[t];
                     VF[own + o] = yf[t];
                 }
             }
@@ -1081,12 +1143,15 @@ __global__ void __launch_bounds__(Tile<TJ>::CNT) __attribute__((amdgpu_waves_per
         };
         {
             bool ieee = true;
-            if (ok) ieee = __any(phase_b(std::integral_constant<bool, true>{}) < KEY_MIN);
-            if (ieee) phase_b(std::integral_constant<bool, false>{});
+            if (ok) {
+                const uint32_t key = mid ? phase_b(yes, yes) : phase_b(yes, no);
+                ieee = __any(key < KEY_MIN);
+            }
+            if (ieee) phase_b(no, no);
         }
         if (zf) {
 #pragma unroll
-            for (int t = 0; t < 2; t++) {
+            for (int t = 0; t < RW; t++) {
                 wu2[t] = wu1[t];
                 fz2[t] = fz1[t];
                 wu1[t] = zw[t];
@@ -1096,12 +1161,16 @@ __global__ void __launch_bounds__(Tile<TJ>::CNT) __attribute__((amdgpu_waves_per
         __syncthreads();
 
         // ---------------- (C) FCT: per-cell betas (adv_mpdata_FCT_core.f90:47-116)
-        float Fzc[2] = {0.0f, 0.0f};  // flux on top of level L2
-        float Fxl[2], Fxr[2];  // limited fluxes of the x faces
-        const int o2 = ((L2 + 3) % 3) * PL, o1 = ((L1 + 3) % 3) * PL, om = (m % 3) * PL;
+        float Fzc[RW] = {};  // flux on top of level L2
+        float Fxl[RW], Fxr[RW];  // limited fluxes of the x faces
+        const int o2 = (L2 & 1) * PL, o1 = (L1 & 1) * PL;
+        // the y face south of the row north of the owned ones: its velocity, or
+        // without FCT its flux (read before the barrier: the next level's
+        // phase B overwrites the plane)
+        float yn = 0.0f;
         if (FCT) {
-            auto phase_c = [&](auto fd_c) {
-                constexpr bool F = decltype(fd_c)::value;
+            auto phase_c = [&](auto fd_c, auto mid_c) {
+                constexpr bool F = decltype(fd_c)::value, M = decltype(mid_c)::value;
                 // the betas of a cell from its bounds and the fluxes of its
                 // two faces in one direction
                 auto betas = [&](float q, float hi, float low, float fin, float fout, float &bi,
@@ -1109,16 +1178,16 @@ __global__ void __launch_bounds__(Tile<TJ>::CNT) __attribute__((amdgpu_waves_per
                     bi = fdiv<F>(hi - q, fin + eps15);
                     bo = fdiv<F>(q - low, fout + eps15);
                 };
-                if (xy) {
+                if (M || xy) {
 #pragma unroll
-                    for (int t = 0; t < 2; t++) {
+                    for (int t = 0; t < RW; t++) {
                         const int c = o2 + own + CX * t;
                         const float q = qc[CX * t], ql = qc[CX * t - 1];
                         float xw = MX[c - 1], xc = MX[c], xe = MX[c + 1];
                         float nw = MN[c - 1], nc = MN[c], ne = MN[c + 1];
                         const float fl = xf[t], fr = lane_next(fl);
                         float fin = vpos(fl) - vneg(fr), fout = vpos(fr) - vneg(fl);
-                        if (edge_x) {  // the row's end cells: :50-55, :62-68, :79-83, :95-99
+                        if (!M && edge_x) {  // the row's end cells: :50-55, :62-68, :79-83, :95-99
                             xw = at_w ? xc : xw;
                             nw = at_w ? nc : nw;
                             xc = at_e ? q : xc;
@@ -1137,17 +1206,17 @@ __global__ void __launch_bounds__(Tile<TJ>::CNT) __attribute__((amdgpu_waves_per
                     }
                     // y cells on the owned rows and the halo rows 1 and TJ+2
 #pragma unroll
-                    for (int t = 0; t < 3; t++) {
-                        if (t == 2 && !(w == 1 || w == 2)) continue;
-                        const int o = t < 2 ? CX * t : ext - own;
-                        const int c = o2 + own + o, gj = t < 2 ? gj0 + t : j0 + rx;
+                    for (int t = 0; t < RW + 1; t++) {
+                        if (t == RW && !(w == 1 || w == 2)) continue;
+                        const int o = t < RW ? CX * t : ext - own;
+                        const int c = o2 + own + o, gj = t < RW ? gj0 + t : j0 + rx;
                         const float q = qc[o];
                         float hi, low, fin, fout;
-                        if (gj <= 0) {
+                        if (!M && gj <= 0) {
                             hi = vmax(MX[c], MX[c + CX]);
                             low = vmin(MN[c], MN[c + CX]);
                             fin = fout = 0.0f;
-                        } else if (gj >= ny - 1) {
+                        } else if (!M && gj >= ny - 1) {
                             hi = vmax(MX[c - CX], q);
                             low = vmin(MN[c - CX], q);
                             fin = fout = 0.0f;
@@ -1166,31 +1235,31 @@ __global__ void __launch_bounds__(Tile<TJ>::CNT) __attribute__((amdgpu_waves_per
                 }
                 // z: betas of cell L1 of each owned column, then the limited
                 // velocity and flux on the face between L2 and L1 (flux_is_w ends)
-                if (zf) {
+                if (M || zf) {
 #pragma unroll
-                    for (int t = 0; t < 2; t++) {
+                    for (int t = 0; t < RW; t++) {
                         const int c = own + CX * t;
                         const float q = qu[CX * t];
                         float hi, low, fin, fout;
-                        if (L1 == 0) {
-                            hi = vmax(MX[o1 + c], MX[om + c]);
-                            low = vmin(MN[o1 + c], MN[om + c]);
+                        if (!M && L1 == 0) {
+                            hi = vmax(MX[o1 + c], bx[t]);
+                            low = vmin(MN[o1 + c], bn[t]);
                             fin = 0.0f - vneg(fz1[t]);
                             fout = vpos(fz1[t]);
-                        } else if (L1 == nz - 1) {
+                        } else if (!M && L1 == nz - 1) {
                             hi = vmax(MX[o2 + c], q);
                             low = vmin(MN[o2 + c], q);
                             fin = vpos(fz2[t]) - vneg(fz2[t]);
                             fout = fin;
                         } else {
-                            hi = vmax3(MX[o2 + c], MX[o1 + c], MX[om + c]);
-                            low = vmin3(MN[o2 + c], MN[o1 + c], MN[om + c]);
+                            hi = vmax3(MX[o2 + c], MX[o1 + c], bx[t]);
+                            low = vmin3(MN[o2 + c], MN[o1 + c], bn[t]);
                             fin = vpos(fz2[t]) - vneg(fz1[t]);
                             fout = vpos(fz1[t]) - vneg(fz2[t]);
                         }
                         float bi, bo;
                         betas(q, hi, low, fin, fout, bi, bo);
-                        if (L2 >= m0) {
+                        if (M || L2 >= m0) {
                             const float u = limit_u(wu2[t], wu2[t] > 0.0f, bi, bo, bzi[t], bzo[t]);
                             Fzc[t] = flux1(qc[CX * t], q, u);
                         }
@@ -1199,11 +1268,14 @@ __global__ void __launch_bounds__(Tile<TJ>::CNT) __attribute__((amdgpu_waves_per
                     }
                 }
             };
-            if (ok) phase_c(std::integral_constant<bool, true>{});
-            else phase_c(std::integral_constant<bool, false>{});
+            if (!ok) phase_c(no, no);
+            else if (mid && inner) phase_c(yes, yes);
+            else phase_c(yes, no);
+            yn = VU[own + RW * CX];
         } else {
+            yn = VF[own + RW * CX];
 #pragma unroll
-            for (int t = 0; t < 2; t++) {
+            for (int t = 0; t < RW; t++) {
                 if (L2 >= m0 && L2 <= nz - 2) Fzc[t] = fz2[t];
                 if (xy) {
                     Fxl[t] = xf[t];
@@ -1212,32 +1284,32 @@ __global__ void __launch_bounds__(Tile<TJ>::CNT) __attribute__((amdgpu_waves_per
             }
         }
         stage(m + 1);
-        prefetch(m + 2);
         __syncthreads();
 
         // ---------------- (D) flux divergence on level L2 (upwind_advection
         // :86-97) with the limited velocities of the cell's four side faces
         if (threadIdx.x < 2) out_of[(m + 2) & 3][threadIdx.x] = 0;
-        stage_bounds(m + 1);
-        if (PF) load_coef(m + 1);
+        put_bounds(m);
+        bounds(m + 1);
+        prefetch(m + 2);
         if (xy) {
             // the y faces south of the owned rows and of the row north of them
-            float Fy[3];
+            float Fy[RW + 1];
             if (FCT) {
 #pragma unroll
-                for (int t = 0; t < 3; t++) {
+                for (int t = 0; t < RW + 1; t++) {
                     const int c = own + CX * t;
-                    const float v = t < 2 ? yu[t] : vu[c];
+                    const float v = t < RW ? yu[t] : yn;
                     const float u = limit_u(v, v > 0.0f, BI[c], BO[c], BI[c - CX], BO[c - CX]);
                     Fy[t] = flux1(qc[CX * (t - 1)], qc[CX * t], u);
                 }
             } else {
-                Fy[0] = yf[0];
-                Fy[1] = yf[1];
-                Fy[2] = VF[own + 2 * CX];
+#pragma unroll
+                for (int t = 0; t < RW; t++) Fy[t] = yf[t];
+                Fy[RW] = yn;
             }
 #pragma unroll
-            for (int t = 0; t < 2; t++) {
+            for (int t = 0; t < RW; t++) {
                 const int gj = gj0 + t;
                 float q = qc[CX * t];
                 if (gj > 0 && gj < ny - 1) {  // the ring keeps its values
@@ -1253,6 +1325,7 @@ __global__ void __launch_bounds__(Tile<TJ>::CNT) __attribute__((amdgpu_waves_per
                 }
                 if (lane_out && gj < ny) {  // gj >= 0: owned rows start at the tile's first
                     const size_t c = ra[t] + sk * (size_t)L2;
+                    fresh();
                     const uint32_t rnd = is_sr(p.kindo) ? sr_bits((uint32_t)c + lo, s, tstep) : 0u;
                     if (QK == QK_F32 || p.kindo == ICAR_ADV_STORE_F32)
                         *(gfloat *)((gchar *)(gfloat *)((float *)p.out + c) + lo * 4u) = q;
@@ -1262,7 +1335,7 @@ __global__ void __launch_bounds__(Tile<TJ>::CNT) __attribute__((amdgpu_waves_per
             }
         }
 #pragma unroll
-        for (int t = 0; t < 2; t++) Fzp[t] = Fzc[t];
+        for (int t = 0; t < RW; t++) Fzp[t] = Fzc[t];
     }
 }
 
@@ -1322,8 +1395,7 @@ struct FastBatch {
     std::vector<float> dts;              // dt values in the device tables
     unsigned total_cb = 0, total_work = 0;
     double cells = 0, cell_species = 0;  // for the algorithmic byte counts
-    int corr_cfg = 1;    // corrective kernel: bit 0 -> 4 waves/SIMD, bit 1 -> no prefetch,
-                         // bit 2 -> 60x32 tiles
+    int corr_cfg = 3;    // corrective kernel's tile (launch_corr_t)
     int tj = 16;         // output rows per corrective tile (tile_rows(corr_cfg))
     int nks = 1;         // requested column chunks along k
     bool tuned = false;  // launch configuration chosen (autotuned or fixed by the environment)
@@ -1544,19 +1616,21 @@ int upload_tables(FastBatch *b, std::string *err)
     return 0;
 }
 
-// corr_cfg: bit 1 -> coefficients loaded where they are used, bit 2 -> 60x8
-// tiles of 4 waves (60x16 tiles of 8 waves otherwise)
+// corr_cfg: bit 2 -> 8 tile rows (16 otherwise); bit 0 -> two rows per wave, or,
+// clear and with 8 tile rows, one; bit 1 has no effect
 template <bool FCT, int QK>
 void launch_corr_t(unsigned nb, hipStream_t s, const DomDesc *D, int n, int pass, unsigned nw,
                    int cfg, int fast)
 {
-    constexpr unsigned T16 = Tile<16>::CNT, T8 = Tile<8>::CNT;
-    switch (cfg & 6) {
-    case 0: hipLaunchKernelGGL((k_corr<FCT, 4, true, QK, 16>), dim3(nb), dim3(T16), 0, s, D, n, pass, nw, fast); break;
-    case 2: hipLaunchKernelGGL((k_corr<FCT, 4, false, QK, 16>), dim3(nb), dim3(T16), 0, s, D, n, pass, nw, fast); break;
-    case 4: hipLaunchKernelGGL((k_corr<FCT, 4, true, QK, 8>), dim3(nb), dim3(T8), 0, s, D, n, pass, nw, fast); break;
-    default: hipLaunchKernelGGL((k_corr<FCT, 4, false, QK, 8>), dim3(nb), dim3(T8), 0, s, D, n, pass, nw, fast); break;
-    }
+    auto go = [&](auto rw, auto tj) {
+        hipLaunchKernelGGL((k_corr<FCT, rw.value, QK, tj.value>), dim3(nb),
+                           dim3(Tile<tj.value, rw.value>::CNT), 0, s, D, n, pass, nw, fast);
+    };
+    constexpr std::integral_constant<int, 1> one;
+    constexpr std::integral_constant<int, 2> two;
+    if (!(cfg & 4)) go(two, std::integral_constant<int, 16>{});
+    else if (cfg & 1) go(two, std::integral_constant<int, 8>{});
+    else go(one, std::integral_constant<int, 8>{});
 }
 
 // the kernels' storage class for a batch: FP32 only, FP32 and BF16, or any kind
@@ -1678,10 +1752,10 @@ int fast_batch_tune(FastBatch *b, hipStream_t s, std::string *err)
             return 0;
         }
     }
-    // candidates: the tile heights and launch configurations, and column
-    // chunks while one chunk per column leaves the GPU with few blocks
+    // candidates: the tiles, and column chunks while one chunk per column
+    // leaves the GPU with few blocks
     std::vector<int> cfgs = fix_cfg ? std::vector<int>{b->corr_cfg}
-                                    : std::vector<int>{1, 3, 5, 7};
+                                    : std::vector<int>{3, 7, 6};
     const int n = (int)b->doms.size();
     const int par = b->doms[0].st->cur;
     // The timed launches are pass 2, which writes only the FP32 pass buffer

@@ -12,7 +12,8 @@ from test_gpu_parity import fresh_species, random_domain
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(61, 7, 4, 1), (60, 8, 3, 1), (63, 9, 9, 2), (122, 17, 13, 3), (59, 25, 8, 1)]
+SHAPES = [(61, 7, 4, 1), (60, 8, 3, 1), (63, 9, 9, 2), (122, 17, 13, 3), (59, 25, 8, 1),
+          (185, 40, 9, 2)]  # the last has tiles and levels away from every edge
 
 
 def spread(case, seed):
@@ -32,7 +33,7 @@ def spread(case, seed):
     q[3][...] = ends[r.integers(0, len(ends), shape)]
 
 
-@pytest.mark.parametrize("cfg", [1, 3, 5, 7])
+@pytest.mark.parametrize("cfg", [3, 6, 7])
 @pytest.mark.parametrize("order,fct", [(2, True), (3, True), (2, False)])
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
 def test_corrective_tiles_and_ranges_match_oracle(oracle32, monkeypatch, shape, order, fct, cfg):
