@@ -92,10 +92,10 @@ __device__ __forceinline__ bool wind_in_range(float u)
 __device__ __forceinline__ bool divisor_in_range(float r) { return r >= 0x1p-30f && r <= 0x1p30f; }
 
 // x / C for the constants C = 12 and 60 of flux3, with R = 1/C rounded: the
-// quotient estimate q = x*R, its remainder x - q*C (exact in one FMA) and
-// q + remainder*R rounded once.  Compared with the IEEE division over every
-// float for both constants, this returns the IEEE quotient for each x with
-// |x| >= 2^-124 and for +-0 (whose sign copysign restores).  F: the guard
+// quotient estimate q = x*R, its remainder negated, q*C - x (exact in one FMA),
+// and q - (that)*R rounded once; so a zero x keeps its sign.  Compared with the
+// IEEE division over every float for both constants, this returns the IEEE
+// quotient for each x with |x| >= 2^-124 and for +-0.  F: the guard
 // takes x whose estimate is not a normal number or zero; otherwise smaller x,
 // infinities and NaNs take the IEEE division, a branch the lanes of a wave
 // skip unless one needs it.
@@ -109,8 +109,7 @@ __device__ __forceinline__ float div_const(float x, Guard &g)
     }
     const float q = x * R;
     if (F) g.bad |= __builtin_amdgcn_classf(q, NOT_REGULAR);
-    const float e = __builtin_fmaf(-q, (float)C, x);
-    return __builtin_copysignf(__builtin_fmaf(e, R, q), x);
+    return __builtin_fmaf(-__builtin_fmaf(q, (float)C, -x), R, q);
 }
 
 // |u| / C for a wind (F: in range, k_std_wind)
@@ -338,27 +337,32 @@ typedef __attribute__((address_space(1))) char gchar;
 typedef __attribute__((address_space(1))) const float gcfloat;
 typedef __attribute__((address_space(1))) float gfloat;
 
-// element c (uniform) plus a lane's 32-bit offset in elements
+// element c (uniform) plus a lane's 32-bit offset in bytes.  With an offset the
+// compiler knows nothing of (unknown) the base stays in scalar registers and
+// the access takes both; one it can widen ahead of the loop takes a 64-bit
+// addition per access and register pairs.
+__device__ __forceinline__ void unknown(unsigned &o) { asm("" : "+v"(o)); }
+// the same for a scalar: sums of it with every base are not kept over the loop
+__device__ __forceinline__ void unknown(size_t &o) { asm("" : "+s"(o)); }
 __device__ __forceinline__ float gld(const float *p, size_t c, unsigned lane)
 {
-    return *(gcfloat *)((gcchar *)(gcfloat *)(p + c) + lane * 4u);
+    return *(gcfloat *)((gcchar *)(gcfloat *)(p + c) + lane);
 }
 __device__ __forceinline__ void gst(float *p, size_t c, unsigned lane, float v)
 {
-    *(gfloat *)((gchar *)(gfloat *)(p + c) + lane * 4u) = v;
+    *(gfloat *)((gchar *)(gfloat *)(p + c) + lane) = v;
 }
 
-// the value of the next lane (lane 63: its own) and of the previous lane
-// (lane 0: its own)
+// the value of the next lane (lane 63: 0) and of the previous lane (lane 0: 0)
 __device__ __forceinline__ float lane_next(float v)
 {
     const int b = __float_as_int(v);
-    return __int_as_float(__builtin_amdgcn_update_dpp(b, b, 0x130, 0xf, 0xf, false));  // wave_shl:1
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, b, 0x130, 0xf, 0xf, true));  // wave_shl:1
 }
 __device__ __forceinline__ float lane_prev(float v)
 {
     const int b = __float_as_int(v);
-    return __int_as_float(__builtin_amdgcn_update_dpp(b, b, 0x138, 0xf, 0xf, false));  // wave_shr:1
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, b, 0x138, 0xf, 0xf, true));  // wave_shr:1
 }
 
 // A block's place: species, tile and chunk; lane L holds column ib + L, row r
@@ -368,7 +372,7 @@ struct Place {
     int s, ib, j0, k0, k1;
     int L, w;
     int x0;             // first column of the tile's addresses
-    unsigned lane;      // this lane's clamped column - x0
+    unsigned lane;      // this lane's clamped column - x0, in bytes
     size_t sk, sj;
     // cell (x0, 0, row r), the row clamped to the domain
     __device__ __forceinline__ size_t row(int r) const
@@ -380,10 +384,10 @@ struct Place {
     {
         return (size_t)x0 + (sk + 1) * (size_t)d.nz * (size_t)min(max(j0 + r, 0), d.ny - 1);
     }
-    // clamped column ib + c as an offset from x0
+    // clamped column ib + c as an offset from x0 in bytes
     __device__ __forceinline__ unsigned col(int c) const
     {
-        return (unsigned)(min(max(ib + c, 0), d.nx - 1) - x0);
+        return (unsigned)(min(max(ib + c, 0), d.nx - 1) - x0) * 4u;
     }
 };
 
@@ -451,12 +455,12 @@ __device__ __forceinline__ float face_under(float w, const float *q, size_t o, u
 // One barrier per level: iteration k reads plane k (x, y) and its own columns
 // of the ring (z), stages level k + LA into the slot of the lowest level only
 // its own columns read, and passes the y faces through a buffer per parity.
-// Measured on 1024 x 1024 x 30, 10 species, h5/v3: mode 0 1.68 ms (6.9 GB,
-// 4.1 TB/s; VALU 0.61 of its issue rate), mode 1 2.04 ms (6.2 GB; VALU 0.73),
-// against 1.93 and 2.29 ms for one-row waves over 7-row tiles whose quotients
-// took the IEEE sequence.  Six waves per SIMD: 80 registers hold mode 1 with
-// a few values in scratch; five waves (no scratch) and eight take 2.3 and 3.4
-// ms.
+// Measured on 1024 x 1024 x 30, 10 species, h5/v3: mode 0 1.62 ms (6.9 GB,
+// 4.3 TB/s: near the rate of a copy), mode 1 1.94 ms (6.2 GB; waiting for
+// memory and barriers half of the time), against 1.93 and 2.29 ms for one-row
+// waves over 7-row tiles whose quotients took the IEEE sequence.  Six waves
+// per SIMD: 80 registers hold mode 1 with a few values in scratch; five waves
+// (no scratch) and eight took 2.3 and 3.4 ms.
 template <int H, int V, int MODE, int RW>
 __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(6)))
     k_std_stage(StdGeom g, float t, StdBatch b, Region r)
@@ -466,7 +470,7 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(6)))
     constexpr bool FL = MODE <= 1, DQ = MODE >= 1;
     __shared__ float sq[P::WORDS];
     __shared__ float sy[2][NWAVE + 1][64], sh[2][DQ ? NWAVE + 1 : 1][64];
-    const Place p = place<SCOLS, TJ>(g.d, r, 0, HH);
+    Place p = place<SCOLS, TJ>(g.d, r, 0, HH);
     const bool ok = *g.general == 0u;  // winds and divisors in range (k_std_wind)
     const int nz = p.d.nz, w = p.w, L = p.L;
     const size_t sk = p.sk, su = p.sk + 1;
@@ -483,14 +487,14 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(6)))
         ca[e] = p.row(ra + e);
         ua[e] = p.urow(ra + e);
     }
-    const size_t cx = p.row(hx ? rx : ra), cl = p.row(last ? TJ : ra);
+    size_t cx = p.row(hx ? rx : ra), cl = p.row(last ? TJ : ra);
     // columns beside the own rows: lanes 0..7 for row ra, 8..15 for ra + 1.  A
     // lane's element offset from row ra holds in 32 bits, also in bytes (a
     // domain has at most 2^30 cells).
     const int he = L & 7, hr = (L >> 3) & 1;
     const bool hc = L < 8 * RW && he < P::XH;
     const int hcol = he < HH ? he - HH : 64 + he - HH;
-    const unsigned hoff = (hr ? (unsigned)(ca[RW - 1] - ca[0]) : 0u) + p.col(hcol);
+    unsigned hoff = (hr ? (unsigned)(ca[RW - 1] - ca[0]) * 4u : 0u) + p.col(hcol);
     const int own = P::at(ra, L), ext = P::at(rx, L), hdst = P::at(ra + hr, hcol);
     const bool cell = L < SCOLS && p.ib + L <= r.i_hi;
     const bool put_x = MODE == 0 ? cell : cell && p.ib + L >= g.its && p.ib + L <= g.ite;
@@ -499,10 +503,17 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(6)))
     auto fetch = [&](int k) {
         if (k >= nz) return;
         const size_t o = sk * (size_t)k;
+        unknown(p.lane);
 #pragma unroll
         for (int e = 0; e < RW; e++) n0[e] = gld(qin, ca[e] + o, p.lane);
-        if (hx) nx_ = gld(qin, cx + o, p.lane);
-        if (hc) nh = gld(qin, ca[0] + o, hoff);
+        if (hx) {
+            unknown(p.lane);
+            nx_ = gld(qin, cx + o, p.lane);
+        }
+        if (hc) {
+            unknown(hoff);
+            nh = gld(qin, ca[0] + o, hoff);
+        }
     };
     auto stage = [&](int k) {
         if (k >= nz) return;
@@ -516,13 +527,17 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(6)))
     float fu[RW], fv[RW + 1], fw[RW];
     auto winds = [&](int k) {
         const size_t o = sk * (size_t)k;
+        unknown(p.lane);
 #pragma unroll
         for (int e = 0; e < RW; e++) {
             fu[e] = gld(g.Um, ua[e] + su * (size_t)k, p.lane);
             fv[e] = gld(g.Vm, ca[e] + o, p.lane);
             fw[e] = gld(g.Wm, ca[e] + o, p.lane);
         }
-        if (last) fv[RW] = gld(g.Vm, cl + o, p.lane);
+        if (last) {
+            unknown(p.lane);
+            fv[RW] = gld(g.Vm, cl + o, p.lane);
+        }
     };
 
     float fzb[RW], hzb[RW];  // the faces under the level
@@ -545,10 +560,18 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(6)))
     __syncthreads();
 #pragma unroll 1
     for (int k = p.k0; k < p.k1; k++) {
+#pragma unroll
+        for (int e = 0; e < RW; e++) {
+            unknown(ca[e]);
+            unknown(ua[e]);
+        }
+        unknown(cx);
+        unknown(cl);
         const size_t o = sk * (size_t)k;
         const bool top = k == nz - 1;
         const float *const q = sq + P::level(k) + own;  // plane k, row ra, this lane
         float rj[RW], rdj[RW], o0[RW];
+        unknown(p.lane);
 #pragma unroll
         for (int e = 0; e < RW; e++) {
             rj[e] = gld(g.Rj, ca[e] + o, p.lane);
@@ -628,6 +651,7 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(6)))
 #pragma unroll
         for (int e = 0; e < RW; e++) {
             const int j = p.j0 + ra + e;
+            unknown(p.lane);
             if (FL && put_x && j <= g.jte && (MODE == 0 || j >= g.jts)) gst(out, ca[e] + o, p.lane, qn[e]);
             if (DQ && cell && j <= r.j_hi) gst(odq, ca[e] + o, p.lane, dn[e]);
             if (FL) fzb[e] = fz[e];
@@ -646,12 +670,12 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(6)))
 // ring: wave w holds the RW rows from RW w - 1 of the tile on, lane L column ib + L (x
 // faces on lanes 0..63, scales on 0..62 of rows -1..LROWS, cells 1..61 of
 // rows 0..LROWS-1; the last row supplies its south face only).  Two barriers
-// per level.  Bound by VALU issue (about 0.85 of its rate) with two blocks of
-// eight waves per CU; what a level carries to the next is kept small (126
-// registers at h5/v3: the state after the horizontal update instead of its
-// parts, one register for the one halo row a wave stages) because spilling it
-// took 4.7 ms and keeping it in three-row slots 9.3.  1024 x 1024 x 30, 10
-// species, h5/v3: 4.2 ms, against 6.4 ms for two marches that each computed
+// per level.  Bound by VALU issue and the waits at the barriers, with two
+// blocks of eight waves per CU; what a level carries to the next is kept small
+// (113 registers at h5/v3: the state after the horizontal update instead of
+// its parts, one register for the one halo row a wave stages) because spilling
+// it took 4.7 ms and keeping it in three-row slots 9.3.  1024 x 1024 x 30, 10
+// species, h5/v3: 4.1 ms, against 6.4 ms for two marches that each computed
 // the faces, the first writing the scales for the second (and 8 bytes per
 // cell and species of device memory).
 template <int H, int V, int RW>
@@ -667,7 +691,7 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(4, 4)
     // y faces south of a wave's first row: upwind, flux3, wind
     __shared__ float yu[NWAVE + 1][64], yh[NWAVE + 1][64], yv[NWAVE + 1][64];
     __shared__ float ssi[TJ + 2][64], sso[TJ + 2][64];  // scale_in, scale_out of row r - 2 at [r]
-    const Place p = place<LCOLS, LROWS>(g.d, r, -1, HH);
+    Place p = place<LCOLS, LROWS>(g.d, r, -1, HH);
     const bool ok = *g.general == 0u;  // winds and divisors in range (k_std_wind)
     const int nz = p.d.nz, w = p.w, L = p.L;
     const size_t sk = p.sk, su = p.sk + 1;
@@ -684,7 +708,7 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(4, 4)
         ca[e] = p.row(ra + e);
         ua[e] = p.urow(ra + e);
     }
-    const size_t cq = p.row(hq ? rq : ra), cb = p.row(-2);
+    size_t cq = p.row(hq ? rq : ra), cb = p.row(-2);
     // columns beside the rows: lanes 0..7 row ra, 8..15 row ra + 1; the first
     // XH of qin, the last two column -1 of dq and of qold.  A lane's element
     // offset from row ra holds in 32 bits, also in bytes (a domain has at
@@ -692,8 +716,8 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(4, 4)
     const int he = L & 7, hr = (L >> 3) & 1;
     const bool hcq = L < 8 * RW && he < P::XH, hcb = L < 8 * RW && he >= 6;
     const int hcol = he < HH ? he - HH : 64 + he - HH;
-    const unsigned hrow = hr ? (unsigned)(ca[RW - 1] - ca[0]) : 0u;
-    const unsigned hqoff = hrow + p.col(hcol), hboff = hrow + p.col(-1);
+    const unsigned hrow = hr ? (unsigned)(ca[RW - 1] - ca[0]) * 4u : 0u;
+    unsigned hqoff = hrow + p.col(hcol), hboff = hrow + p.col(-1);
     const int hqdst = P::at(ra + hr, hcol), hbdst = B::at(ra + hr, -1);
     const int ownq = P::at(ra, L), ownb = B::at(ra, L);
     const int extq = P::at(rq, L), extb = B::at(-2, L);
@@ -705,10 +729,17 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(4, 4)
     auto fetch_q = [&](int k) {
         if (k >= nz) return;
         const size_t o = sk * (size_t)k;
+        unknown(p.lane);
 #pragma unroll
         for (int e = 0; e < RW; e++) nq[e] = gld(qin, ca[e] + o, p.lane);
-        if (hq) nrow = gld(qin, cq + o, p.lane);
-        if (hcq) nhq = gld(qin, ca[0] + o, hqoff);
+        if (hq) {
+            unknown(p.lane);
+            nrow = gld(qin, cq + o, p.lane);
+        }
+        if (hcq) {
+            unknown(hqoff);
+            nhq = gld(qin, ca[0] + o, hqoff);
+        }
     };
     auto stage_q = [&](int k) {
         if (k >= nz) return;
@@ -721,14 +752,20 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(4, 4)
     auto fetch_b = [&](int k) {
         if (k >= nz) return;
         const size_t o = sk * (size_t)k;
+        unknown(p.lane);
 #pragma unroll
         for (int e = 0; e < RW; e++) {
             no[e] = gld(qo, ca[e] + o, p.lane);
             nd[e] = gld(dq, ca[e] + o, p.lane);
         }
-        if (ho) nrow = gld(qo, cb + o, p.lane);
-        if (hd) nrow = gld(dq, cb + o, p.lane);
-        if (hcb) nhb = he == 7 ? gld(qo, ca[0] + o, hboff) : gld(dq, ca[0] + o, hboff);
+        if (ho || hd) {
+            unknown(p.lane);
+            nrow = gld(ho ? qo : dq, cb + o, p.lane);
+        }
+        if (hcb) {
+            unknown(hboff);
+            nhb = he == 7 ? gld(qo, ca[0] + o, hboff) : gld(dq, ca[0] + o, hboff);
+        }
     };
     auto stage_b = [&](int k) {
         if (k >= nz) return;
@@ -745,6 +782,7 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(4, 4)
     float fu[RW], fv[RW], fw[RW];
     auto winds = [&](int k) {
         const size_t o = sk * (size_t)k;
+        unknown(p.lane);
 #pragma unroll
         for (int e = 0; e < RW; e++) {
             fv[e] = gld(g.Vm, ca[e] + o, p.lane);
@@ -768,13 +806,13 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(4, 4)
             mzb[e] = face_under<V>(wb[e], qin, o, p.lane, kb, nz, sk) - uzb[e];
         }
     }
-    // of the level below: its state after the horizontal fluxes, scales and
-    // vertical divisor, and the limited flux through its lower face
-    float ph[RW], psi[RW], pso[RW], prdj[RW], Fzb[RW];
+    // of the level below: its state after the horizontal fluxes, scales,
+    // vertical divisor and its reciprocal, and the limited flux through its lower face
+    float ph[RW], psi[RW], pso[RW], prdj[RW], pydj[RW], Fzb[RW];
 #pragma unroll
     for (int e = 0; e < RW; e++) {
         ph[e] = Fzb[e] = 0.0f;
-        psi[e] = pso[e] = prdj[e] = 1.0f;
+        psi[e] = pso[e] = prdj[e] = pydj[e] = 1.0f;
     }
     for (int k = max(0, kb - LA + 1); k < min(nz, kb + LA); k++) {
         fetch_q(k);
@@ -802,14 +840,14 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(4, 4)
             constexpr bool FD = F.value;
 #pragma unroll
             for (int e = 0; e < RW; e++) {
-                const float ydj = FD ? recip_nr(prdj[e]) : 0.0f;
-                v[e] = ph[e] - div_by<FD>(Fzt[e] - Fzb[e], prdj[e], ydj, gd);
+                v[e] = ph[e] - div_by<FD>(Fzt[e] - Fzb[e], prdj[e], pydj[e], gd);
                 if (FD) gd.bad |= __builtin_amdgcn_classf(v[e], NOT_FINITE);
             }
         });
 #pragma unroll
         for (int e = 0; e < RW; e++) {
             const int row = ra + e;
+            unknown(p.lane);
             if (put_x && row >= 0 && row < LROWS && p.j0 + row <= g.jte)
                 gst(out, ca[e] + sk * (size_t)k, p.lane, v[e]);
         }
@@ -817,11 +855,19 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(4, 4)
     bool below_fine = kb == 0;
 #pragma unroll 1
     for (int k = kb; k <= ke; k++) {
+#pragma unroll
+        for (int e = 0; e < RW; e++) {
+            unknown(ca[e]);
+            unknown(ua[e]);
+        }
+        unknown(cq);
+        unknown(cb);
         const size_t o = sk * (size_t)k;
         const bool top = k == nz - 1;
         const float *const q = sq + P::level(k) + ownq;
         const float *const po = so + B::level(k) + ownb, *const pd = sd + B::level(k) + ownb;
         float rj[RW], rdj[RW];
+        unknown(p.lane);
 #pragma unroll
         for (int e = 0; e < RW; e++) {
             rj[e] = gld(g.Rj, ca[e] + o, p.lane);
@@ -877,6 +923,12 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(4, 4)
 
         // the north faces: the own next row's, or the next wave's first
         float si[RW], sc[RW], un[RW], mn[RW], vn[RW];
+        float yj[RW], ydj[RW];  // reciprocals of the divisors (used where they are in range)
+#pragma unroll
+        for (int e = 0; e < RW; e++) {
+            yj[e] = recip_nr(rj[e]);
+            ydj[e] = recip_nr(rdj[e]);
+        }
 #pragma unroll
         for (int e = 0; e < RW; e++) {
             un[e] = e + 1 < RW ? uy[RW - 1] : yu[w + 1][L];
@@ -908,17 +960,16 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(4, 4)
                 const float qmin = mn2(vt, mn2(vb, mn2(vy, mn2(vx, o0))));
                 const float zero = 0.0f;
                 if (FD) gd.bad |= __builtin_amdgcn_classf(mn[e], NOT_FINITE);
-                const float yj = FD ? recip_nr(rj[e]) : 0.0f, ydj = FD ? recip_nr(rdj[e]) : 0.0f;
                 // :75-78 the upwind-only value
                 const float temp = flux_update<FD>(o0, ux[e], uxe, uy[e], un[e], uzl, uz[e], rj[e],
-                                                   rdj[e], yj, ydj, gd);
+                                                   rdj[e], yj[e], ydj[e], gd);
                 // :88-96
                 float fin = div_by<FD>(-((mn2(zero, me) - mx2(zero, mx[e])) + (mn2(zero, mn[e]) - mx2(zero, my[e]))),
-                                       rj[e], yj, gd);
-                fin = fin - div_by<FD>(mn2(zero, mz[e]) - mx2(zero, mb), rdj[e], ydj, gd);
+                                       rj[e], yj[e], gd);
+                fin = fin - div_by<FD>(mn2(zero, mz[e]) - mx2(zero, mb), rdj[e], ydj[e], gd);
                 float fout = div_by<FD>((mx2(zero, me) - mn2(zero, mx[e])) + (mx2(zero, mn[e]) - mn2(zero, my[e])),
-                                        rj[e], yj, gd);
-                fout = fout + div_by<FD>(mx2(zero, mz[e]) - mn2(zero, mb), rdj[e], ydj, gd);
+                                        rj[e], yj[e], gd);
+                fout = fout + div_by<FD>(mx2(zero, mz[e]) - mn2(zero, mb), rdj[e], ydj[e], gd);
                 // :124-125
                 const float up = qmax - temp, dn = temp - qmin;
                 const float di = fin + 1.E-15f, dd = fout + 1.E-15f;
@@ -980,7 +1031,7 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(4, 4)
             constexpr bool FD = F.value;
 #pragma unroll
             for (int e = 0; e < RW; e++) {
-                ph[e] = po[e * B::QC] - div_by<FD>(hs[e], rj[e], FD ? recip_nr(rj[e]) : 0.0f, gd);
+                ph[e] = po[e * B::QC] - div_by<FD>(hs[e], rj[e], yj[e], gd);
                 if (FD) gd.bad |= __builtin_amdgcn_classf(ph[e], NOT_FINITE);
             }
         });
@@ -989,6 +1040,7 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(4, 4)
             psi[e] = si[e];
             pso[e] = sc[e];
             prdj[e] = rdj[e];
+            pydj[e] = ydj[e];
             mzb[e] = mz[e];
             uzb[e] = uz[e];
         }
