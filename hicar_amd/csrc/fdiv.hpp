@@ -12,7 +12,7 @@
 // icar_adv_verify_division compares the quotient with the IEEE division for
 // every pair of significands on the device, and the kernels take this path
 // only inside the range where every operation scales exactly with the
-// operands' exponents (fdiv_in_range), so the significand pairs cover all of
+// operands' exponents, so the significand pairs cover all of
 // it.
 //
 // The remainder is formed negated, rn = q0*d - x, and the quotient as
@@ -33,7 +33,7 @@ __device__ __forceinline__ float recip_nr(float d)
     return __builtin_fmaf(e, y0, y0);
 }
 
-// RN(x/d) from y = recip_nr(d), for operands fdiv_in_range accepts
+// RN(x/d) from y = recip_nr(d), for operands in range (below)
 __device__ __forceinline__ float div_y(float x, float d, float y)
 {
     const float q0 = x * y;
@@ -41,61 +41,20 @@ __device__ __forceinline__ float div_y(float x, float d, float y)
     return __builtin_fmaf(-rn, y, q0);
 }
 
-// The range the fast quotient is taken in: d in [2^-60, 2^40] (positive,
-// down to the 1e-15 the FCT limiter adds to a zero inflow), x zero or |x|
-// in [2^-78, 2^64].  Then 1/d, x*y and the quotient are normal (|x/d| in
-// [2^-118, 2^124]), and the remainder is zero or at least 2^-125 (x is a
-// multiple of 2^(ex-23), q0*d of 2^(ex-48)), so it is exact and normal:
-// every step equals, scaled by a power of two, the same step on the
-// operands' significands.  The device check covers the reciprocal's scaling
-// over d's exponents FDIV_E_LO..FDIV_E_HI.
+// The quotient is taken where the divisor is positive and in [2^-60, 2^60] and
+// the numerator zero or at least 2^-101 (a kernel's own bounds lie inside
+// these), so that 1/d, x*y and the quotient are normal numbers and the
+// remainder is exact: every step then equals, scaled by a power of two, the
+// same step on the operands' significands.  The device check covers the
+// reciprocal's scaling over d's exponents FDIV_E_LO..FDIV_E_HI.
 constexpr int FDIV_E_LO = -60, FDIV_E_HI = 60;
-constexpr float FDIV_D_LO = 0x1p-60f, FDIV_D_HI = 0x1p40f;
-constexpr float FDIV_X_LO = 0x1p-78f, FDIV_X_HI = 0x1p64f;
 
-// Guard accumulators of a group of fast quotients, checked once for the
-// group: the smallest and largest divisor, the largest |numerator| and the
-// smallest non-zero |numerator| (as 2*bits - 1 unsigned, so that +-0 maps to
-// the largest value and never counts as small).
-struct DivGuard {
-    float dlo = FDIV_D_HI, dhi = FDIV_D_LO, xhi = 0.0f;
-    uint32_t xlo = 0xffffffffu;
-};
-
+// The key of a numerator by which the kernels find the smallest non-zero one
+// of a group: 2*bits - 1 unsigned, so that +-0 maps to the largest value and
+// never counts as small
 __device__ __forceinline__ uint32_t nz_key(float x)
 {
-    return (__float_as_uint(x) << 1) - 1u;  // +-0 -> 0xffffffff
-}
-
-// a division's operands into the guard
-__device__ __forceinline__ void guard_div(DivGuard &g, float x, float d)
-{
-    g.dlo = fminf(g.dlo, d);
-    g.dhi = fmaxf(g.dhi, d);
-    g.xhi = fmaxf(g.xhi, fabsf(x));
-    g.xlo = min(g.xlo, nz_key(x));
-}
-
-// a numerator only (its divisor is known to be in range)
-__device__ __forceinline__ void guard_num(DivGuard &g, float x)
-{
-    g.xhi = fmaxf(g.xhi, fabsf(x));
-    g.xlo = min(g.xlo, nz_key(x));
-}
-
-// a divisor only
-__device__ __forceinline__ void guard_den(DivGuard &g, float d)
-{
-    g.dlo = fminf(g.dlo, d);
-    g.dhi = fmaxf(g.dhi, d);
-}
-
-// true when every guarded quotient of this lane was in range (NaN operands
-// pass: the quotient is NaN either way)
-__device__ __forceinline__ bool guard_ok(const DivGuard &g)
-{
-    return g.dlo >= FDIV_D_LO && g.dhi <= FDIV_D_HI && g.xhi <= FDIV_X_HI &&
-           g.xlo >= ((__float_as_uint(FDIV_X_LO) << 1) - 1u);
+    return (__float_as_uint(x) << 1) - 1u;
 }
 
 }  // namespace icaradv

@@ -72,41 +72,6 @@ __device__ __forceinline__ bool is_bf16(int kind)
     return kind == ICAR_ADV_STORE_BF16 || kind == ICAR_ADV_STORE_BF16_SR;
 }
 
-// A species value in two steps: the raw bits (a 32- or 16-bit load), then the
-// conversion.  Kernels that keep several loads in flight load raw bits first
-// and convert when the values are used, so that no conversion right after a
-// load makes the wave wait for it.
-typedef __attribute__((address_space(1))) const uint32_t gcu32;
-
-// One 32-bit load for either width: FP32 element i, or the aligned pair of
-// 16-bit elements holding element i (16-bit buffers are padded so that the
-// pair of the last element is in bounds).  The same instruction for every
-// storage kind, so a batch mixing kinds needs no branch around its loads.
-__device__ __forceinline__ uint32_t ld_raw(const void *p, size_t i, int kind)
-{
-    return ((gcu32 *)p)[kind == ICAR_ADV_STORE_F32 ? i : (i >> 1)];
-}
-
-// the value of element i from the word ld_raw returned for it, without a
-// branch: both 16-bit forms are decoded and the kind selects, so that no conversion waits on a branch while loads are in flight
-__device__ __forceinline__ float cvt_q(uint32_t w, size_t i, int kind, float scale)
-{
-    const uint32_t raw = (i & 1) ? (w >> 16) : (w & 0xFFFFu);
-    const float vb = __uint_as_float(raw << 16);
-    const float vh = __half2float(__ushort_as_half((uint16_t)raw));
-    const float v16 = (is_bf16(kind) ? vb : vh) * scale;
-    return kind == ICAR_ADV_STORE_F32 ? __uint_as_float(w) : v16;
-}
-
-__device__ __forceinline__ float ld_q(const void *p, size_t i, int kind, float scale)
-{
-    if (kind == ICAR_ADV_STORE_F32) return ((gcfloat *)p)[i];
-    const uint16_t b = ((gcu16 *)p)[i];
-    const float v = is_bf16(kind) ? __uint_as_float((uint32_t)b << 16)
-                                  : __half2float(__ushort_as_half(b));
-    return v * scale;
-}
-
 // 16 random bits for the stochastic rounding of cell c of species s at step t:
 // a counter-based hash (the murmur3 32-bit finaliser of a mixed key), so the
 // rounding is deterministic and reproducible off the device.
@@ -155,66 +120,44 @@ __device__ __forceinline__ uint16_t to16(float v, int kind, float inv_scale, uin
     return __half_as_ushort(__float2half_rn(x));
 }
 
-__device__ __forceinline__ void st_q(void *p, size_t i, int kind, float inv_scale, float v,
-                                     uint32_t rnd)
-{
-    if (kind == ICAR_ADV_STORE_F32)
-        ((gfloat *)p)[i] = v;
-    else
-        ((gu16 *)p)[i] = to16(v, kind, inv_scale, rnd);
-}
-
 __device__ __forceinline__ bool is_sr(int kind)
 {
     return kind == ICAR_ADV_STORE_BF16_SR || kind == ICAR_ADV_STORE_F16_SR;
 }
 
 // The storage kinds a kernel is compiled for: FP32 only; FP32 and the BF16
-// kinds; any kind.  A species' kind is the same for a whole block (or, in the
-// donor-cell kernel, for a species of the loop), so the BF16 class branches on
-// it around its loads: one 16-bit load of a BF16 element (zero-extended) or
-// one 32-bit load of an FP32 one.  The branch holds the load only, so that the
-// load stays in flight past it; the conversion (a shift into the high half
-// and the scale) comes where the value is used.  No FP16 path.
+// kinds; any kind.  A species' kind is the same for a wave, so the kernels
+// branch on it around its loads and stores.
 constexpr int QK_F32 = 0, QK_BF16 = 1, QK_ANY = 2;
 
-// the raw word of element i: the float's bits (FP32), the 16 bits (BF16
-// class, a 16-bit kind), or the ld_raw word (any kind)
-template <int QK>
-__device__ __forceinline__ uint32_t ld_w(const void *p, size_t i, int kind)
-{
-    if (QK == QK_F32) return ((gcu32 *)p)[i];
-    if (QK == QK_BF16) {
-        if (kind == ICAR_ADV_STORE_F32) return ((gcu32 *)p)[i];
-        return ((gcu16 *)p)[i];
-    }
-    return ld_raw(p, i, kind);
-}
+// Accesses of the marching kernels: a scalar element index and the lane's
+// offset in elements.  The species' values come in two steps, the raw bits (a
+// 32- or 16-bit load) and the conversion where the value is used, so that no
+// conversion right after a load makes the wave wait for it.
+typedef __attribute__((address_space(1))) const uint32_t gcu32;
+typedef __attribute__((address_space(1))) const char gcchar;
+typedef __attribute__((address_space(1))) char gchar;
 
-// the value of element i from its ld_w word
-template <int QK>
-__device__ __forceinline__ float cv_w(uint32_t w, size_t i, int kind, float scale)
+__device__ __forceinline__ float ld1(const float *b, size_t c, unsigned lane)
 {
-    if (QK == QK_F32) return __uint_as_float(w);
-    if (QK == QK_BF16)
-        return kind == ICAR_ADV_STORE_F32 ? __uint_as_float(w) : __uint_as_float(w << 16) * scale;
-    return cvt_q(w, i, kind, scale);
+    return *(gcfloat *)((gcchar *)(gcfloat *)(b + c) + lane * 4u);
 }
 
 template <int QK>
-__device__ __forceinline__ void st_w(void *p, size_t i, int kind, float inv_scale, float v,
-                                     uint32_t rnd)
+__device__ __forceinline__ uint32_t ldq(const void *b, size_t c, unsigned lane, int kind)
 {
-    if (QK == QK_F32) {
-        ((gfloat *)p)[i] = v;
-    } else if (QK == QK_BF16) {
-        if (kind == ICAR_ADV_STORE_F32)
-            ((gfloat *)p)[i] = v;
-        else
-            ((gu16 *)p)[i] = bf16_of(v * inv_scale, kind == ICAR_ADV_STORE_BF16_SR, rnd);
-    } else {
-        st_q(p, i, kind, inv_scale, v, rnd);
-    }
+    if (QK == QK_F32 || kind == ICAR_ADV_STORE_F32)
+        return *(gcu32 *)((gcchar *)(gcfloat *)((const float *)b + c) + lane * 4u);
+    return *(gcu16 *)((gcchar *)(gcu16 *)((const uint16_t *)b + c) + lane * 2u);
+}
+
+// the value of ldq's bits
+template <int QK>
+__device__ __forceinline__ float cvq(uint32_t b, int kind, float scale)
+{
+    if (QK == QK_F32 || kind == ICAR_ADV_STORE_F32) return __uint_as_float(b);
+    if (QK == QK_BF16 || is_bf16(kind)) return __uint_as_float(b << 16) * scale;
+    return __half2float(__ushort_as_half((uint16_t)b)) * scale;
 }
 
 // the stored bits of a value at a 16-bit kind of the class
@@ -225,6 +168,16 @@ __device__ __forceinline__ uint16_t q16_of(float v, int kind, float inv_scale, u
     return to16(v, kind, inv_scale, rnd);
 }
 
+template <int QK>
+__device__ __forceinline__ void stq(void *b, size_t c, unsigned lane, int kind, float inv_scale,
+                                    float v, uint32_t rnd)
+{
+    if (QK == QK_F32 || kind == ICAR_ADV_STORE_F32)
+        *(gfloat *)((gchar *)(gfloat *)((float *)b + c) + lane * 4u) = v;
+    else
+        *(gu16 *)((gchar *)(gu16 *)((uint16_t *)b + c) + lane * 2u) =
+            q16_of<QK>(v, kind, inv_scale, rnd);
+}
 
 // One pass of one species: where to read q0 (and q1) and where to write.
 struct SpecPass {
@@ -235,30 +188,20 @@ struct SpecPass {
     float scale0, inv_scaleo;
 };
 
-// The entry in scalar registers: it is the same for every lane of a wave, and
-// known to be it its addresses take no vector registers and branches on the
-// kinds are scalar.
-template <class T>
-__device__ __forceinline__ T uniform_word(T v)
+// Entry s of a species table.  The tables change between launches only, so an
+// entry that is the same for every lane of a wave (as it is in the kernels)
+// comes by scalar loads: read through a plain pointer it would sit in vector
+// registers, and with it every address formed from it.
+__device__ __forceinline__ SpecPass species(const SpecPass *tab, int s)
 {
-    constexpr int W = sizeof(T) / 4;
-    static_assert(sizeof(T) == 4 * W, "whole words");
-    int b[W];
-    __builtin_memcpy(b, &v, sizeof(T));
+    typedef __attribute__((address_space(4))) const uint32_t ccu32;
+    constexpr int W = sizeof(SpecPass) / 4;
+    ccu32 *const w = (ccu32 *)(uintptr_t)(tab + __builtin_amdgcn_readfirstlane(s));
+    uint32_t b[W];
 #pragma unroll
-    for (int e = 0; e < W; e++) b[e] = __builtin_amdgcn_readfirstlane(b[e]);
-    __builtin_memcpy(&v, b, sizeof(T));
-    return v;
-}
-__device__ __forceinline__ SpecPass uniform(SpecPass p)
-{
-    p.q0 = uniform_word(p.q0);
-    p.q1 = uniform_word(p.q1);
-    p.out = uniform_word(p.out);
-    p.kind0 = uniform_word(p.kind0);
-    p.kindo = uniform_word(p.kindo);
-    p.scale0 = uniform_word(p.scale0);
-    p.inv_scaleo = uniform_word(p.inv_scaleo);
+    for (int e = 0; e < W; e++) b[e] = w[e];
+    SpecPass p;
+    __builtin_memcpy(&p, b, sizeof(p));
     return p;
 }
 
@@ -269,6 +212,9 @@ constexpr int MAXP = 16;  // mpdata_order limit
 struct DomDesc {
     Dims d;
     unsigned cb0, bx;     // first global cell block; cell blocks along x
+    unsigned f0;          // first global block of the donor-cell kernel
+    int ftx, fnk, fkch;   // its tiles along x, level chunks and levels per chunk
+    int fng, fsb, fsr;    // its species groups: fsr of fsb + 1 species, then of fsb
     unsigned w0;          // first global corrective work item
     int tiles_x, nspec;
     int nks, kch;         // corrective kernel: column chunks along k and levels per chunk
@@ -291,6 +237,16 @@ __device__ __forceinline__ int find_dom_cb(const DomDesc *D, int nd, unsigned b)
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
         if (D[mid].cb0 <= b) lo = mid; else hi = mid - 1;
+    }
+    return lo;
+}
+
+__device__ __forceinline__ int find_dom_f(const DomDesc *D, int nd, unsigned b)
+{
+    int lo = 0, hi = nd - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (D[mid].f0 <= b) lo = mid; else hi = mid - 1;
     }
     return lo;
 }
@@ -322,12 +278,12 @@ __device__ __forceinline__ void cell_of(const DomDesc &D, unsigned b, int &i, in
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(256) k_courant_b(const DomDesc *__restrict__ DD, int nd)
 {
-    const int dm = find_dom_cb(DD, nd, blockIdx.x);
-    const DomDesc &D = DD[dm];
+    const unsigned blk = xcd_block();
+    const DomDesc &D = DD[find_dom_cb(DD, nd, blk)];
     int i, k, j;
-    cell_of(D, blockIdx.x, i, k, j);
+    cell_of(D, blk, i, k, j);
     const Dims d = D.d;
-    if (blockIdx.x == D.cb0 && threadIdx.x + threadIdx.y == 0) D.step[1] = 0u;
+    if (blk == D.cb0 && threadIdx.x + threadIdx.y == 0) D.step[1] = 0u;
     if (i >= d.nx || j >= d.ny) return;
     gcfloat *__restrict__ den = gp(D.f.density), *__restrict__ fu = gp(D.f.u);
     gcfloat *__restrict__ fv = gp(D.f.v), *__restrict__ fw = gp(D.f.w);
@@ -386,10 +342,10 @@ enum { CUX = 0, CXV, CXW, SGX, CUY, CYU, CYW, SGY, CUZ, CZU, CZV, SGZ, NCOEF };
 
 __global__ void __launch_bounds__(256) k_coef(const DomDesc *__restrict__ DD, int nd)
 {
-    const int dm = find_dom_cb(DD, nd, blockIdx.x);
-    const DomDesc &D = DD[dm];
+    const unsigned blk = xcd_block();
+    const DomDesc &D = DD[find_dom_cb(DD, nd, blk)];
     int i, k, j;
-    cell_of(D, blockIdx.x, i, k, j);
+    cell_of(D, blk, i, k, j);
     const Dims d = D.d;
     if (i >= d.nx || j >= d.ny) return;
     gcfloat *__restrict__ U = gp(D.sf.U), *__restrict__ V = gp(D.sf.V), *__restrict__ Wd = gp(D.sf.Wd);
@@ -456,8 +412,89 @@ __global__ void __launch_bounds__(64) k_tick(const DomDesc *__restrict__ DD, int
 // ---------------------------------------------------------------------------
 // donor-cell pass for every species (upwind_advection, adv_mpdata.f90:43-103)
 // ---------------------------------------------------------------------------
-constexpr int FBX = 64, FBY = 4;
-constexpr int FSB = 4;  // species per load group in k_first
+// the value of the next lane (lane 63: 0) and of the previous lane (lane 0:
+// 0): one move within the wave, no LDS
+__device__ __forceinline__ float lane_next(float v)
+{
+    const int b = __float_as_int(v);
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, b, 0x130, 0xf, 0xf, true));  // wave_shl:1
+}
+__device__ __forceinline__ float lane_prev(float v)
+{
+    const int b = __float_as_int(v);
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, b, 0x138, 0xf, 0xf, true));  // wave_shr:1
+}
+
+// x/d: the IEEE division, or (F) the three-operation quotient of fdiv.hpp
+template <bool F>
+__device__ __forceinline__ float fdiv(float x, float d)
+{
+    if constexpr (F) return div_y(x, d, recip_nr(d));
+    else return x / d;
+}
+
+// the same with y = recip_nr(d) computed once for several numerators
+template <bool F>
+__device__ __forceinline__ float fdiv_y(float x, float d, float y)
+{
+    if constexpr (F) return div_y(x, d, y);
+    else return x / d;
+}
+
+// Maxima and minima of values that come from memory.  fmaxf on such a value
+// first quiets a possible signalling NaN with an instruction of its own; the
+// hardware's max and min ignore quiet NaNs as fmaxf does.
+__device__ __forceinline__ float vmax(float a, float b)
+{
+    float r;
+    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float vmin(float a, float b)
+{
+    float r;
+    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float vmax3(float a, float b, float c)
+{
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+__device__ __forceinline__ float vmin3(float a, float b, float c)
+{
+    float r;
+    asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+// max(0, a), min(0, a), and min(1, a, b)
+__device__ __forceinline__ float vpos(float a)
+{
+    float r;
+    asm("v_max_f32 %0, 0, %1" : "=v"(r) : "v"(a));
+    return r;
+}
+__device__ __forceinline__ float vneg(float a)
+{
+    float r;
+    asm("v_min_f32 %0, 0, %1" : "=v"(r) : "v"(a));
+    return r;
+}
+__device__ __forceinline__ float vmin1(float a, float b)
+{
+    float r;
+    asm("v_min3_f32 %0, 1.0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
+// the largest magnitude of a (not negative), b and c
+__device__ __forceinline__ float vmax3a(float a, float b, float c)
+{
+    float r;
+    asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
 
 // flux1 (adv_mpdata.f90:39)
 __device__ __forceinline__ float flux1(float l, float r, float U)
@@ -465,147 +502,229 @@ __device__ __forceinline__ float flux1(float l, float r, float U)
     return ((U + fabsf(U)) * l + (U - fabsf(U)) * r) / 2.0f;
 }
 
-// FD: the two divisions of each species by G and Gz (the same for every
-// species of the cell: one reciprocal each) as the three-operation quotient
-// of fdiv.hpp where the operands are in range, else, for the whole wave, the
-// IEEE division
-template <int QK, bool FD>
-__global__ void __launch_bounds__(FBX *FBY) k_first(const DomDesc *__restrict__ DD, int nd)
+// A block of four waves covers a tile of 62 columns x 8 rows for up to NS
+// species and marches up a chunk of levels; a wave holds two adjacent rows, one
+// lane per column (lanes 0 and 63 are the neighbours' columns).  So each x face
+// is computed once (the east face comes from the next lane), the y face between
+// the rows once, the z face above a level is the next level's face below, and a
+// level's own values are loaded once: two loads per cell and species and about
+// 35 operations, against seven and 71 with a thread per cell.  The winds'
+// positive and negative parts and the reciprocals of G and Gz serve all species
+// of the block.  The next level's loads are issued before the level is
+// computed.  What bounds it is memory: its accesses' latency and, with species
+// groups re-reading the winds, the traffic (1024 x 1024 x 30, 10 FP32 species:
+// 3.1 GB it cannot do without, 0.67 ms at the rate of a copy).  Measured
+// against a thread per cell: that case 1.20 -> 1.01 ms, 1500 x 1201 x 40, 10
+// BF16 and two FP32 species 4.24 -> 2.36 ms, 517 x 389 x 40, 7 species 0.283 ->
+// 0.214 ms, 256 x 64 x 20, 12 species 24.4 -> 18.7 us, one species 6.6 -> 7.2.
+// NS = 4: two and three species per block take 1.10 and 1.12 ms in the first
+// case, six 0.95 but 2.45 in the second; two where the grid is small
+// (set_first_blocks), 18.7 us against 26 with four.
+constexpr int FCOLS = 62;           // columns a wave writes
+constexpr int FWAVES = 4;           // waves of a block
+constexpr int FROWS = 2 * FWAVES;   // rows of a block
+
+template <int QK, int NS>
+__global__ void __launch_bounds__(64 * FWAVES)
+    k_first(const DomDesc *__restrict__ DD, int nd, int fast)
 {
-    const int dm = find_dom_cb(DD, nd, blockIdx.x);
-    const DomDesc &D = DD[dm];
-    int i, k, j;
-    cell_of(D, blockIdx.x, i, k, j);
-    const Dims d = D.d;
-    if (i >= d.nx || j >= d.ny) return;
-    gcfloat *__restrict__ U = gp(D.sf.U), *__restrict__ V = gp(D.sf.V), *__restrict__ W = gp(D.sf.W);
-    gcfloat *__restrict__ G = gp(D.sf.G), *__restrict__ Gz = gp(D.sf.Gz);
-    const SpecPass *__restrict__ sp = D.pass[0];
-    const int nspec = D.nspec;
-    const size_t sk = (size_t)d.nx, sj = (size_t)d.nx * d.nz;
-    const size_t c = (size_t)i + sk * ((size_t)k + (size_t)d.nz * j);
-    const bool ring = i == 0 || i == d.nx - 1 || j == 0 || j == d.ny - 1;
-    float Ul = 0, Ur = 0, Vs = 0, Vn = 0, Wt = 0, Wb = 0, g = 1, gz = 1;
-    if (!ring) {
-        Ul = U[c];
-        Ur = U[c + 1];
-        Vs = V[c];
-        Vn = V[c + sj];
-        Wt = W[c];
-        Wb = k > 0 ? W[c - sk] : 0.0f;
-        g = G[c];
-        gz = Gz[c];
+    const unsigned blk = xcd_block();
+    const DomDesc &D = DD[find_dom_f(DD, nd, blk)];
+    unsigned l = blk - D.f0;
+    // the species in even groups; those of a tile share its winds in L2
+    const int sg = (int)(l % (unsigned)D.fng);
+    const int s0 = sg * D.fsb + min(sg, D.fsr), nb = D.fsb + (sg < D.fsr);
+    l /= (unsigned)D.fng;
+    const int kc = (int)(l % (unsigned)D.fnk), tile = (int)(l / (unsigned)D.fnk);
+    const int tx = tile % D.ftx, ty = tile / D.ftx;
+    const int nx = D.d.nx, ny = D.d.ny, nz = D.d.nz;
+    const int k0 = kc * D.fkch, k1 = min(nz, k0 + D.fkch);
+    const int lx = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int gi = tx * FCOLS - 1 + lx, j0 = ty * FROWS + 2 * w;  // own rows j0, j0 + 1
+    if (j0 >= ny) return;
+    const size_t sk = (size_t)nx, sj = (size_t)nx * nz;
+    const int x0 = max(0, tx * FCOLS - 1);
+    unsigned lane = (unsigned)(min(max(gi, 0), nx - 1) - x0);
+    // an offset of which nothing is known: accesses stay scalar plus offset
+    auto fresh = [&] { asm("" : "+v"(lane)); };
+    size_t rb[4];  // cell (x0, 0) of rows j0 - 1 .. j0 + 2, clamped to the domain
+#pragma unroll
+    for (int r = 0; r < 4; r++) rb[r] = (size_t)x0 + sj * (size_t)min(max(j0 - 1 + r, 0), ny - 1);
+    const bool lane_out = lx >= 1 && lx <= FCOLS && gi < nx;  // gi >= 0 there
+    const bool ring_x = gi == 0 || gi == nx - 1;
+    SpecPass p[NS];
+#pragma unroll
+    for (int b = 0; b < NS; b++) {
+        p[b] = species(D.pass[0], min(s0 + b, D.nspec - 1));
+        if (QK == QK_F32) p[b].kind0 = p[b].kindo = ICAR_ADV_STORE_F32;
     }
     const unsigned tstep = *D.step;
-    const float yg = (FD && !ring) ? recip_nr(g) : 1.0f, ygz = (FD && !ring) ? recip_nr(gz) : 1.0f;
-    // Species in groups of FSB: every load of a group is issued before the
-    // first store, so a thread keeps several species' reads in flight (the
-    // compiler cannot move loads above the stores of other species itself:
-    // the table's pointers may alias).
-    for (int s0 = 0; s0 < nspec; s0 += FSB) {
-        uint32_t rc[FSB], rw[FSB], re[FSB], rs[FSB], rn[FSB], ru[FSB], rd[FSB];
+
+    // four values of a species: the raw bits, and the values (one branch on
+    // the kind for the four)
+    auto load = [&](const SpecPass &s, const size_t (&c)[4], uint32_t (&r)[4]) {
+        fresh();
+        if (QK == QK_F32 || s.kind0 == ICAR_ADV_STORE_F32) {
 #pragma unroll
-        for (int b = 0; b < FSB; b++) {
-            rc[b] = rw[b] = re[b] = rs[b] = rn[b] = ru[b] = rd[b] = 0u;
-            if (s0 + b < nspec) {
-                SpecPass p = sp[s0 + b];
-                if (QK == QK_F32) p.kind0 = ICAR_ADV_STORE_F32;  // an FP32-only batch: no 16-bit code
-                p.kind0 = __builtin_amdgcn_readfirstlane(p.kind0);
-                rc[b] = ld_w<QK>(p.q0, c, p.kind0);
-                if (!ring) {
-                    rw[b] = ld_w<QK>(p.q0, c - 1, p.kind0);
-                    re[b] = ld_w<QK>(p.q0, c + 1, p.kind0);
-                    rs[b] = ld_w<QK>(p.q0, c - sj, p.kind0);
-                    rn[b] = ld_w<QK>(p.q0, c + sj, p.kind0);
-                    if (k < d.nz - 1) ru[b] = ld_w<QK>(p.q0, c + sk, p.kind0);
-                    if (k > 0) rd[b] = ld_w<QK>(p.q0, c - sk, p.kind0);
-                }
+            for (int e = 0; e < 4; e++) r[e] = ldq<QK_F32>(s.q0, c[e], lane, s.kind0);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; e++) r[e] = ldq<QK>(s.q0, c[e], lane, s.kind0);
+        }
+    };
+    auto convert = [&](const SpecPass &s, const uint32_t (&r)[4], float (&v)[4]) {
+        if (QK == QK_F32 || s.kind0 == ICAR_ADV_STORE_F32) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] = __uint_as_float(r[e]);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] = cvq<QK>(r[e], s.kind0, s.scale0);
+        }
+    };
+    // the level to come: raw q of rows j0 - 1 and j0 + 2 ([0], [3]) and of the
+    // own rows one level further up ([1], [2]), and the winds and divisors
+    uint32_t nq[NS][4];
+    float nU[2], nV[3], nW[2], nG[2], nZ[2];
+    auto fetch = [&](int k) {
+        if (k >= k1) return;
+        const size_t o = sk * (size_t)k, ou = sk * (size_t)min(k + 1, nz - 1);
+        const size_t c[4] = {rb[0] + o, rb[1] + ou, rb[2] + ou, rb[3] + o};
+        fresh();
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            nU[t] = ld1(D.sf.U, rb[1 + t] + o, lane);
+            nW[t] = ld1(D.sf.W, rb[1 + t] + o, lane);
+            nG[t] = ld1(D.sf.G, rb[1 + t] + o, lane);
+            nZ[t] = ld1(D.sf.Gz, rb[1 + t] + o, lane);
+        }
+#pragma unroll
+        for (int t = 0; t < 3; t++) nV[t] = ld1(D.sf.V, rb[1 + t] + o, lane);
+#pragma unroll
+        for (int b = 0; b < NS; b++)
+            if (b < nb) load(p[b], c, nq[b]);
+    };
+    // the own rows at level k0 and at the level below it, and the wind between
+    uint32_t r0[NS][4];
+    float wb[2];
+    {
+        const size_t o = sk * (size_t)k0, od = sk * (size_t)max(k0 - 1, 0);
+        const size_t c[4] = {rb[1] + o, rb[2] + o, rb[1] + od, rb[2] + od};
+        fresh();
+#pragma unroll
+        for (int t = 0; t < 2; t++) wb[t] = ld1(D.sf.W, c[2 + t], lane);
+#pragma unroll
+        for (int b = 0; b < NS; b++)
+            if (b < nb) load(p[b], c, r0[b]);
+    }
+    fetch(k0);
+    float q[NS][2], Fb[NS][2];  // the level's own values, the fluxes through the faces below
+#pragma unroll
+    for (int b = 0; b < NS; b++) {
+        float v[4] = {};
+        if (b < nb) convert(p[b], r0[b], v);
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            q[b][t] = v[t];
+            Fb[b][t] = k0 > 0 ? flux1(v[2 + t], v[t], wb[t]) : 0.0f;
+        }
+    }
+    for (int k = k0; k < k1; k++) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) asm("" : "+s"(rb[r]));  // no sums of them with every base over the loop
+        // this level's winds and values, the next level's on their way
+        float U[2], V[3], W[2], G[2], Z[2], qs[NS], qn[NS], qu[NS][2];
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            U[t] = nU[t];
+            W[t] = nW[t];
+            G[t] = nG[t];
+            Z[t] = nZ[t];
+        }
+#pragma unroll
+        for (int t = 0; t < 3; t++) V[t] = nV[t];
+#pragma unroll
+        for (int b = 0; b < NS; b++) {
+            if (b >= nb) continue;
+            float v[4];
+            convert(p[b], nq[b], v);
+            qs[b] = v[0];
+            qn[b] = v[3];
+            qu[b][0] = k + 1 < nz ? v[1] : 0.0f;
+            qu[b][1] = k + 1 < nz ? v[2] : 0.0f;
+        }
+        fetch(k + 1);
+        // flux1 with the winds' parts formed once for the species of the block
+        struct Wind {
+            float up, dn;
+            __device__ __forceinline__ explicit Wind(float u) : up(u + fabsf(u)), dn(u - fabsf(u)) {}
+            __device__ __forceinline__ float flux(float l, float r) const { return (up * l + dn * r) / 2.0f; }
+        };
+        const Wind wy[3] = {Wind(V[0]), Wind(V[1]), Wind(V[2])};
+        float xh[NS][2], xv[NS][2];
+#pragma unroll
+        for (int b = 0; b < NS; b++) {
+            if (b >= nb) continue;
+            const float fy[3] = {wy[0].flux(qs[b], q[b][0]), wy[1].flux(q[b][0], q[b][1]),
+                                 wy[2].flux(q[b][1], qn[b])};
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                const float fl = Wind(U[t]).flux(lane_prev(q[b][t]), q[b][t]), fr = lane_next(fl);
+                // the top flux is not upwinded (:96-97)
+                const float fz = k > 0 && k == nz - 1 ? q[b][t] * W[t] : Wind(W[t]).flux(q[b][t], qu[b][t]);
+                xh[b][t] = (fr - fl) + (fy[t + 1] - fy[t]);  // :86-87
+                xv[b][t] = fz - Fb[b][t];                    // :90-94
+                Fb[b][t] = fz;
             }
         }
-        float qc[FSB], qw[FSB], qe[FSB], qs[FSB], qn[FSB], qu[FSB], qd[FSB];
-#pragma unroll
-        for (int b = 0; b < FSB; b++) {
-            int kind = ICAR_ADV_STORE_F32;
-            float sc = 1.0f;
-            if (QK != QK_F32 && s0 + b < nspec) {
-                kind = __builtin_amdgcn_readfirstlane(sp[s0 + b].kind0);
-                sc = sp[s0 + b].scale0;
-            }
-            if (QK == QK_BF16) {
-                // one branch per species (the kind is uniform): FP32 words as
-                // they are, BF16 ones shifted into place and scaled
-                if (kind == ICAR_ADV_STORE_F32) {
-                    qc[b] = __uint_as_float(rc[b]);
-                    qw[b] = __uint_as_float(rw[b]);
-                    qe[b] = __uint_as_float(re[b]);
-                    qs[b] = __uint_as_float(rs[b]);
-                    qn[b] = __uint_as_float(rn[b]);
-                    qu[b] = __uint_as_float(ru[b]);
-                    qd[b] = __uint_as_float(rd[b]);
-                } else {
-                    qc[b] = __uint_as_float(rc[b] << 16) * sc;
-                    qw[b] = __uint_as_float(rw[b] << 16) * sc;
-                    qe[b] = __uint_as_float(re[b] << 16) * sc;
-                    qs[b] = __uint_as_float(rs[b] << 16) * sc;
-                    qn[b] = __uint_as_float(rn[b] << 16) * sc;
-                    qu[b] = __uint_as_float(ru[b] << 16) * sc;
-                    qd[b] = __uint_as_float(rd[b] << 16) * sc;
-                }
-                continue;
-            }
-            qc[b] = cv_w<QK>(rc[b], c, kind, sc);
-            qw[b] = cv_w<QK>(rw[b], c - 1, kind, sc);
-            qe[b] = cv_w<QK>(re[b], c + 1, kind, sc);
-            qs[b] = cv_w<QK>(rs[b], c - sj, kind, sc);
-            qn[b] = cv_w<QK>(rn[b], c + sj, kind, sc);
-            qu[b] = cv_w<QK>(ru[b], c + sk, kind, sc);
-            qd[b] = cv_w<QK>(rd[b], c - sk, kind, sc);
-        }
-        float qo[FSB];
+        float v[NS][2];
+        // The fast quotients hold for divisors in [2^-30, 2^30] and numerators
+        // that are zero or in [2^-96, 2^90]
         auto update = [&](auto fd_c) -> bool {
             constexpr bool F = decltype(fd_c)::value;
-            DivGuard gd;
+            float yG[2] = {}, yZ[2] = {}, big = 0.0f;
+            uint32_t key = 0xffffffffu;
+            bool in = true;
             if (F) {
-                guard_den(gd, g);
-                guard_den(gd, gz);
+#pragma unroll
+                for (int t = 0; t < 2; t++) {
+                    yG[t] = recip_nr(G[t]);
+                    yZ[t] = recip_nr(Z[t]);
+                }
+                in = vmin3(G[0], G[1], fminf(Z[0], Z[1])) >= 0x1p-30f &&
+                     vmax3(G[0], G[1], fmaxf(Z[0], Z[1])) <= 0x1p30f;
             }
 #pragma unroll
-            for (int b = 0; b < FSB; b++) {
-                qo[b] = qc[b];
-                if (s0 + b >= nspec || ring) continue;  // the ring is copied (:61-63)
-                const float fr = flux1(qc[b], qe[b], Ur), fl = flux1(qw[b], qc[b], Ul);
-                const float fn = flux1(qc[b], qn[b], Vn), fs = flux1(qs[b], qc[b], Vs);
-                const float xh = (fr - fl) + (fn - fs);  // :86-87
-                float xv;
-                if (k == 0)
-                    xv = flux1(qc[b], qu[b], Wt);  // :93-94
-                else if (k == d.nz - 1)
-                    xv = qc[b] * Wt - flux1(qd[b], qc[b], Wb);  // top flux not upwinded (:96-97)
-                else
-                    xv = flux1(qc[b], qu[b], Wt) - flux1(qd[b], qc[b], Wb);  // :90-91
-                if constexpr (F) {
-                    guard_num(gd, xh);
-                    guard_num(gd, xv);
-                    const float q = qc[b] - div_y(xh, g, yg);
-                    qo[b] = q - div_y(xv, gz, ygz);
-                } else {
-                    const float q = qc[b] - xh / g;
-                    qo[b] = q - xv / gz;
+            for (int b = 0; b < NS; b++) {
+                if (b >= nb) continue;
+#pragma unroll
+                for (int t = 0; t < 2; t++) {
+                    const float x = q[b][t] - fdiv_y<F>(xh[b][t], G[t], yG[t]);
+                    v[b][t] = x - fdiv_y<F>(xv[b][t], Z[t], yZ[t]);
+                    if (F) {
+                        key = min(key, min(nz_key(xh[b][t]), nz_key(xv[b][t])));
+                        big = vmax3a(big, xh[b][t], xv[b][t]);
+                    }
                 }
             }
-            return guard_ok(gd);
+            return in && key >= ((127u - 96u) << 24) - 1u && big <= 0x1p90f;
         };
-        if (!FD || __any(!update(std::integral_constant<bool, true>{})))
+        if (!fast || !__all(update(std::integral_constant<bool, true>{})))
             update(std::integral_constant<bool, false>{});
 #pragma unroll
-        for (int b = 0; b < FSB; b++) {
-            const int s = s0 + b;
-            if (s >= nspec) continue;
-            SpecPass p = sp[s];
-            if (QK == QK_F32) p.kindo = ICAR_ADV_STORE_F32;
-            p.kindo = __builtin_amdgcn_readfirstlane(p.kindo);
-            const uint32_t rnd = is_sr(p.kindo) ? sr_bits((uint32_t)c, s, tstep) : 0u;
-            st_w<QK>(p.out, c, p.kindo, p.inv_scaleo, qo[b], rnd);
+        for (int b = 0; b < NS; b++) {
+            if (b >= nb) continue;
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                const int j = j0 + t;
+                const float r = ring_x || j == 0 || j == ny - 1 ? q[b][t] : v[b][t];  // the ring is copied (:61-63)
+                if (lane_out && j < ny) {
+                    const size_t c = rb[1 + t] + sk * (size_t)k;
+                    fresh();
+                    const uint32_t rnd = is_sr(p[b].kindo) ? sr_bits((uint32_t)c + lane, s0 + b, tstep) : 0u;
+                    stq<QK>(p[b].out, c, lane, p[b].kindo, p[b].inv_scaleo, r, rnd);
+                }
+                q[b][t] = qu[b][t];
+            }
         }
     }
 }
@@ -667,82 +786,6 @@ __device__ __forceinline__ float divergence_compensated(float q1, float fl, floa
     const float t = two_sum(q1, -dh, e1);
     const float u = two_sum(t, -dz, e2);
     return u + ((e1 + e2) - (ch + cz));
-}
-
-// Maxima and minima of values that come from memory.  fmaxf on such a value
-// first quiets a possible signalling NaN with an instruction of its own; the
-// hardware's max and min ignore quiet NaNs as fmaxf does.
-__device__ __forceinline__ float vmax(float a, float b)
-{
-    float r;
-    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
-__device__ __forceinline__ float vmin(float a, float b)
-{
-    float r;
-    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
-__device__ __forceinline__ float vmax3(float a, float b, float c)
-{
-    float r;
-    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
-}
-__device__ __forceinline__ float vmin3(float a, float b, float c)
-{
-    float r;
-    asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
-}
-// max(0, a), min(0, a), and min(1, a, b)
-__device__ __forceinline__ float vpos(float a)
-{
-    float r;
-    asm("v_max_f32 %0, 0, %1" : "=v"(r) : "v"(a));
-    return r;
-}
-__device__ __forceinline__ float vneg(float a)
-{
-    float r;
-    asm("v_min_f32 %0, 0, %1" : "=v"(r) : "v"(a));
-    return r;
-}
-__device__ __forceinline__ float vmin1(float a, float b)
-{
-    float r;
-    asm("v_min3_f32 %0, 1.0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
-
-// the value of the next lane (lane 63: 0) and of the previous lane (lane 0:
-// 0): one move within the wave, no LDS
-__device__ __forceinline__ float lane_next(float v)
-{
-    const int b = __float_as_int(v);
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, b, 0x130, 0xf, 0xf, true));  // wave_shl:1
-}
-__device__ __forceinline__ float lane_prev(float v)
-{
-    const int b = __float_as_int(v);
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, b, 0x138, 0xf, 0xf, true));  // wave_shr:1
-}
-
-// x/d: the IEEE division, or (F) the three-operation quotient of fdiv.hpp
-template <bool F>
-__device__ __forceinline__ float fdiv(float x, float d)
-{
-    if constexpr (F) return div_y(x, d, recip_nr(d));
-    else return x / d;
-}
-
-// the same with y = recip_nr(d) computed once for several numerators
-template <bool F>
-__device__ __forceinline__ float fdiv_y(float x, float d, float y)
-{
-    if constexpr (F) return div_y(x, d, y);
-    else return x / d;
 }
 
 // A face velocity u limited by the betas of the cells on its positive (p)
@@ -845,7 +888,7 @@ __global__ void __launch_bounds__((Tile<TJ, RW>::CNT))
     const bool has_x = w < 4;     // this wave stages a halo row as well
     const int rx = w < 2 ? w : TJ + w;  // rows 0, 1, TJ+2, TJ+3
 
-    SpecPass p = uniform(D.pass[pass - 1][s]);
+    SpecPass p = species(D.pass[pass - 1], s);
     if (QK == QK_F32) p.kind0 = p.kindo = ICAR_ADV_STORE_F32;  // an FP32-only batch: no 16-bit code
     const bool same = p.q1 == nullptr;
     const unsigned tstep = is_sr(p.kindo) ? *D.step : 0u;
@@ -865,27 +908,15 @@ __global__ void __launch_bounds__((Tile<TJ, RW>::CNT))
     size_t ra[RW];
 #pragma unroll
     for (int t = 0; t < RW; t++) ra[t] = row_at(r0 + t);
-    size_t rax = uniform_word(row_at(has_x ? rx : r0));
-    typedef __attribute__((address_space(1))) const char gcchar;
-    typedef __attribute__((address_space(1))) char gchar;
+    size_t rax = row_at(has_x ? rx : r0);
     typedef float f4 __attribute__((ext_vector_type(4)));
     typedef __attribute__((address_space(1))) const f4 gcf4;
-    auto ld1 = [&](const float *b, size_t c) -> float {
-        return *(gcfloat *)((gcchar *)(gcfloat *)(b + c) + lo * 4u);
-    };
+    auto ld1 = [&](const float *b, size_t c) -> float { return icaradv::ld1(b, c, lo); };
     auto ld4 = [&](const float *b, size_t c) -> f4 {
         return *(gcf4 *)((gcchar *)(gcfloat *)(b + 4 * c) + lo * 16u);
     };
-    auto ldq = [&](size_t c) -> uint32_t {  // raw bits of q0
-        if (QK == QK_F32 || p.kind0 == ICAR_ADV_STORE_F32)
-            return *(gcu32 *)((gcchar *)(gcfloat *)((const float *)p.q0 + c) + lo * 4u);
-        return *(gcu16 *)((gcchar *)(gcu16 *)((const uint16_t *)p.q0 + c) + lo * 2u);
-    };
-    auto cvq = [&](uint32_t b) -> float {
-        if (QK == QK_F32 || p.kind0 == ICAR_ADV_STORE_F32) return __uint_as_float(b);
-        if (QK == QK_BF16 || is_bf16(p.kind0)) return __uint_as_float(b << 16) * p.scale0;
-        return __half2float(__ushort_as_half((uint16_t)b)) * p.scale0;
-    };
+    auto ldq = [&](size_t c) -> uint32_t { return icaradv::ldq<QK>(p.q0, c, lo, p.kind0); };
+    auto cvq = [&](uint32_t b) -> float { return icaradv::cvq<QK>(b, p.kind0, p.scale0); };
 
     // LDS planes of CY rows of 64 floats (a wave reads one row, lane i at
     // word i, so no bank conflicts)
@@ -1327,10 +1358,7 @@ __global__ void __launch_bounds__((Tile<TJ, RW>::CNT))
                     const size_t c = ra[t] + sk * (size_t)L2;
                     fresh();
                     const uint32_t rnd = is_sr(p.kindo) ? sr_bits((uint32_t)c + lo, s, tstep) : 0u;
-                    if (QK == QK_F32 || p.kindo == ICAR_ADV_STORE_F32)
-                        *(gfloat *)((gchar *)(gfloat *)((float *)p.out + c) + lo * 4u) = q;
-                    else
-                        *(gu16 *)((gchar *)(gu16 *)((uint16_t *)p.out + c) + lo * 2u) = q16_of<QK>(q, p.kindo, p.inv_scaleo, rnd);
+                    stq<QK>(p.out, c, lo, p.kindo, p.inv_scaleo, q, rnd);
                 }
             }
         }
@@ -1393,7 +1421,8 @@ struct FastBatch {
     DomDesc *d_desc = nullptr;           // [2 parities][n]
     std::vector<DomDesc> h_desc[2];
     std::vector<float> dts;              // dt values in the device tables
-    unsigned total_cb = 0, total_work = 0;
+    unsigned total_cb = 0, total_fb = 0, total_work = 0;
+    int fns = 4;         // most species of a block of the donor-cell kernel
     double cells = 0, cell_species = 0;  // for the algorithmic byte counts
     int corr_cfg = 3;    // corrective kernel's tile (launch_corr_t)
     int tj = 16;         // output rows per corrective tile (tile_rows(corr_cfg))
@@ -1652,21 +1681,9 @@ void launch_corr_q(const FastBatch *b, unsigned nb, hipStream_t s, const DomDesc
 
 int tile_rows(int cfg) { return (cfg & 4) ? 8 : 16; }
 
-// ICAR_ADV_FAST_DIV=1 takes the guarded three-operation quotient of fdiv.hpp
-// in the corrective and donor-cell kernels (the same results).  Off by
-// default: its range guard costs about what the cheaper quotient saves.
-bool fast_division()
-{
-    static const bool on = [] {
-        const char *e = getenv("ICAR_ADV_FAST_DIV");
-        return e && atoi(e) != 0;
-    }();
-    return on;
-}
-
-// ICAR_ADV_FAST_DIV=0 makes the corrective kernel divide by the IEEE sequence
-// throughout (the same results)
-int corr_fast_division()
+// ICAR_ADV_FAST_DIV=0 makes the donor-cell and corrective kernels divide by the
+// IEEE sequence throughout (the same results)
+int fast_division()
 {
     static const int on = [] {
         const char *e = getenv("ICAR_ADV_FAST_DIV");
@@ -1679,7 +1696,7 @@ void launch_corr(const FastBatch *b, hipStream_t s, const DomDesc *D, int n, int
 {
     const unsigned nw = b->total_work;
     const unsigned nb = (nw + 7) / 8 * 8;
-    const int fast = corr_fast_division();
+    const int fast = fast_division();
     if (b->fct) launch_corr_q<true>(b, nb, s, D, n, pass, nw, cfg, fast);
     else launch_corr_q<false>(b, nb, s, D, n, pass, nw, cfg, fast);
 }
@@ -1687,6 +1704,46 @@ void launch_corr(const FastBatch *b, hipStream_t s, const DomDesc *D, int n, int
 // Tuned configurations by batch shape, shared by every batch of the process.
 std::mutex g_tune_mu;
 std::map<std::string, std::pair<int, int>> g_tuned;
+
+// The donor-cell kernel's blocks: columns of four species where those fill the
+// GPU, else of two species and in as many level chunks as it takes (a chunk
+// loads one level more).
+void set_first_blocks(FastBatch *b)
+{
+    constexpr int FILL = 1024;  // four blocks per CU
+    auto groups = [&](size_t k) { return ((int)b->doms[k].st->sp.size() + b->fns - 1) / b->fns; };
+    auto tiles = [&](size_t k) {
+        const Dims &d = b->doms[k].st->d;
+        return ((d.nx + FCOLS - 1) / FCOLS) * ((d.ny + FROWS - 1) / FROWS);
+    };
+    auto columns = [&] {
+        long long n = 0;
+        for (size_t k = 0; k < b->doms.size(); k++) n += (long long)tiles(k) * groups(k);
+        return n;
+    };
+    b->fns = 4;
+    if (columns() < FILL / 2) b->fns = 2;
+    const long long chunks = (FILL + columns() - 1) / columns();
+    unsigned f = 0;
+    for (size_t k = 0; k < b->doms.size(); k++) {
+        const Dims &d = b->doms[k].st->d;
+        const int S = (int)b->doms[k].st->sp.size(), ng = groups(k);
+        const int kch = chunks >= d.nz ? 1 : (int)((d.nz + chunks - 1) / chunks);
+        const int nk = (d.nz + kch - 1) / kch;
+        for (int par = 0; par < 2; par++) {
+            DomDesc &E = b->h_desc[par][k];
+            E.f0 = f;
+            E.ftx = (d.nx + FCOLS - 1) / FCOLS;
+            E.fnk = nk;
+            E.fkch = kch;
+            E.fng = ng;
+            E.fsb = S / ng;
+            E.fsr = S % ng;
+        }
+        f += (unsigned)(tiles(k) * nk * ng);
+    }
+    b->total_fb = f;
+}
 
 std::string tune_key(const FastBatch *b)
 {
@@ -1713,21 +1770,17 @@ void launch_coef(const FastBatch *b, hipStream_t s, const DomDesc *D, int n)
 
 void launch_first(const FastBatch *b, hipStream_t s, const DomDesc *D, int n)
 {
-    const bool fd = fast_division();
-    const dim3 g(b->total_cb), t(FBX, FBY);
+    const int fast = fast_division();
+    auto go = [&](auto qk) {
+        if (b->fns == 4)
+            hipLaunchKernelGGL((k_first<qk.value, 4>), dim3(b->total_fb), dim3(64 * FWAVES), 0, s, D, n, fast);
+        else
+            hipLaunchKernelGGL((k_first<qk.value, 2>), dim3(b->total_fb), dim3(64 * FWAVES), 0, s, D, n, fast);
+    };
     switch (storage_class(b)) {
-    case QK_F32:
-        if (fd) hipLaunchKernelGGL((k_first<QK_F32, true>), g, t, 0, s, D, n);
-        else hipLaunchKernelGGL((k_first<QK_F32, false>), g, t, 0, s, D, n);
-        break;
-    case QK_BF16:
-        if (fd) hipLaunchKernelGGL((k_first<QK_BF16, true>), g, t, 0, s, D, n);
-        else hipLaunchKernelGGL((k_first<QK_BF16, false>), g, t, 0, s, D, n);
-        break;
-    default:
-        if (fd) hipLaunchKernelGGL((k_first<QK_ANY, true>), g, t, 0, s, D, n);
-        else hipLaunchKernelGGL((k_first<QK_ANY, false>), g, t, 0, s, D, n);
-        break;
+    case QK_F32: go(std::integral_constant<int, QK_F32>{}); break;
+    case QK_BF16: go(std::integral_constant<int, QK_BF16>{}); break;
+    default: go(std::integral_constant<int, QK_ANY>{}); break;
     }
 }
 
@@ -1924,6 +1977,7 @@ FastBatch *fast_batch_create(const FastDomain *doms, int n, int order, int fct, 
         }
     }
     b->total_cb = cb;
+    set_first_blocks(b);
     set_ksplit(b, b->nks);
     if (hipMalloc(&b->d_desc, 2 * (size_t)n * sizeof(DomDesc)) != hipSuccess) {
         *err = "hipMalloc of the domain table failed";
@@ -2052,7 +2106,7 @@ __global__ void k_unpack(size_t n, const uint16_t *__restrict__ src, float *__re
 {
     for (size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x; p < n;
          p += (size_t)gridDim.x * blockDim.x)
-        dst[p] = ld_q(src, p, storage, scale);
+        dst[p] = cvq<QK_ANY>(ldq<QK_ANY>(src, p, 0u, storage), storage, scale);
 }
 
 }  // namespace
