@@ -5,7 +5,7 @@
 //                 horz_only, :201-234) and w integrated up each column so
 //                 that it balances (calc_w, :166-199).  One thread per
 //                 column, threads along i (coalesced rows), the level below
-//                 carried in registers.
+//                 carried in registers, a few levels' loads in flight.
 //   k_dt_partials compute_dt (src/main/time_step.f90:51-168) with
 //                 use_density=.false.: per block the maxima of |u|, |v|, |w|
 //                 over the whole arrays and of the tile's per-cell Courant
@@ -25,80 +25,86 @@ namespace icaradv {
 
 namespace {
 
-// u_met of x face fi (0..nx) of row (k, j), wind.f90:222-228
-__device__ __forceinline__ float u_met(const Dims &d, int fi, int k, int j, int adv_den,
-                                       const float *__restrict__ u, const float *__restrict__ ju,
-                                       const float *__restrict__ rho)
+// u_met and v_met of a face (wind.f90:222-228) from the wind, its Jacobian and
+// the density of the cells on both sides; at the domain's edge (e) from the
+// cell next to it (a) and the one behind that (b).
+template <bool RHO>
+__device__ __forceinline__ float met(float u, float ju, float a, float b, bool e)
 {
-    const size_t f = (size_t)fi + (size_t)(d.nx + 1) * ((size_t)k + (size_t)d.nz * j);
-    if (!adv_den) return u[f] * ju[f];
-    const size_t c = ix(d, 0, k, j);
-    if (fi == 0) return u[f] * ju[f] * (1.5f * rho[c] - 0.5f * rho[c + 1]);
-    if (fi == d.nx) return u[f] * ju[f] * (1.5f * rho[c + d.nx - 1] - 0.5f * rho[c + d.nx - 2]);
-    return u[f] * ju[f] * (rho[c + fi - 1] + rho[c + fi]) / 2.0f;
+    if (!RHO) return u * ju;
+    return e ? u * ju * (1.5f * a - 0.5f * b) : u * ju * (a + b) / 2.0f;
 }
 
-// v_met of y face fj (0..ny) of column (i, k), wind.f90:225-227
-__device__ __forceinline__ float v_met(const Dims &d, int i, int k, int fj, int adv_den,
-                                       const float *__restrict__ v, const float *__restrict__ jv,
-                                       const float *__restrict__ rho)
-{
-    const size_t f = ix(d, i, k, fj);
-    if (!adv_den) return v[f] * jv[f];
-    const size_t sj = (size_t)d.nx * d.nz;
-    const size_t c0 = ix(d, i, k, 0);
-    if (fj == 0) return v[f] * jv[f] * (1.5f * rho[c0] - 0.5f * rho[c0 + sj]);
-    if (fj == d.ny)
-        return v[f] * jv[f] * (1.5f * rho[c0 + (d.ny - 1) * sj] - 0.5f * rho[c0 + (d.ny - 2) * sj]);
-    return v[f] * jv[f] * (rho[f - sj] + rho[f]) / 2.0f;
-}
+// Only the balance itself runs up the column; what it takes from a level (its
+// divergence and divisor) does not depend on the level below, so LB levels'
+// loads are issued together.  With a level at a time the column's 3 waves per
+// SIMD waited for memory at every level: 517 x 389 x 40 0.212 ms, now 0.115 ms
+// (258 MB, 0.055 ms at the rate of a copy).
+constexpr int LB = 4;
 
+template <bool RHO>
 __global__ void __launch_bounds__(256)
-    k_balance_w(Dims d, int i_s, int i_e, int j_s, int j_e, float dx, int adv_den, DomainFields f,
+    k_balance_w(Dims d, int i_s, int i_e, int j_s, int j_e, float dx, DomainFields f,
                 float *__restrict__ w)
 {
     const int i = blockIdx.x * 64 + threadIdx.x;
     const int j = blockIdx.y * 4 + threadIdx.y;
     if (i >= d.nx || j >= d.ny) return;
-    const size_t sk = (size_t)d.nx;
+    const size_t sk = (size_t)d.nx, sj = (size_t)d.nx * d.nz;
     const size_t c0 = ix(d, i, 0, j);
     if (i < i_s || i > i_e || j < j_s || j > j_e) {  // w = 0 outside the balanced columns (:179)
         for (int k = 0; k < d.nz; k++) w[c0 + sk * k] = 0.0f;
         return;
     }
-    const float *__restrict__ rho = f.density;
-    const float *__restrict__ dz = f.dz;
-    const float *__restrict__ jw = f.jaco_w;
+    const float *__restrict__ rho = f.density, *__restrict__ dz = f.dz, *__restrict__ jw = f.jaco_w;
+    const float *__restrict__ u = f.u, *__restrict__ ju = f.jaco_u;
+    const float *__restrict__ v = f.v, *__restrict__ jv = f.jaco_v;
+    const bool west = i == 0, east = i == d.nx - 1, south = j == 0, north = j == d.ny - 1;
     float wb = 0.0f, rib = 0.0f, jwb = 0.0f;  // w, rho_i and jacobian_w of the level below
-    for (int k = 0; k < d.nz; k++) {
-        const size_t c = c0 + sk * k;
-        const float dU = u_met(d, i + 1, k, j, adv_den, f.u, f.jaco_u, rho) -
-                         u_met(d, i, k, j, adv_den, f.u, f.jaco_u, rho);
-        const float dV = v_met(d, i, k, j + 1, adv_den, f.v, f.jaco_v, rho) -
-                         v_met(d, i, k, j, adv_den, f.v, f.jaco_v, rho);
-        const float div = (dU + dV) / dx;  // :232
-        float wc;
-        if (adv_den) {
+    for (int k0 = 0; k0 < d.nz; k0 += LB) {
+        float dd[LB], den[LB], ri[LB], jl[LB];  // divergence * dz, divisor, rho_i, jacobian_w
+#pragma unroll
+        for (int b = 0; b < LB; b++) {
+            const int k = min(k0 + b, d.nz - 1);  // past the top: the top again, not used
+            const size_t c = c0 + sk * k;
+            const size_t fu = (size_t)i + (size_t)(d.nx + 1) * ((size_t)k + (size_t)d.nz * j);
+            float rc = 0.0f, rw = 0.0f, re = 0.0f, rs = 0.0f, rn = 0.0f, ru = 0.0f, dzu = 0.0f;
+            if (RHO) {
+                const size_t cu = k < d.nz - 1 ? c + sk : c;
+                rc = rho[c];
+                rw = rho[west ? c + 1 : c - 1];
+                re = rho[east ? c - 1 : c + 1];
+                rs = rho[south ? c + sj : c - sj];
+                rn = rho[north ? c - sj : c + sj];
+                ru = rho[cu];
+                dzu = dz[cu];
+            }
+            const float dzc = dz[c];
+            // the west and south faces' cells in the order of the sum
+            const float dU = met<RHO>(u[fu + 1], ju[fu + 1], rc, re, east) -
+                             met<RHO>(u[fu], ju[fu], west ? rc : rw, west ? rw : rc, west);
+            const float dV = met<RHO>(v[c + sj], jv[c + sj], rc, rn, north) -
+                             met<RHO>(v[c], jv[c], south ? rc : rs, south ? rs : rc, south);
+            dd[b] = (dU + dV) / dx * dzc;  // :232
+            jl[b] = jw[c];
             // rho_i(k) = (rho(k)dz(k) + rho(k+1)dz(k+1)) / (dz(k)+dz(k+1)), :177
-            const float ri = (k < d.nz - 1)
-                                 ? (rho[c] * dz[c] + rho[c + sk] * dz[c + sk]) / (dz[c] + dz[c + sk])
-                                 : 0.0f;
-            if (k == 0)
-                wc = 0.0f - div * dz[c] / (jw[c] * ri);                           // :183-184
-            else if (k == d.nz - 1)
-                wc = ((wb * rib * jwb) - div * dz[c]) / (jw[c] * rho[c]);          // :185-188
-            else
-                wc = ((wb * rib * jwb) - div * dz[c]) / (jw[c] * ri);              // :189-192
-            rib = ri;
-        } else {
-            if (k == 0)
-                wc = (0.0f - div * dz[c]) / (jw[c]);                               // :195
-            else
-                wc = (wb * jwb - div * dz[c]) / (jw[c]);                           // :197-198
+            ri[b] = RHO && k < d.nz - 1 ? (rc * dzc + ru * dzu) / (dzc + dzu) : 0.0f;
+            den[b] = RHO ? jl[b] * (k < d.nz - 1 ? ri[b] : rc) : jl[b];  // :183-192, :195-198
         }
-        w[c] = wc;
-        wb = wc;
-        jwb = jw[c];
+#pragma unroll
+        for (int b = 0; b < LB; b++) {
+            const int k = k0 + b;
+            if (k >= d.nz) break;
+            float wc;
+            if (RHO)
+                wc = k == 0 ? 0.0f - dd[b] / den[b] : ((wb * rib * jwb) - dd[b]) / den[b];
+            else
+                wc = ((k == 0 ? 0.0f : wb * jwb) - dd[b]) / den[b];
+            w[c0 + sk * k] = wc;
+            wb = wc;
+            rib = ri[b];
+            jwb = jl[b];
+        }
     }
 }
 
@@ -117,35 +123,45 @@ __device__ __forceinline__ float block_max(float v, float *sm)
     return r;
 }
 
+// A wave takes the rows (k, j) of the grid in turn, 64 columns at a time: the
+// arrays' maxima and the tile's Courant rates from one set of loads, without
+// an integer division per cell.  517 x 389 x 40: 0.074 -> 0.034 ms (the three
+// winds are 97 MB, 0.021 ms at the rate of a copy).
 __global__ void __launch_bounds__(DT_THREADS)
     k_dt_partials(Dims d, int its, int ite, int jts, int jte, float dx, const float *__restrict__ u,
                   const float *__restrict__ v, const float *__restrict__ w,
                   const float *__restrict__ dzl, float *__restrict__ part)
 {
     __shared__ float sm[DT_THREADS];
-    const size_t stride = (size_t)gridDim.x * DT_THREADS;
-    const size_t t0 = (size_t)blockIdx.x * DT_THREADS + threadIdx.x;
-    const size_t nu = (size_t)(d.nx + 1) * d.nz * d.ny, nv = (size_t)d.nx * d.nz * (d.ny + 1);
-    const size_t nw = (size_t)d.nx * d.nz * d.ny;
+    const int lane = threadIdx.x & 63;
+    const long long wave = (long long)blockIdx.x * (DT_THREADS / 64) +
+                           __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const long long waves = (long long)gridDim.x * (DT_THREADS / 64), rows = (long long)d.nz * (d.ny + 1);
     float mu = 0.0f, mv = 0.0f, mw = 0.0f, m3 = 0.0f;
-    for (size_t p = t0; p < nu; p += stride) mu = fmaxf(mu, fabsf(u[p]));
-    for (size_t p = t0; p < nv; p += stride) mv = fmaxf(mv, fabsf(v[p]));
-    for (size_t p = t0; p < nw; p += stride) mw = fmaxf(mw, fabsf(w[p]));
-    // the tile, :101-126: i fastest so that neighbouring threads read a row
-    const int ti = ite - its + 1, tj = jte - jts + 1;
-    const size_t nt = (size_t)ti * d.nz * tj;
-    for (size_t p = t0; p < nt; p += stride) {
-        const int i = its + (int)(p % (size_t)ti);
-        const size_t r = p / (size_t)ti;
-        const int k = (int)(r % (size_t)d.nz);
-        const int j = jts + (int)(r / (size_t)d.nz);
-        const size_t fu = (size_t)i + (size_t)(d.nx + 1) * ((size_t)k + (size_t)d.nz * j);
-        const size_t c = ix(d, i, k, j);
-        const size_t cb = k == 0 ? c : c - (size_t)d.nx;  // zoffset, :104-108
-        const float a = fmaxf(fabsf(u[fu]), fabsf(u[fu + 1])) / dx;
-        const float b = fmaxf(fabsf(v[c]), fabsf(v[c + (size_t)d.nx * d.nz])) / dx;
-        const float e = fmaxf(fabsf(w[c]), fabsf(w[cb])) / dzl[k];
-        m3 = fmaxf(m3, fmaxf(fmaxf(a, b), e));
+    for (long long r = wave; r < rows; r += waves) {  // row ny: the last y faces only
+        const int j = (int)(r / d.nz), k = (int)(r % d.nz);
+        const size_t c0 = ix(d, 0, k, j), sj = (size_t)d.nx * d.nz;
+        const size_t u0 = (size_t)(d.nx + 1) * ((size_t)k + (size_t)d.nz * j);
+        const size_t cb0 = k == 0 ? c0 : c0 - (size_t)d.nx;  // zoffset, :104-108
+        if (j == d.ny) {
+            for (int i = lane; i < d.nx; i += 64) mv = fmaxf(mv, fabsf(v[c0 + i]));
+            continue;
+        }
+        const bool tile = j >= jts && j <= jte;
+        const float dzk = dzl[k];
+#pragma unroll 4
+        for (int i = lane; i < d.nx; i += 64) {
+            const float uc = fabsf(u[u0 + i]), ue = fabsf(u[u0 + i + 1]);
+            const float vc = fabsf(v[c0 + i]), vn = fabsf(v[c0 + sj + i]);
+            const float wc = fabsf(w[c0 + i]), wd = fabsf(w[cb0 + i]);
+            mu = fmaxf(mu, fmaxf(uc, ue));
+            mv = fmaxf(mv, vc);
+            mw = fmaxf(mw, wc);
+            const float a = fmaxf(uc, ue) / dx;  // :101-126
+            const float b = fmaxf(vc, vn) / dx;
+            const float e = fmaxf(wc, wd) / dzk;
+            if (tile && i >= its && i <= ite) m3 = fmaxf(m3, fmaxf(fmaxf(a, b), e));
+        }
     }
     mu = block_max(mu, sm);
     mv = block_max(mv, sm);
@@ -164,8 +180,11 @@ __global__ void __launch_bounds__(DT_THREADS)
 void launch_balance_w(hipStream_t s, Dims d, int i_s, int i_e, int j_s, int j_e, float dx,
                       int adv_den, const DomainFields &f, float *w)
 {
-    hipLaunchKernelGGL(k_balance_w, dim3((d.nx + 63) / 64, (d.ny + 3) / 4), dim3(64, 4), 0, s, d,
-                       i_s, i_e, j_s, j_e, dx, adv_den, f, w);
+    const dim3 g((d.nx + 63) / 64, (d.ny + 3) / 4), t(64, 4);
+    if (adv_den)
+        hipLaunchKernelGGL(k_balance_w<true>, g, t, 0, s, d, i_s, i_e, j_s, j_e, dx, f, w);
+    else
+        hipLaunchKernelGGL(k_balance_w<false>, g, t, 0, s, d, i_s, i_e, j_s, j_e, dx, f, w);
 }
 
 int dt_partial_blocks() { return DT_BLOCKS; }
@@ -190,20 +209,28 @@ namespace {
 // double precision in the reference (dt%seconds()), so the tendency and the
 // relaxation term are formed in FP64 and rounded to FP32 on assignment, as
 // the Fortran does; forcing - value is an FP32 difference.
+// A wave takes the rows (k, j) in turn, so no cell needs an integer division:
+// 517 x 389 x 40 0.046 -> 0.040 ms.
 __global__ void __launch_bounds__(256)
     k_forcing(Dims d, double dt, const float *__restrict__ filt, float *__restrict__ q,
               float *__restrict__ fhi, const float *__restrict__ dqdt)
 {
-    const size_t n = (size_t)d.nx * d.nz * d.ny;
-    for (size_t c = (size_t)blockIdx.x * 256 + threadIdx.x; c < n; c += (size_t)gridDim.x * 256) {
-        const float f = (float)((double)fhi[c] + ((double)dqdt[c] * dt));
-        fhi[c] = f;
-        const size_t i = c % (size_t)d.nx, j = c / ((size_t)d.nx * d.nz);
-        const float rf = filt[j * (size_t)d.nx + i];
-        if (rf == 1.0f)
-            q[c] = f;
-        else if (rf < 1.0f)
-            q[c] = (float)((double)q[c] + ((double)rf * dt / 3600.0) * (double)(f - q[c]));
+    const int lane = threadIdx.x & 63;
+    const long long rows = (long long)d.nz * d.ny;
+    for (long long r = (long long)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+         r < rows; r += (long long)gridDim.x * 4) {
+        const size_t c0 = (size_t)r * d.nx, f0 = (size_t)(r / d.nz) * d.nx;
+#pragma unroll 4
+        for (int i = lane; i < d.nx; i += 64) {
+            const size_t c = c0 + i;
+            const float f = (float)((double)fhi[c] + ((double)dqdt[c] * dt));
+            fhi[c] = f;
+            const float rf = filt[f0 + i];
+            if (rf == 1.0f)
+                q[c] = f;
+            else if (rf < 1.0f)
+                q[c] = (float)((double)q[c] + ((double)rf * dt / 3600.0) * (double)(f - q[c]));
+        }
     }
 }
 
@@ -212,8 +239,7 @@ __global__ void __launch_bounds__(256)
 void launch_forcing(hipStream_t s, Dims d, double dt, const float *filt, float *q, float *fhi,
                     const float *dqdt)
 {
-    const size_t n = (size_t)d.nx * d.nz * d.ny;
-    size_t blocks = (n + 255) / 256;
+    size_t blocks = ((size_t)d.nz * d.ny + 3) / 4;
     if (blocks > 65536) blocks = 65536;
     hipLaunchKernelGGL(k_forcing, dim3((unsigned)blocks), dim3(256), 0, s, d, dt, filt, q, fhi,
                        dqdt);
