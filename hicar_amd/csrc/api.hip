@@ -142,6 +142,7 @@ struct Handle {
     float *host_field[ICAR_ADV_NFIELDS] = {};
     float *dev_field[ICAR_ADV_NFIELDS] = {};
     StepFields sf{};
+    PlainState *plain = nullptr;  // kernel_variant 0
     float *q2 = nullptr, *u2 = nullptr, *v2 = nullptr, *w2 = nullptr;
     float *u2l = nullptr, *v2l = nullptr, *w2l = nullptr;
     float *stage = nullptr;  // FP32 staging for reduced-precision species
@@ -351,6 +352,7 @@ void free_all(Handle *h)
     if (h->gexec) (void)hipGraphExecDestroy(h->gexec);
     fast_batch_destroy(h->batch);
     fast_destroy(h->fast);
+    plain_destroy(h->plain);
     if (h->stream) (void)hipStreamDestroy(h->stream);
     delete h;
 }
@@ -409,7 +411,8 @@ SpeciesList species_list(Handle *h)
     return l;
 }
 
-// One species through mpdata_advect3d with the exact kernels.
+// One species through mpdata_advect3d with a kernel per subroutine of the
+// reference, for handles whose memory does not hold the fused passes' buffers.
 int advect_species_exact(Handle *h, float *q)
 {
     const Dims d = h->d;
@@ -444,6 +447,47 @@ int advect_species_exact(Handle *h, float *q)
         } else if (iord == 1) {
             timed(h, K_COPY, 2 * 4 * n, [&] { launch_copy(h->stream, h->N, h->q2, q); });
         }
+    }
+    HIPCHK(h, hipGetLastError());
+    return 0;
+}
+
+int plain_ready(Handle *h)
+{
+    std::vector<float *> q;
+    for (int s = 0; s < h->nspecies; s++) {
+        if (!h->sp[s].bound) continue;
+        float *p = nullptr;
+        const int rc = species_f32_ptr(h, s, &p);
+        if (rc) return rc;
+        q.push_back(p);
+    }
+    std::string e;
+    const int rc = plain_prepare(h->plain, h->stream, q, domain_fields(h), h->sf, &e);
+    return rc ? set_err(h, rc, "%s", e.c_str()) : 0;
+}
+
+// Every species through its passes, a launch per pass and species.
+int advect_plain(Handle *h, bool winds)
+{
+    const int rc = plain_ready(h);
+    if (rc) return rc;
+    const int order = h->o.mpdata_order;
+    const double n = cells(h);
+    if (winds && order > 1)
+        timed(h, K_COEF, (4.0 + 12.0) * 4 * n, [&] { plain_coef(h->plain, h->stream); });
+    for (int s = 0, k = 0; s < h->nspecies; s++) {
+        if (!h->sp[s].bound) continue;
+        for (int pass = 1; pass <= order; pass++) {
+            const double bytes = (pass == 1 ? 5.0 + 2.0 : pass == 2 ? 15.0 + 3.0 : 15.0 + 2.0) * 4 * n;
+            timed(h, pass == 1 ? K_FUSED_FIRST : K_FUSED_CORR, bytes,
+                  [&] { plain_pass(h->plain, h->stream, k, pass); });
+        }
+        if (order == 1)
+            timed(h, K_COPY, 2 * 4 * n, [&] {
+                launch_copy(h->stream, h->N, plain_result(h->plain), static_cast<float *>(h->sp[s].dev));
+            });
+        k++;
     }
     HIPCHK(h, hipGetLastError());
     return 0;
@@ -661,6 +705,7 @@ int do_advect(Handle *h, float dt, bool winds = true)
         if (rc) return rc;
     }
     if (h->o.rk3) return 0;  // advection_driver.f90:112-115
+    if (h->plain) return advect_plain(h, winds);
     for (int s = 0; s < h->nspecies; s++) {
         if (!h->sp[s].bound) continue;
         float *q = nullptr;
@@ -1026,6 +1071,9 @@ int icar_adv_create(const icar_adv_grid *grid, const icar_adv_opts *opts, void *
                 free_all(h);
                 return set_err(nullptr, ICAR_ADV_ENOMEM, "%s", m.c_str());
             }
+    } else if (h->o.kernel_variant == 0 && !h->o.rk3 && h->o.mpdata_order >= 1 &&
+               (h->plain = plain_create(h->d, h->o.mpdata_order, h->o.mpdata_fct))) {
+        // the passes one species at a time
     } else if (h->o.kernel_variant == 0) {
         float **work[] = {&h->q2, &h->u2, &h->v2, &h->w2, &h->u2l, &h->v2l, &h->w2l};
         for (float **p : work)
@@ -1878,6 +1926,9 @@ int icar_adv_run(void *handle, float dt, int nsteps, int bc_x, int bc_y)
         std::string e;
         rc = fast_batch_ready(h->batch, h->stream, &dt, &e);  // autotuning, if due, runs here
         if (rc) return set_err(h, rc, "%s", e.c_str());
+    } else if (h->plain) {
+        rc = plain_ready(h);
+        if (rc) return rc;
     }
     HIPCHK(h, hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
     rc = steps();

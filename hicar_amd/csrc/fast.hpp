@@ -3,6 +3,7 @@
 #pragma once
 #include <functional>
 #include <string>
+#include <vector>
 
 #include "common.hpp"
 
@@ -55,7 +56,7 @@ int fast_batch_prepare(FastBatch *b, const float *dt, std::string *err);
 // capture.
 int fast_batch_tune(FastBatch *b, hipStream_t s, std::string *err);
 int fast_batch_ready(FastBatch *b, hipStream_t s, const float *dt, std::string *err);
-// The chosen configuration (corr_cfg 0..3) and the column chunks of the
+// The chosen configuration (corr_cfg 0..7) and the column chunks of the
 // first domain.
 void fast_batch_config(const FastBatch *b, int *corr_cfg, int *ksplit);
 
@@ -68,6 +69,20 @@ int fast_batch_advect(FastBatch *b, hipStream_t s, const float *dt, bool winds,
 // The ring conditions (bc_x 0/1/2, bc_y 0/2, as icar_adv_apply_bc) on the
 // current buffer of every species of every domain of the batch, in one launch.
 int fast_batch_bc(const FastBatch *b, hipStream_t s, int bc_x, int bc_y);
+
+// The passes of one FP32 species at a time, in place (kernel_variant 0).
+struct PlainState;
+// nullptr if its pass buffers and coefficients (14 fields; 1 at order 1) do
+// not fit in memory
+PlainState *plain_create(Dims d, int order, int fct);
+void plain_destroy(PlainState *st);
+// Sets the device tables up for these species; a no-op (and safe in a graph
+// capture) while they stay the same.
+int plain_prepare(PlainState *st, hipStream_t s, const std::vector<float *> &q, const DomainFields &f,
+                  const StepFields &sf, std::string *err);
+void plain_coef(PlainState *st, hipStream_t s);  // after the Courant numbers
+void plain_pass(PlainState *st, hipStream_t s, int species, int pass);
+float *plain_result(PlainState *st);  // where order 1 leaves its result
 
 // FP32 <-> scaled BF16/FP16 conversion.
 void launch_pack(hipStream_t s, size_t n, const float *src, void *dst, int storage, int pow2);

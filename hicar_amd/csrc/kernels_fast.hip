@@ -33,6 +33,7 @@
 #include <hip/hip_fp16.h>
 
 #include <cstdlib>
+#include <cstring>
 #include <map>
 #include <mutex>
 #include <string>
@@ -226,6 +227,7 @@ struct DomDesc {
     float *coef;          // face coefficients (float4 groups)
     unsigned *step;       // [0] steps taken (drives the stochastic rounding); [1] a coefficient
                           // is out of the bounds of the fast quotients (k_coef)
+    float *keep;                 // the donor-cell pass copies its FP32 species here (or nullptr)
     const SpecPass *pass[MAXP];  // species table of pass p at index p-1
 };
 
@@ -722,6 +724,7 @@ __global__ void __launch_bounds__(64 * FWAVES)
                     fresh();
                     const uint32_t rnd = is_sr(p[b].kindo) ? sr_bits((uint32_t)c + lane, s0 + b, tstep) : 0u;
                     stq<QK>(p[b].out, c, lane, p[b].kindo, p[b].inv_scaleo, r, rnd);
+                    if (QK == QK_F32 && D.keep) stq<QK_F32>(D.keep, c, lane, 0, 1.0f, q[b][t], 0u);
                 }
                 q[b][t] = qu[b][t];
             }
@@ -2084,6 +2087,153 @@ int fast_batch_advect(FastBatch *b, hipStream_t s, const float *dt, bool winds,
     if (b->order <= 2)  // the results landed in the other home buffers
         for (auto &dm : b->doms) dm.st->cur = 1 - dm.st->cur;
     return 0;
+}
+
+// ---------------------------------------------------------------------------
+// One species at a time (kernel_variant 0)
+// ---------------------------------------------------------------------------
+// The same kernels, a launch per pass and species, in place: the species keep
+// their buffers and share two pass buffers, a and b.
+//   order 1   q -> a (the caller copies a to q)
+//   order 2   q -> a, with q copied to b; (b, a) -> q
+//   order 3+  q -> a; (q, a) -> b; then b -> a, a -> b, ..., -> q
+struct PlainState {
+    FastState fs;        // the domain with one species, for the launch sizes
+    FastBatch b;
+    int order = 0;
+    float *coef = nullptr, *a = nullptr, *c = nullptr;
+    unsigned *d_step = nullptr;
+    DomDesc *d_desc = nullptr;  // one per species
+    SpecPass *d_tab = nullptr;  // [species][pass]
+    std::vector<float *> q;     // the species and fields the tables are for
+    DomainFields f{};
+    int cap = 0;
+};
+
+PlainState *plain_create(Dims d, int order, int fct)
+{
+    // ICAR_ADV_PASS_KERNELS=0: the kernel per subroutine and its 7 work fields
+    const char *env = getenv("ICAR_ADV_PASS_KERNELS");
+    if (env && *env && atoi(env) == 0) return nullptr;
+    PlainState *st = new PlainState();
+    st->order = order;
+    st->fs.d = d;
+    st->fs.N = (size_t)d.nx * d.ny * d.nz;
+    st->fs.sp.assign(1, {nullptr, ICAR_ADV_STORE_F32, 0});
+    st->b.order = order;
+    st->b.fct = fct;
+    st->b.total_cb = cell_blocks(d);
+    st->b.doms.resize(1);
+    st->b.doms[0].st = &st->fs;
+    for (auto &h : st->b.h_desc) h.resize(1);
+    // the tile and the column chunks: 16-row tiles where they fill the GPU
+    // several times over, else 8-row tiles in as many chunks as make about
+    // four blocks per CU
+    auto tiles = [&](int tj) { return ((d.nx + CTI - 1) / CTI) * ((d.ny + tj - 1) / tj); };
+    st->b.corr_cfg = tiles(16) >= 4096 ? 3 : 6;
+    st->b.tj = tile_rows(st->b.corr_cfg);
+    set_ksplit(&st->b, st->b.corr_cfg == 3 ? 1 : (1024 + tiles(8) / 2) / tiles(8));
+    set_first_blocks(&st->b);
+    const size_t fb = st->fs.N * sizeof(float);
+    if (hipMalloc(&st->a, fb) != hipSuccess ||
+        (order > 1 && (hipMalloc(&st->c, fb) != hipSuccess || hipMalloc(&st->coef, NCOEF * fb) != hipSuccess)) ||
+        hipMalloc(&st->d_step, 2 * sizeof(unsigned)) != hipSuccess ||
+        hipMemset(st->d_step, 0, 2 * sizeof(unsigned)) != hipSuccess) {
+        (void)hipGetLastError();  // the caller takes the kernels that need less memory
+        plain_destroy(st);
+        return nullptr;
+    }
+    return st;
+}
+
+void plain_destroy(PlainState *st)
+{
+    if (!st) return;
+    void *bufs[] = {st->coef, st->a, st->c, st->d_step, st->d_desc, st->d_tab};
+    for (void *p : bufs) (void)hipFree(p);
+    delete st;
+}
+
+float *plain_result(PlainState *st) { return st->a; }
+
+int plain_prepare(PlainState *st, hipStream_t s, const std::vector<float *> &q, const DomainFields &f,
+                  const StepFields &sf, std::string *err)
+{
+    const int n = (int)q.size(), P = st->order;
+    if (n == 0 || (q == st->q && memcmp(&f, &st->f, sizeof(f)) == 0)) return 0;
+    st->q.clear();
+    if (hipStreamSynchronize(s) != hipSuccess) {
+        *err = "a previous step failed";
+        return ICAR_ADV_EINVAL;
+    }
+    if (n > st->cap) {
+        (void)hipFree(st->d_desc);
+        (void)hipFree(st->d_tab);
+        st->d_desc = nullptr;
+        st->d_tab = nullptr;
+        st->cap = 0;
+        if (hipMalloc(&st->d_desc, n * sizeof(DomDesc)) != hipSuccess ||
+            hipMalloc(&st->d_tab, (size_t)n * P * sizeof(SpecPass)) != hipSuccess) {
+            *err = "hipMalloc of the species pass tables failed";
+            return ICAR_ADV_ENOMEM;
+        }
+        st->cap = n;
+    }
+    DomDesc D = st->b.h_desc[0][0];  // the launch sizes
+    D.d = st->fs.d;
+    D.cb0 = 0;
+    D.bx = (unsigned)((D.d.nx + 63) / 64);
+    D.tiles_x = (D.d.nx + CTI - 1) / CTI;
+    D.nspec = 1;
+    D.f = f;
+    D.sf = sf;
+    D.coef = st->coef;
+    D.step = st->d_step;
+    D.keep = P == 2 ? st->c : nullptr;
+    std::vector<DomDesc> hd(n, D);
+    std::vector<SpecPass> ht((size_t)n * P);
+    for (int k = 0; k < n; k++)
+        for (int p = 1; p <= P; p++) {
+            SpecPass e{};
+            e.kind0 = e.kindo = ICAR_ADV_STORE_F32;
+            e.scale0 = e.inv_scaleo = 1.0f;
+            float *const pass_buf[2] = {st->c, st->a};  // results of even and odd passes
+            if (p == 1) {
+                e.q0 = q[k];
+            } else if (p == 2) {
+                e.q0 = P == 2 ? st->c : q[k];
+                e.q1 = st->a;
+            } else {
+                e.q0 = pass_buf[(p - 1) & 1];
+            }
+            e.out = p == P && P > 1 ? q[k] : pass_buf[p & 1];
+            ht[(size_t)k * P + p - 1] = e;
+            hd[k].pass[p - 1] = st->d_tab + (size_t)k * P + p - 1;
+        }
+    if (hipMemcpy(st->d_tab, ht.data(), ht.size() * sizeof(SpecPass), hipMemcpyHostToDevice) != hipSuccess ||
+        hipMemcpy(st->d_desc, hd.data(), hd.size() * sizeof(DomDesc), hipMemcpyHostToDevice) != hipSuccess) {
+        *err = "upload of the species pass tables failed";
+        return ICAR_ADV_ENOMEM;
+    }
+    st->q = q;
+    st->f = f;
+    return 0;
+}
+
+namespace {
+__global__ void k_clear(unsigned *flag) { *flag = 0u; }
+}  // namespace
+
+void plain_coef(PlainState *st, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_clear, dim3(1), dim3(1), 0, s, st->d_step + 1);
+    launch_coef(&st->b, s, st->d_desc, 1);
+}
+
+void plain_pass(PlainState *st, hipStream_t s, int species, int pass)
+{
+    if (pass == 1) launch_first(&st->b, s, st->d_desc + species, 1);
+    else launch_corr(&st->b, s, st->d_desc + species, 1, pass, st->b.corr_cfg);
 }
 
 void launch_pack(hipStream_t s, size_t n, const float *src, void *dst, int storage, int pow2);

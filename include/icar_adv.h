@@ -54,8 +54,12 @@ typedef struct {
  *   rk3             &time_parameters RK3: MPDATA under RK3 does nothing
  *                   (advection_driver.f90:112-115); advect returns 0
  *   kernel_variant  no reference counterpart: 0 = one kernel per MPDATA pass
- *                   and species, 1 = fused kernels batched over all species
- *                   of the handle (about twice as fast); both keep the reference's
+ *                   and species, in place, with 14 fields of work memory
+ *                   (1 at order 1; where they do not fit, or with
+ *                   ICAR_ADV_PASS_KERNELS=0 in the environment, a kernel per
+ *                   subroutine and 7), 1 = fused kernels batched over all
+ *                   species of the handle (faster with several species);
+ *                   both keep the reference's
  *                   IEEE FP32 operation order and give bit-identical results
  *                   for FP32 storage.  MPDATA only.
  *   advection       &physics adv (options_obj.f90:470-490): 1 the standard
@@ -339,12 +343,12 @@ int icar_adv_kernel_stats(void *handle, int id, double *total_ms, long long *lau
  * the candidates on the handle's own grid and species count and keeps the
  * fastest (cached for the process by shape).  The tile is a column of 60 x 16
  * or 60 x 8 cells with a halo of 2, marched up through the levels; corr_cfg
- * bit 1 selects when a level's coefficients are loaded (0: a phase ahead),
- * bit 2 the 60 x 8 tile; bit 0 has no effect; ksplit is the number of chunks
+ * bit 2 selects the 60 x 8 tile, with two rows per wave or, with bit 0 clear,
+ * one; bit 1 has no effect; ksplit is the number of chunks
  * each column march is split into, i.e. the tile's extent in k (more blocks
  * for small grids).  The
  * environment variables ICAR_ADV_CORR_CFG (0..7) and ICAR_ADV_KSPLIT fix
- * them, ICAR_ADV_AUTOTUNE=0 keeps 1 and 1. */
+ * them, ICAR_ADV_AUTOTUNE=0 keeps 3 and 1. */
 int icar_adv_launch_config(void *handle, int *corr_cfg, int *ksplit);
 
 /* Records the nsteps loop of icar_adv_run in a HIP graph on its first call
