@@ -132,7 +132,9 @@ struct XferItem {
     char *host;
     char *dev;
     size_t bytes;
+    int species16 = -1;  // a 16-bit species: dev is the FP32 staging it is converted through
 };
+constexpr int XFER_SLOTS = 4;
 
 struct Handle {
     icar_adv_grid g{};
@@ -191,10 +193,10 @@ struct Handle {
         size_t off, n;
     };
     std::vector<SnapItem> snap_items;
-    // upload / download through pinned staging: two chunks (the DMA of one
-    // overlaps the CPU copy of the other) and their events
-    char *xfer_pin[2] = {};
-    hipEvent_t xfer_ev[2] = {};
+    // upload / download through pinned staging: a ring of slots (the DMA of one
+    // chunk overlaps the CPU copies of others) and their events
+    char *xfer_pin[XFER_SLOTS] = {};
+    hipEvent_t xfer_ev[XFER_SLOTS] = {};
     bool xfer_failed = false;  // pinned staging unavailable: the runtime's copies
     // profiling
     bool prof = false;
@@ -345,7 +347,7 @@ void free_all(Handle *h)
     if (h->snap_ready) (void)hipEventDestroy(h->snap_ready);
     if (h->snap_done) (void)hipEventDestroy(h->snap_done);
     if (h->copy_stream) (void)hipStreamDestroy(h->copy_stream);
-    for (int b = 0; b < 2; b++) {
+    for (int b = 0; b < XFER_SLOTS; b++) {
         if (h->xfer_pin[b]) (void)hipHostFree(h->xfer_pin[b]);
         if (h->xfer_ev[b]) (void)hipEventDestroy(h->xfer_ev[b]);
     }
@@ -816,11 +818,16 @@ size_t strip_table(Handle *h, const Box &b, HaloStrips *hs, bool as_source)
 }
 
 // Host transfers of at least XFER_MIN bytes go through the handle's pinned
-// staging in XFER_CHUNK pieces: the runtime stages pageable copies through
-// small buffers with one CPU thread; here the DMA of one chunk overlaps the
-// copy of the previous one by several threads.  Smaller transfers, or a
-// process where pinned memory cannot be had, use the runtime's copies.
-constexpr size_t XFER_CHUNK = 32u << 20, XFER_MIN = 8u << 20;
+// staging in chunks: the runtime stages pageable copies through small buffers
+// with one CPU thread; here the DMA of one chunk overlaps the copies of others
+// by several threads.  Smaller transfers, or a process where pinned memory
+// cannot be had, use the runtime's copies.  An array over 16 MiB is cut into
+// equal parts, since the first chunk's DMA and the last one's copy overlap
+// nothing; arrays below a sixteenth of the transfer share a chunk; others are
+// a chunk each (cutting them further costs more in calls than it overlaps).
+// Two slots of 32 MiB and a transfer per 16-bit species: 208 MB 5.5 ms, 15.7
+// MB of which 13.1 are 16-bit species 1.06 ms; now 4.0 and 0.56.
+constexpr size_t XFER_SLOT = 16u << 20, XFER_MIN = 8u << 20;
 
 // copy-pool workers besides the caller: ICAR_ADV_COPY_THREADS, default 7
 // (0: every copy on the calling thread)
@@ -871,9 +878,9 @@ bool xfer_ready(Handle *h)
 {
     if (h->xfer_failed) return false;
     if (h->xfer_pin[0]) return true;
-    for (int b = 0; b < 2; b++) {
+    for (int b = 0; b < XFER_SLOTS; b++) {
         // non-coherent: cacheable for the CPU side of the copies
-        if (hipHostMalloc((void **)&h->xfer_pin[b], XFER_CHUNK, hipHostMallocNonCoherent) !=
+        if (hipHostMalloc((void **)&h->xfer_pin[b], XFER_SLOT, hipHostMallocNonCoherent) !=
                 hipSuccess ||
             hipEventCreateWithFlags(&h->xfer_ev[b], hipEventDisableTiming) != hipSuccess) {
             (void)hipGetLastError();
@@ -884,6 +891,38 @@ bool xfer_ready(Handle *h)
     return true;
 }
 
+// A transfer cut into chunks of one slot each; a piece is the part of one
+// item in a chunk.
+struct XferPiece {
+    char *host, *dev;
+    size_t slot_off, n;
+    int convert;  // a 16-bit species that starts (download) or ends (upload) here, or -1
+};
+
+std::vector<std::vector<XferPiece>> xfer_chunks(const std::vector<XferItem> &items, bool down)
+{
+    size_t total = 0;
+    for (const auto &it : items) total += it.bytes;
+    std::vector<std::vector<XferPiece>> chunks;
+    size_t used = XFER_SLOT;  // of the last chunk
+    for (const auto &it : items) {
+        const size_t parts = (it.bytes + XFER_SLOT - 1) / XFER_SLOT;
+        const size_t part = ((it.bytes + parts - 1) / parts + 4095) / 4096 * 4096;
+        for (size_t o = 0; o < it.bytes;) {
+            const size_t n = std::min(part, it.bytes - o);
+            if (used >= total / 16 || used + n > XFER_SLOT) {
+                chunks.emplace_back();
+                used = 0;
+            }
+            const bool edge = down ? o == 0 : o + n == it.bytes;
+            chunks.back().push_back({it.host + o, it.dev + o, used, n, edge ? it.species16 : -1});
+            o += n;
+            used += n;
+        }
+    }
+    return chunks;
+}
+
 size_t xfer_bytes(const std::vector<XferItem> &items)
 {
     size_t n = 0;
@@ -891,37 +930,49 @@ size_t xfer_bytes(const std::vector<XferItem> &items)
     return n;
 }
 
+// a 16-bit species to (unpack) or from the FP32 staging, in stream order with
+// the copies of the staging
+void xfer_convert(Handle *h, int s, bool unpack)
+{
+    const SpeciesSlot &sl = h->sp[s];
+    timed(h, K_CONVERT, 6.0 * h->N, [&] {
+        if (unpack) launch_unpack(h->stream, h->N, species_dev(h, s), h->stage, sl.storage, sl.pow2);
+        else launch_pack(h->stream, h->N, h->stage, species_dev(h, s), sl.storage, sl.pow2);
+    });
+}
+
 // device -> host, in stream order after the work enqueued so far; returns
 // once the host arrays hold the data
 int xfer_down(Handle *h, const std::vector<XferItem> &items)
 {
     if (xfer_bytes(items) < XFER_MIN || !xfer_ready(h)) {
-        for (const auto &it : items)
+        for (const auto &it : items) {
+            if (it.species16 >= 0) xfer_convert(h, it.species16, true);
             HIPCHK(h, hipMemcpyAsync(it.host, it.dev, it.bytes, hipMemcpyDeviceToHost, h->stream));
+        }
+        HIPCHK(h, hipGetLastError());
         HIPCHK(h, hipStreamSynchronize(h->stream));
         return 0;
     }
-    struct Piece {
-        char *host;
-        const char *dev;
-        size_t n;
-    };
-    std::vector<Piece> ps;
-    for (const auto &it : items)
-        for (size_t o = 0; o < it.bytes; o += XFER_CHUNK)
-            ps.push_back({it.host + o, it.dev + o, std::min(XFER_CHUNK, it.bytes - o)});
-    for (size_t i = 0; i <= ps.size(); i++) {
-        if (i < ps.size()) {  // chunk i into buffer i%2 (its previous contents are copied out)
-            HIPCHK(h, hipMemcpyAsync(h->xfer_pin[i & 1], ps[i].dev, ps[i].n, hipMemcpyDeviceToHost,
-                                     h->stream));
-            HIPCHK(h, hipEventRecord(h->xfer_ev[i & 1], h->stream));
+    const auto chunks = xfer_chunks(items, true);
+    const size_t nc = chunks.size(), lag = XFER_SLOTS - 1;
+    for (size_t i = 0; i < nc + lag; i++) {
+        if (i < nc) {  // chunk i into its slot (chunk i - XFER_SLOTS is copied out)
+            const size_t b = i % XFER_SLOTS;
+            for (const XferPiece &p : chunks[i]) {
+                if (p.convert >= 0) xfer_convert(h, p.convert, true);
+                HIPCHK(h, hipMemcpyAsync(h->xfer_pin[b] + p.slot_off, p.dev, p.n, hipMemcpyDeviceToHost,
+                                         h->stream));
+            }
+            HIPCHK(h, hipEventRecord(h->xfer_ev[b], h->stream));
         }
-        if (i > 0) {  // chunk i-1 out of its buffer while chunk i moves
-            const size_t b = (i - 1) & 1;
+        if (i >= lag && i - lag < nc) {  // chunk i - lag out of its slot while later ones move
+            const size_t b = (i - lag) % XFER_SLOTS;
             HIPCHK(h, hipEventSynchronize(h->xfer_ev[b]));
-            host_copy(h, ps[i - 1].host, h->xfer_pin[b], ps[i - 1].n);
+            for (const XferPiece &p : chunks[i - lag]) host_copy(h, p.host, h->xfer_pin[b] + p.slot_off, p.n);
         }
     }
+    HIPCHK(h, hipGetLastError());
     return 0;
 }
 
@@ -931,25 +982,51 @@ int xfer_down(Handle *h, const std::vector<XferItem> &items)
 int xfer_up(Handle *h, const std::vector<XferItem> &items)
 {
     if (xfer_bytes(items) < XFER_MIN || !xfer_ready(h)) {
-        for (const auto &it : items)
+        for (const auto &it : items) {
             HIPCHK(h, hipMemcpyAsync(it.dev, it.host, it.bytes, hipMemcpyHostToDevice, h->stream));
+            if (it.species16 >= 0) xfer_convert(h, it.species16, false);
+        }
+        HIPCHK(h, hipGetLastError());
         HIPCHK(h, hipStreamSynchronize(h->stream));
         return 0;
     }
-    size_t i = 0;
-    for (const auto &it : items)
-        for (size_t o = 0; o < it.bytes; o += XFER_CHUNK, i++) {
-            const size_t b = i & 1, n = std::min(XFER_CHUNK, it.bytes - o);
-            // the buffer's last DMA has left: chunk i-2's, or for i < 2 one a
-            // previous call enqueued (complete unless that call failed part way;
-            // an event never recorded returns at once)
-            HIPCHK(h, hipEventSynchronize(h->xfer_ev[b]));
-            host_copy(h, h->xfer_pin[b], it.host + o, n);
-            HIPCHK(h, hipMemcpyAsync(it.dev + o, h->xfer_pin[b], n, hipMemcpyHostToDevice, h->stream));
-            HIPCHK(h, hipEventRecord(h->xfer_ev[b], h->stream));
+    const auto chunks = xfer_chunks(items, false);
+    for (size_t i = 0; i < chunks.size(); i++) {
+        const size_t b = i % XFER_SLOTS;
+        // the slot's last DMA has left: that of XFER_SLOTS chunks ago, or one a
+        // previous call enqueued (complete unless that call failed part way;
+        // an event never recorded returns at once)
+        HIPCHK(h, hipEventSynchronize(h->xfer_ev[b]));
+        for (const XferPiece &p : chunks[i]) {
+            host_copy(h, h->xfer_pin[b] + p.slot_off, p.host, p.n);
+            HIPCHK(h, hipMemcpyAsync(p.dev, h->xfer_pin[b] + p.slot_off, p.n, hipMemcpyHostToDevice,
+                                     h->stream));
+            if (p.convert >= 0) xfer_convert(h, p.convert, false);
         }
+        HIPCHK(h, hipEventRecord(h->xfer_ev[b], h->stream));
+    }
+    HIPCHK(h, hipGetLastError());
     HIPCHK(h, hipStreamSynchronize(h->stream));
     return 0;
+}
+
+// the arrays of a transfer mask
+std::vector<XferItem> xfer_items(Handle *h, unsigned long long mask)
+{
+    std::vector<XferItem> items;
+    for (int f = 0; f < ICAR_ADV_NFIELDS; f++) {
+        if (!(mask & ICAR_ADV_MASK_FIELD(f)) || !h->host_field[f]) continue;
+        items.push_back({(char *)h->host_field[f], (char *)h->dev_field[f],
+                         field_elems(h, f) * sizeof(float)});
+    }
+    for (int s = 0; s < h->nspecies; s++) {
+        const SpeciesSlot &sl = h->sp[s];
+        if (!(mask & ICAR_ADV_MASK_SPECIES(s)) || !sl.bound) continue;
+        const bool f32 = sl.storage == ICAR_ADV_STORE_F32;
+        items.push_back({(char *)sl.host, (char *)(f32 ? species_dev(h, s) : (void *)h->stage),
+                         h->N * sizeof(float), f32 ? -1 : s});
+    }
+    return items;
 }
 
 // Completes a pending snapshot into the host arrays.
@@ -1207,35 +1284,7 @@ int icar_adv_upload(void *handle, unsigned long long mask)
         return set_err(h, ICAR_ADV_EINVAL,
                        "a snapshot of these arrays is pending: icar_adv_snapshot_wait before "
                        "uploading them");
-    // FP32 arrays in one pipelined transfer; each 16-bit species through the
-    // FP32 staging and the pack kernel (stream order keeps the staging's uses
-    // apart)
-    std::vector<XferItem> items;
-    for (int f = 0; f < ICAR_ADV_NFIELDS; f++) {
-        if (!(mask & ICAR_ADV_MASK_FIELD(f)) || !h->host_field[f]) continue;
-        items.push_back({(char *)h->host_field[f], (char *)h->dev_field[f],
-                         field_elems(h, f) * sizeof(float)});
-    }
-    for (int s = 0; s < h->nspecies; s++) {
-        SpeciesSlot &sl = h->sp[s];
-        if (!(mask & ICAR_ADV_MASK_SPECIES(s)) || !sl.bound) continue;
-        if (sl.storage == ICAR_ADV_STORE_F32)
-            items.push_back({(char *)sl.host, (char *)species_dev(h, s), h->N * sizeof(float)});
-    }
-    rc = xfer_up(h, items);
-    if (rc) return rc;
-    for (int s = 0; s < h->nspecies; s++) {
-        SpeciesSlot &sl = h->sp[s];
-        if (!(mask & ICAR_ADV_MASK_SPECIES(s)) || !sl.bound || sl.storage == ICAR_ADV_STORE_F32)
-            continue;
-        rc = xfer_up(h, {{(char *)sl.host, (char *)h->stage, h->N * sizeof(float)}});
-        if (rc) return rc;
-        timed(h, K_CONVERT, 6.0 * h->N,
-              [&] { launch_pack(h->stream, h->N, h->stage, species_dev(h, s), sl.storage, sl.pow2); });
-    }
-    HIPCHK(h, hipGetLastError());
-    HIPCHK(h, hipStreamSynchronize(h->stream));
-    return 0;
+    return xfer_up(h, xfer_items(h, mask));
 }
 
 int icar_adv_download(void *handle, unsigned long long mask)
@@ -1247,33 +1296,7 @@ int icar_adv_download(void *handle, unsigned long long mask)
     // values of this download are the ones that stay
     rc = finish_snapshot(h);
     if (rc) return rc;
-    std::vector<XferItem> items;
-    for (int f = 0; f < ICAR_ADV_NFIELDS; f++) {
-        if (!(mask & ICAR_ADV_MASK_FIELD(f)) || !h->host_field[f]) continue;
-        items.push_back({(char *)h->host_field[f], (char *)h->dev_field[f],
-                         field_elems(h, f) * sizeof(float)});
-    }
-    for (int s = 0; s < h->nspecies; s++) {
-        SpeciesSlot &sl = h->sp[s];
-        if (!(mask & ICAR_ADV_MASK_SPECIES(s)) || !sl.bound) continue;
-        if (sl.storage == ICAR_ADV_STORE_F32)
-            items.push_back({(char *)sl.host, (char *)species_dev(h, s), h->N * sizeof(float)});
-    }
-    rc = xfer_down(h, items);
-    if (rc) return rc;
-    for (int s = 0; s < h->nspecies; s++) {
-        SpeciesSlot &sl = h->sp[s];
-        if (!(mask & ICAR_ADV_MASK_SPECIES(s)) || !sl.bound || sl.storage == ICAR_ADV_STORE_F32)
-            continue;
-        timed(h, K_CONVERT, 6.0 * h->N,
-              [&] { launch_unpack(h->stream, h->N, species_dev(h, s), h->stage, sl.storage, sl.pow2); });
-        HIPCHK(h, hipGetLastError());
-        rc = xfer_down(h, {{(char *)sl.host, (char *)h->stage, h->N * sizeof(float)}});
-        if (rc) return rc;
-    }
-    HIPCHK(h, hipGetLastError());
-    HIPCHK(h, hipStreamSynchronize(h->stream));
-    return 0;
+    return xfer_down(h, xfer_items(h, mask));
 }
 
 int icar_adv_advect(void *handle, float dt)
