@@ -906,6 +906,7 @@ std::vector<std::vector<XferPiece>> xfer_chunks(const std::vector<XferItem> &ite
     std::vector<std::vector<XferPiece>> chunks;
     size_t used = XFER_SLOT;  // of the last chunk
     for (const auto &it : items) {
+        if (it.bytes == 0) continue;
         const size_t parts = (it.bytes + XFER_SLOT - 1) / XFER_SLOT;
         const size_t part = ((it.bytes + parts - 1) / parts + 4095) / 4096 * 4096;
         for (size_t o = 0; o < it.bytes;) {

@@ -2,8 +2,9 @@
 // the order the Fortran writes it, no FMA contraction (this translation unit
 // is compiled with -ffp-contract=off) and IEEE-correct FP32 division, so an
 // FP32 step is bit-identical to a strict IEEE FP32 build of the reference.
-// These kernels are the parity baseline; the fused kernels of
-// kernels_fast.hip are checked against them and against the oracle.
+// kernel_variant 0 takes them where the fused passes' work fields
+// (kernels_fast.hip) do not fit in memory; the reductions and the ring
+// conditions serve every path.
 //
 // Reference: src/physics/adv_mpdata.f90 and adv_mpdata_FCT_core.f90.
 #include "common.hpp"

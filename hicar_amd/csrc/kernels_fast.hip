@@ -1,21 +1,21 @@
-// Fused, species-batched MPDATA path (kernel_variant 1).
+// MPDATA with fused passes: batched over species and domains (kernel_variant
+// 1), or one species at a time (0, at the end of this file).
 //
 // One advect() step of mpdata_order n (adv_mpdata.f90:352-413) becomes
 //   k_coef     species-invariant face coefficients of the pseudo-velocities
 //              (|U|(1-|U|/avg G), the cross-term wind products and the face
 //              sums of G), once per step
 //   k_first    the donor-cell pass (upwind_advection, :43-103) for every
-//              species in one launch, the Courant numbers loaded once per
-//              cell and reused across species (bit-identical to the
-//              reference order)
+//              species in one launch, the Courant numbers of a cell reused
+//              across a block's species
 //   k_corr     one launch per corrective pass (iord >= 2) for every species:
 //              antidiffusive pseudo-velocities (mpdata_fluxes, :105-252),
 //              the 1-D FCT limiter in x, y and z (flux_limiter, :254-350 and
 //              adv_mpdata_FCT_core.f90) and the donor-cell flux divergence
 //              with the limited velocities, fused in one kernel.
 // k_courant_b mpdata_compute_wind for every domain of the batch
-// k_corr marches upward through the levels of a 60 x 16 column tile (halo 2,
-// 64 x 20 columns staged in LDS); x/y neighbours come from LDS planes, the z
+// k_corr marches upward through the levels of a 60 x 16 or 60 x 8 column tile
+// (halo 2, staged in LDS); x/y neighbours come from LDS planes, the z
 // direction (including the column-wise FCT) stays in registers of the thread
 // that owns the column.  Species are independent inside advect, so a launch
 // covers (tile, species) pairs; blocks are mapped so that the species of one

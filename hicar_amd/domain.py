@@ -65,7 +65,7 @@ class Options:
     time_options: TimeOptions = field(default_factory=TimeOptions)
     # names requested for advection (options%vars_to_advect); ordered
     vars_to_advect: list = field(default_factory=list)
-    # no reference counterpart: 0 exact kernels, 1 fused/batched kernels
+    # no reference counterpart: 0 one species at a time, 1 batched over species
     kernel_variant: int = 0
 
     def advect_vars(self, names) -> None:
