@@ -347,8 +347,8 @@ void free_all(Handle *h)
     if (h->snap_ready) (void)hipEventDestroy(h->snap_ready);
     if (h->snap_done) (void)hipEventDestroy(h->snap_done);
     if (h->copy_stream) (void)hipStreamDestroy(h->copy_stream);
+    if (h->xfer_pin[0]) (void)hipHostFree(h->xfer_pin[0]);
     for (int b = 0; b < XFER_SLOTS; b++) {
-        if (h->xfer_pin[b]) (void)hipHostFree(h->xfer_pin[b]);
         if (h->xfer_ev[b]) (void)hipEventDestroy(h->xfer_ev[b]);
     }
     if (h->gexec) (void)hipGraphExecDestroy(h->gexec);
@@ -878,16 +878,19 @@ bool xfer_ready(Handle *h)
 {
     if (h->xfer_failed) return false;
     if (h->xfer_pin[0]) return true;
-    for (int b = 0; b < XFER_SLOTS; b++) {
-        // non-coherent: cacheable for the CPU side of the copies
-        if (hipHostMalloc((void **)&h->xfer_pin[b], XFER_SLOT, hipHostMallocNonCoherent) !=
-                hipSuccess ||
-            hipEventCreateWithFlags(&h->xfer_ev[b], hipEventDisableTiming) != hipSuccess) {
-            (void)hipGetLastError();
-            h->xfer_failed = true;
-            return false;
-        }
+    // one allocation for the slots; non-coherent: cacheable for the CPU side of
+    // the copies
+    char *pin = nullptr;
+    bool ok = hipHostMalloc((void **)&pin, XFER_SLOTS * XFER_SLOT, hipHostMallocNonCoherent) == hipSuccess;
+    for (int b = 0; ok && b < XFER_SLOTS; b++)
+        ok = h->xfer_ev[b] || hipEventCreateWithFlags(&h->xfer_ev[b], hipEventDisableTiming) == hipSuccess;
+    if (!ok) {
+        (void)hipGetLastError();
+        if (pin) (void)hipHostFree(pin);
+        h->xfer_failed = true;
+        return false;
     }
+    for (int b = 0; b < XFER_SLOTS; b++) h->xfer_pin[b] = pin + b * XFER_SLOT;
     return true;
 }
 
