@@ -2137,8 +2137,7 @@ PlainState *plain_create(Dims d, int order, int fct)
     const size_t fb = st->fs.N * sizeof(float);
     if (hipMalloc(&st->a, fb) != hipSuccess ||
         (order > 1 && (hipMalloc(&st->c, fb) != hipSuccess || hipMalloc(&st->coef, NCOEF * fb) != hipSuccess)) ||
-        hipMalloc(&st->d_step, 2 * sizeof(unsigned)) != hipSuccess ||
-        hipMemset(st->d_step, 0, 2 * sizeof(unsigned)) != hipSuccess) {
+        hipMalloc(&st->d_step, 2 * sizeof(unsigned)) != hipSuccess) {  // [0] unused, [1] set by plain_coef
         (void)hipGetLastError();  // the caller takes the kernels that need less memory
         plain_destroy(st);
         return nullptr;
