@@ -469,11 +469,12 @@ int plain_ready(Handle *h)
     return rc ? set_err(h, rc, "%s", e.c_str()) : 0;
 }
 
-// Every species through its passes, a launch per pass and species.
+// Every species through its passes, a launch per pass and species.  Without a
+// species there are no tables and nothing to launch after the Courant numbers.
 int advect_plain(Handle *h, bool winds)
 {
     const int rc = plain_ready(h);
-    if (rc) return rc;
+    if (rc || h->nspecies == 0) return rc;
     const int order = h->o.mpdata_order;
     const double n = cells(h);
     if (winds && order > 1)

@@ -2225,12 +2225,14 @@ __global__ void k_clear(unsigned *flag) { *flag = 0u; }
 
 void plain_coef(PlainState *st, hipStream_t s)
 {
+    if (!st->d_desc) return;  // no species was prepared: no table to read
     hipLaunchKernelGGL(k_clear, dim3(1), dim3(1), 0, s, st->d_step + 1);
     launch_coef(&st->b, s, st->d_desc, 1);
 }
 
 void plain_pass(PlainState *st, hipStream_t s, int species, int pass)
 {
+    if (species < 0 || species >= (int)st->q.size()) return;  // no table entry
     if (pass == 1) launch_first(&st->b, s, st->d_desc + species, 1);
     else launch_corr(&st->b, s, st->d_desc + species, 1, pass, st->b.corr_cfg);
 }
