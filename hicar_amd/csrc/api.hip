@@ -573,6 +573,17 @@ int advect_std(Handle *h, float dt, bool winds)
     std::vector<int> idx;
     for (int s = 0; s < h->nspecies; s++)
         if (h->sp[s].bound) idx.push_back(s);
+    // after a ring launch that clears the flag this may set
+    auto form_winds = [&] {
+        timed(h, K_STD_WIND, 14.0 * 4 * n, [&] {  // 9 inputs, 5 outputs
+            launch_std_wind(h->stream, h->d, h->g.dx, dt, h->o.advect_density, f, h->Um, h->Vm,
+                            h->Wm, h->Rj, h->Rdj, h->std_general);
+        });
+    };
+    if (winds && idx.empty()) {  // nothing to advect: the step's winds all the same
+        launch_std_ring(h->stream, g, StdBatch{}, 0, h->std_general);
+        form_winds();
+    }
     for (size_t b0 = 0; b0 < idx.size(); b0 += STD_MAX_BATCH) {
         StdBatch b{};
         b.n = (int)std::min(idx.size() - b0, (size_t)STD_MAX_BATCH);
@@ -600,15 +611,11 @@ int advect_std(Handle *h, float dt, bool winds)
         fill(0);
         outs(1);
         for (int m = 0; m < b.n; m++) b.out2[m] = rk3 ? h->std_b[idx[b0 + m]] : nullptr;
+        const bool form = winds && b0 == 0;
         timed(h, K_STD_RING, 0.0, [&] {
-            launch_std_ring(h->stream, g, b, fc ? 1 : 0,
-                            winds && b0 == 0 ? h->std_general : nullptr);
+            launch_std_ring(h->stream, g, b, fc ? 1 : 0, form ? h->std_general : nullptr);
         });
-        if (winds && b0 == 0)  // after the first ring copy, which clears the flag this may set
-            timed(h, K_STD_WIND, 14.0 * 4 * n, [&] {  // 9 inputs, 5 outputs
-                launch_std_wind(h->stream, h->d, h->g.dx, dt, h->o.advect_density, f, h->Um, h->Vm,
-                                h->Wm, h->Rj, h->Rdj, h->std_general);
-            });
+        if (form) form_winds();
         if (rk3) {  // advection_driver.f90:103-110
             fill(0);
             outs(1);

@@ -4,7 +4,7 @@ advected."""
 import numpy as np
 import pytest
 
-from hicar_amd import _lib
+from hicar_amd import _lib, synthetic
 from hicar_amd.advection import Advection, _ptr
 from test_gpu_parity import random_domain
 
@@ -47,3 +47,37 @@ def test_mpdata_without_species(oracle32, step, variant, order):
     finally:
         st.close()
     np.testing.assert_array_equal(q.view(np.uint32), ref["s0"].view(np.uint32))
+
+
+@pytest.mark.parametrize("step", ["advect", "run", "graph"])
+@pytest.mark.parametrize("h,v,fc,rk3", [(5, 3, 1, True), (1, 1, 0, False)])
+def test_std_without_species(oracle32, h, v, fc, rk3, step):
+    case = synthetic.config_std(nx=37, ny=29, nz=8, steps=1, nspecies=1, h_order=h, v_order=v,
+                                flux_corr=fc, rk3=rk3, cfl=0.4)
+    d, o = case.domain, case.options
+    name, q = next(iter(d.species.items()))
+    d.species.clear()
+    o.vars_to_advect = []
+    Um, Vm, Wm, _ = oracle32.std_compute_wind(d, case.dt, o.parameters.advect_density)
+    inner = (slice(1, -1), slice(None), slice(1, -1))
+    want = (np.abs(Um[1:-1, :, 1:-1]).max(), np.abs(Vm[1:-1, :, 1:-1]).max(),
+            np.abs(Wm / d.advection_dz.astype(np.float32))[inner].max())
+    st = Advection(d, o)
+    try:
+        if step == "advect":
+            st.advect(case.dt)
+        else:
+            st.set_graph(step == "graph")
+            for _ in range(2):
+                st.run(case.dt, 2)
+        np.testing.assert_array_equal(st.max_courant(), np.array(want, np.float64))
+        bind_late(st, d, name, q)
+        o.vars_to_advect = [name]
+        ref = {name: q.copy()}
+        for _ in range(2):
+            ref = oracle32.std_advect(d, o, 0.5 * case.dt, ref)
+        st.run(0.5 * case.dt, 2)
+        st.download()
+    finally:
+        st.close()
+    np.testing.assert_array_equal(q.view(np.uint32), ref[name].view(np.uint32))
