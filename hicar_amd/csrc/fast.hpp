@@ -45,9 +45,10 @@ struct FastDomain {
 struct FastBatch;
 FastBatch *fast_batch_create(const FastDomain *doms, int n, int order, int fct, std::string *err);
 void fast_batch_destroy(FastBatch *b);
-// Uploads the domain tables for these time steps (one per domain) if they
-// changed; fast_batch_advect calls it, graph capture calls it beforehand.
-int fast_batch_prepare(FastBatch *b, const float *dt, std::string *err);
+// Brings the domain tables to these time steps (one per domain), in order with
+// the work on s; a no-op where they hold them.  fast_batch_advect calls it,
+// graph capture calls it beforehand.
+int fast_batch_prepare(FastBatch *b, hipStream_t s, const float *dt, std::string *err);
 
 // Chooses the corrective kernel's launch configuration and column chunking
 // for this batch by timing the candidates once (the result is cached by

@@ -32,6 +32,7 @@
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
 
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <map>
@@ -402,6 +403,22 @@ __global__ void __launch_bounds__(256) k_coef(const DomDesc *__restrict__ DD, in
     for (int g = 0; g < 3; g++)
 #pragma unroll
         for (int e = 0; e < 4; e++) coef[4 * ((size_t)g * N + c) + e] = v[4 * g + e];
+}
+
+// The time steps of domains d0 .. d0 + n - 1, at both parities of the table.
+// They are set in stream order: a step that is still queued reads the ones it
+// was enqueued with.
+constexpr int DT_SET = 64;
+struct DtSet {
+    int d0, n;
+    float dt[DT_SET];
+};
+__global__ void __launch_bounds__(DT_SET) k_set_dt(DomDesc *__restrict__ DD, int nd, DtSet v)
+{
+    const int t = threadIdx.x;
+    if (t >= v.n) return;
+    DD[v.d0 + t].dt = v.dt[t];
+    DD[nd + v.d0 + t].dt = v.dt[t];
 }
 
 // one step taken by every domain of the batch (a vector store per domain)
@@ -1635,9 +1652,15 @@ void set_ksplit(FastBatch *b, int nks)
     b->dirty = true;
 }
 
-int upload_tables(FastBatch *b, std::string *err)
+// The copies are not ordered with the work on s, which may still read the
+// tables: it ends first.
+int upload_tables(FastBatch *b, hipStream_t s, std::string *err)
 {
     const size_t n = b->doms.size();
+    if (hipStreamSynchronize(s) != hipSuccess) {
+        *err = "a previous step failed";
+        return ICAR_ADV_EINVAL;
+    }
     for (int par = 0; par < 2; par++)
         if (hipMemcpy(b->d_desc + (size_t)par * n, b->h_desc[par].data(), n * sizeof(DomDesc),
                       hipMemcpyHostToDevice) != hipSuccess) {
@@ -1827,7 +1850,7 @@ int fast_batch_tune(FastBatch *b, hipStream_t s, std::string *err)
         return 0;
     }
     int rc = 0;
-    if (b->dirty && (rc = upload_tables(b, err))) {
+    if (b->dirty && (rc = upload_tables(b, s, err))) {
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);
         return rc;
@@ -1864,7 +1887,7 @@ int fast_batch_tune(FastBatch *b, hipStream_t s, std::string *err)
         for (const auto &v : seen) dup = dup || v == sig;
         if (dup) continue;
         seen.push_back(sig);
-        if ((rc = upload_tables(b, err))) break;
+        if ((rc = upload_tables(b, s, err))) break;
         const DomDesc *D = b->d_desc + (size_t)par * n;
         for (int cfg : tcfgs) {
             launch_corr(b, s, D, n, 2, cfg);  // warm-up
@@ -2029,7 +2052,7 @@ void fast_batch_destroy(FastBatch *b)
     delete b;
 }
 
-int fast_batch_prepare(FastBatch *b, const float *dt, std::string *err)
+int fast_batch_prepare(FastBatch *b, hipStream_t s, const float *dt, std::string *err)
 {
     const int n = (int)b->doms.size();
     for (int k = 0; k < n; k++)
@@ -2043,15 +2066,23 @@ int fast_batch_prepare(FastBatch *b, const float *dt, std::string *err)
     b->dts.assign(dt, dt + n);
     for (int par = 0; par < 2; par++)
         for (int k = 0; k < n; k++) b->h_desc[par][k].dt = dt[k];
-    return upload_tables(b, err);
+    if (b->dirty) return upload_tables(b, s, err);
+    for (int d0 = 0; d0 < n; d0 += DT_SET) {
+        DtSet v{};
+        v.d0 = d0;
+        v.n = std::min(n - d0, DT_SET);
+        std::copy(dt + d0, dt + d0 + v.n, v.dt);
+        hipLaunchKernelGGL(k_set_dt, dim3(1), dim3(DT_SET), 0, s, b->d_desc, n, v);
+    }
+    return 0;
 }
 
 int fast_batch_ready(FastBatch *b, hipStream_t s, const float *dt, std::string *err)
 {
-    int rc = fast_batch_prepare(b, dt, err);
+    int rc = fast_batch_prepare(b, s, dt, err);
     if (rc || b->tuned) return rc;
     if ((rc = fast_batch_tune(b, s, err))) return rc;
-    return fast_batch_prepare(b, dt, err);
+    return fast_batch_prepare(b, s, dt, err);
 }
 
 int fast_batch_advect(FastBatch *b, hipStream_t s, const float *dt, bool winds,
