@@ -1945,6 +1945,11 @@ int icar_adv_run(void *handle, float dt, int nsteps, int bc_x, int bc_y)
     const int p0 = parity(h);
     if (h->gexec && h->g_dt == dt && h->g_steps == nsteps && h->g_bcx == bc_x &&
         h->g_bcy == bc_y && h->g_par0 == p0) {
+        if (fused) {  // its kernels read dt from the table, where another call may have set its own
+            std::string e;
+            rc = fast_batch_prepare(h->batch, h->stream, &dt, &e);
+            if (rc) return set_err(h, rc, "%s", e.c_str());
+        }
         set_parity(h, h->g_par1);
         HIPCHK(h, hipGraphLaunch(h->gexec, h->stream));
         return 0;
@@ -2209,6 +2214,9 @@ int icar_adv_ensemble_run(void *ens, const float *dt, int nsteps, int bc_x, int 
                e->g_par0 == p0 && (int)e->g_dt.size() == n;
     for (int k = 0; hit && k < n; k++) hit = e->g_dt[k] == dt[k];
     if (hit) {
+        std::string m;  // the kernels read dt from the table, where another run may have set its own
+        const int rc = fast_batch_prepare(e->batch, e->stream, dt, &m);
+        if (rc) return ens_err(e, rc, "%s", m.c_str());
         ens_set_parity(e, e->g_par1);
         hipError_t x = hipGraphLaunch(e->gexec, e->stream);
         return x == hipSuccess ? 0 : ens_err(e, (int)x, "hipGraphLaunch: %s", hipGetErrorString(x));
