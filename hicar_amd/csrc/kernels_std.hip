@@ -27,6 +27,7 @@
 
 #include "common.hpp"
 #include "fdiv.hpp"
+#include "std_planes.hpp"
 
 namespace icaradv {
 
@@ -326,7 +327,6 @@ __global__ void __launch_bounds__(256)
 // the tiles in groups of GY rows, so that the species of a tile and its
 // neighbours run close together on one XCD and share its winds, divisors and
 // halos in L2 (groups of 1, 2 and 8 rows measured 1-4% slower over a step).
-constexpr int NWAVE = 8;        // waves of a block
 constexpr int NTHR = 64 * NWAVE;
 constexpr int SCOLS = 63;       // columns a stage updates (lane 63 supplies a face)
 constexpr int LCOLS = 61;       // columns the limiter updates (lanes 1..61)
@@ -420,18 +420,6 @@ __device__ __forceinline__ Place place(const Dims &d, const Region &r, int first
     return p;
 }
 
-// The planes of a field: NR levels of ROWS rows from row -RB on, columns -W..
-// 63 + E of the tile, QC words per row
-template <int W_, int E_, int RB_, int ROWS_, int NR_>
-struct Plane {
-    static constexpr int W = W_, E = E_, RB = RB_, ROWS = ROWS_, NR = NR_;
-    static constexpr int QC = 64 + W + E, SIZE = ROWS * QC, WORDS = NR * SIZE;
-    static constexpr int XH = W + E;  // columns beside a row's 64 lanes
-    static __device__ __forceinline__ int at(int r, int c) { return (r + RB) * QC + c + W; }
-    // plane of level k (k >= -NR)
-    static __device__ __forceinline__ int level(int k) { return (k + NR) % NR * SIZE; }
-};
-
 // the flux3 face under level k0 (k0 > 0) of a lane's column, from memory; o:
 // the column's cell at level k0
 template <int V>
@@ -465,8 +453,9 @@ template <int H, int V, int MODE, int RW>
 __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(6)))
     k_std_stage(StdGeom g, float t, StdBatch b, Region r)
 {
-    constexpr int HH = (H + 1) / 2, LA = (V + 1) / 2, TJ = NWAVE * RW;
-    using P = Plane<HH, HH - 1, HH, TJ + 2 * HH, V == 1 ? 2 : V>;
+    using T = StagePlanes<H, V, RW>;
+    using P = typename T::P;
+    constexpr int HH = T::HH, LA = T::LA, TJ = T::TJ;
     constexpr bool FL = MODE <= 1, DQ = MODE >= 1;
     __shared__ float sq[P::WORDS];
     __shared__ float sy[2][NWAVE + 1][64], sh[2][DQ ? NWAVE + 1 : 1][64];
@@ -682,10 +671,11 @@ template <int H, int V, int RW>
 __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(4, 4)))
     k_std_limit(StdGeom g, StdBatch b, Region r)
 {
-    constexpr int HH = (H + 1) / 2, LA = (V + 1) / 2, TJ = NWAVE * RW;
-    constexpr int LROWS = TJ - 3;  // rows written
-    using P = Plane<HH, HH - 1, HH + 1, TJ + 2 * HH - 1, V == 1 ? 2 : V>;  // rows -HH-1 .. TJ-3+HH
-    using B = Plane<1, 0, 2, TJ + 1, 2>;                                   // rows -2 .. TJ-2
+    using T = LimitPlanes<H, V, RW>;
+    using P = typename T::P;
+    using B = typename T::B;
+    constexpr int HH = T::HH, LA = T::LA, TJ = T::TJ;
+    constexpr int LROWS = T::LROWS;  // rows written
     __shared__ float sq[P::WORDS];
     __shared__ float so[B::WORDS], sd[B::WORDS];
     // y faces south of a wave's first row: upwind, flux3, wind
