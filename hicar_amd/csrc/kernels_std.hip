@@ -842,7 +842,7 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(4, 4)
                 gst(out, ca[e] + sk * (size_t)k, p.lane, v[e]);
         }
     };
-    bool below_fine = kb == 0;
+    bool below_fine = kb == 0;  // the faces under the ground are 0
 #pragma unroll 1
     for (int k = kb; k <= ke; k++) {
 #pragma unroll
@@ -902,9 +902,23 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(4, 4)
                 my[e] = hy[e] - uy[e];
                 mz[e] = hz[e] - uz[e];
             }
-            // the wave's faces of this level and of the one below are numbers
-            sfin = fine && below_fine;
-            below_fine = fine;
+            // The wave's merged faces of this level and of the one below are
+            // numbers.  Where a face has a quotient its guard says so; an
+            // upwind face (face_up: first order, next to the ground and the
+            // top) has none, and the stage state can hold NaN where the base
+            // state is finite.  The sum is not a number if one of them is not
+            // (one that overflows costs the general forms, no more).  Checked
+            // at every level this took 0.9% of a step at h5/v3.
+            bool numbers = fine;
+            if (H == 1 || V == 1 || k == 0 || k >= nz - 2) {
+                bool nan = false;
+#pragma unroll
+                for (int e = 0; e < RW; e++)
+                    nan |= __builtin_amdgcn_classf((mx[e] + my[e]) + mz[e], NOT_FINITE);
+                numbers = fine && !__any(nan);
+            }
+            sfin = numbers && below_fine;
+            below_fine = numbers;
         }
         yu[w][L] = uy[0];
         yh[w][L] = my[0];
@@ -941,8 +955,8 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(4, 4)
             const float vt = !top && fw[e] < 0.0f ? no[e] : o0;
             guarded(sfin, [&](auto F, Guard &gd) {
                 constexpr bool FD = F.value;
-                // FD: every value here is a number (the faces' guards and
-                // temp's below), so that the hardware's max and min are the
+                // FD: every value here is a number (the faces' check above, the
+                // north face's and temp's below), so that the hardware's max and min are the
                 // Fortran's but for the sign of a zero, which no result keeps
                 auto mx2 = [](float a, float b) { return FD ? hmax(a, b) : fmx(a, b); };
                 auto mn2 = [](float a, float b) { return FD ? hmin(a, b) : fmn(a, b); };
