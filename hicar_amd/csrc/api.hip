@@ -13,6 +13,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <condition_variable>
 #include <cstdarg>
@@ -145,6 +146,10 @@ struct Handle {
     float *dev_field[ICAR_ADV_NFIELDS] = {};
     StepFields sf{};
     PlainState *plain = nullptr;  // kernel_variant 0
+    // held by the calls that use plain or a run recorded over it, which another
+    // handle's call may take away (give_back_pass_buffers)
+    std::mutex plain_mu;
+    int device = 0;
     float *q2 = nullptr, *u2 = nullptr, *v2 = nullptr, *w2 = nullptr;
     float *u2l = nullptr, *v2l = nullptr, *w2l = nullptr;
     float *stage = nullptr;  // FP32 staging for reduced-precision species
@@ -283,15 +288,102 @@ bool grid_ok(const icar_adv_grid *g)
            g->dx > 0.0f;
 }
 
+// The work fields of the kernels per subroutine.
+std::array<float **, 7> exact_work(Handle *h)
+{
+    return {&h->q2, &h->u2, &h->v2, &h->w2, &h->u2l, &h->v2l, &h->w2l};
+}
+
+// The handles whose passes in place hold more memory than the kernels per
+// subroutine, which give the same results, need (14 fields against 7).  What
+// they hold beyond that is only on loan: when an allocation of the library
+// fails, they change over, one after another, until it succeeds.  So a set of
+// handles fits in a GPU's memory wherever it fits with 7.
+struct Holders {
+    std::mutex mu;  // taken before a handle's plain_mu, never after
+    std::vector<Handle *> list;
+};
+
+Holders &holders()
+{
+    static Holders x;
+    return x;
+}
+
+void drop_graph(Handle *h)
+{
+    if (!h->gexec) return;
+    (void)hipStreamSynchronize(h->stream);
+    (void)hipGraphExecDestroy(h->gexec);
+    h->gexec = nullptr;
+}
+
+// Changes one handle on the current device over, h itself if it is one of
+// them; false if there is none.  Not under a plain_mu.
+bool give_back_pass_buffers(Handle *h)
+{
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return false;
+    Holders &hd = holders();
+    std::lock_guard<std::mutex> l(hd.mu);
+    auto at = hd.list.end();
+    for (auto it = hd.list.begin(); it != hd.list.end(); ++it)
+        if ((*it)->device == dev && (at == hd.list.end() || *it == h)) at = it;
+    if (at == hd.list.end()) return false;
+    Handle *p = *at;
+    hd.list.erase(at);
+    std::lock_guard<std::mutex> lp(p->plain_mu);  // no call of p is enqueueing
+    drop_graph(p);
+    (void)hipStreamSynchronize(p->stream);
+    plain_destroy(p->plain);
+    p->plain = nullptr;
+    for (float **w : exact_work(p))  // while there is room; p's next step tries again
+        if (!*w && hipMalloc(w, p->N * sizeof(float)) != hipSuccess) *w = nullptr;
+    (void)hipGetLastError();
+    return true;
+}
+
 int dalloc(Handle *h, void **p, size_t bytes)
 {
     hipError_t e = hipMalloc(p, bytes);
+    while (e == hipErrorOutOfMemory && give_back_pass_buffers(h)) e = hipMalloc(p, bytes);
     if (e != hipSuccess) {
+        (void)hipGetLastError();  // the call returns it; no later launch has failed
         *p = nullptr;
         return set_err(h, ICAR_ADV_ENOMEM, "hipMalloc(%zu bytes) failed: %s", bytes,
                        hipGetErrorString(e));
     }
     return 0;
+}
+
+// Locks h->plain_mu (kernel_variant 0) for a call that advects, with the work
+// memory of one of the two paths in place.
+int lock_work(Handle *h, std::unique_lock<std::mutex> &l)
+{
+    if (h->is_std || h->fast) return 0;
+    l = std::unique_lock<std::mutex>(h->plain_mu);
+    if (h->plain) return 0;
+    l.unlock();
+    // h is not among the holders, so no other thread touches it
+    for (float **w : exact_work(h))
+        if (!*w) {
+            const int rc = dalloc(h, (void **)w, h->N * sizeof(float));
+            if (rc) return rc;
+        }
+    return 0;
+}
+
+// Calls make(), which returns ICAR_ADV_ENOMEM where memory is short, until it
+// has what it needs or there is none to be had.
+template <class F>
+int with_memory(Handle *h, F &&make)
+{
+    int rc;
+    while ((rc = make()) == ICAR_ADV_ENOMEM) {
+        (void)hipGetLastError();
+        if (!give_back_pass_buffers(h)) break;
+    }
+    return rc;
 }
 
 size_t field_elems(const Handle *h, int f)
@@ -319,6 +411,11 @@ DomainFields domain_fields(const Handle *h)
 void free_all(Handle *h)
 {
     if (!h) return;
+    {
+        Holders &hd = holders();
+        std::lock_guard<std::mutex> l(hd.mu);
+        hd.list.erase(std::remove(hd.list.begin(), hd.list.end(), h), hd.list.end());
+    }
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     drain_profile(h);
     for (auto e : h->event_pool) (void)hipEventDestroy(e);
@@ -502,7 +599,11 @@ int ensure_batch(Handle *h)
     FastDomain fd{h->fast, domain_fields(h), h->sf, h->g.dx, h->o.advect_density,
                   h->compensated};
     std::string e;
-    h->batch = fast_batch_create(&fd, 1, h->o.mpdata_order, h->o.mpdata_fct, &e);
+    with_memory(h, [&] {
+        int rc;
+        h->batch = fast_batch_create(&fd, 1, h->o.mpdata_order, h->o.mpdata_fct, &e, &rc);
+        return rc;
+    });
     if (!h->batch) return set_err(h, ICAR_ADV_EINVAL, "%s", e.c_str());
     return 0;
 }
@@ -739,7 +840,8 @@ int sync_fast_species(Handle *h)
     }
     fast_batch_destroy(h->batch);  // its tables point at the old buffers
     h->batch = nullptr;
-    int rc = fast_set_species(h->fast, v.data(), (int)v.size(), h->stream);
+    const int rc = with_memory(
+        h, [&] { return fast_set_species(h->fast, v.data(), (int)v.size(), h->stream); });
     if (rc) return set_err(h, rc, "%s", fast_error(h->fast));
     return 0;
 }
@@ -1135,7 +1237,9 @@ int icar_adv_create(const icar_adv_grid *grid, const icar_adv_opts *opts, void *
     h->Nu = (size_t)(h->d.nx + 1) * h->d.nz * h->d.ny;
     h->Nv = (size_t)h->d.nx * h->d.nz * (h->d.ny + 1);
     hipError_t e = hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking);
+    if (e == hipSuccess) e = hipGetDevice(&h->device);
     if (e != hipSuccess) {
+        if (h->stream) (void)hipStreamDestroy(h->stream);
         delete h;
         return set_err(nullptr, (int)e, "hipStreamCreate failed: %s", hipGetErrorString(e));
     }
@@ -1162,17 +1266,22 @@ int icar_adv_create(const icar_adv_grid *grid, const icar_adv_opts *opts, void *
             }
     } else if (h->o.kernel_variant == 0 && !h->o.rk3 && h->o.mpdata_order >= 1 &&
                (h->plain = plain_create(h->d, h->o.mpdata_order, h->o.mpdata_fct))) {
-        // the passes one species at a time
+        // the passes one species at a time; at order 1 they need less than the
+        // kernels per subroutine
+        if (h->o.mpdata_order > 1) {
+            Holders &hd = holders();
+            std::lock_guard<std::mutex> l(hd.mu);
+            hd.list.push_back(h);
+        }
     } else if (h->o.kernel_variant == 0) {
-        float **work[] = {&h->q2, &h->u2, &h->v2, &h->w2, &h->u2l, &h->v2l, &h->w2l};
-        for (float **p : work)
+        for (float **p : exact_work(h))
             if (dalloc(h, (void **)p, fb)) {
                 std::string m = h->err;
                 free_all(h);
                 return set_err(nullptr, ICAR_ADV_ENOMEM, "%s", m.c_str());
             }
     } else {
-        h->fast = fast_create(h->d);
+        with_memory(h, [&] { return (h->fast = fast_create(h->d)) ? 0 : ICAR_ADV_ENOMEM; });
         if (!h->fast) {
             free_all(h);
             return set_err(nullptr, ICAR_ADV_ENOMEM, "fused-path state allocation failed");
@@ -1248,10 +1357,9 @@ int icar_adv_bind_species(void *handle, int idx, float *host, int storage, int p
     const size_t elem = storage == ICAR_ADV_STORE_F32 ? 4 : 2;
     // a recorded run holds the old buffers and species list: record anew
     h->bind_gen++;
-    if (h->gexec) {
-        (void)hipStreamSynchronize(h->stream);
-        (void)hipGraphExecDestroy(h->gexec);
-        h->gexec = nullptr;
+    {
+        std::lock_guard<std::mutex> l(h->plain_mu);
+        drop_graph(h);
     }
     if (s.dev && s.storage != storage) {
         (void)hipFree(s.dev);
@@ -1315,6 +1423,9 @@ int icar_adv_advect(void *handle, float dt)
 {
     Handle *h;
     int rc = check_handle(handle, &h);
+    if (rc) return rc;
+    std::unique_lock<std::mutex> l;
+    rc = lock_work(h, l);
     if (rc) return rc;
     return do_advect(h, dt);
 }
@@ -1393,11 +1504,7 @@ int icar_adv_set_compensation(void *handle, int on)
     // the batch's tables and a recorded run hold the old setting; ensembles
     // built over this handle refuse to run, as after a binding
     h->bind_gen++;
-    if (h->gexec) {
-        (void)hipStreamSynchronize(h->stream);
-        (void)hipGraphExecDestroy(h->gexec);
-        h->gexec = nullptr;
-    }
+    drop_graph(h);
     fast_batch_destroy(h->batch);
     h->batch = nullptr;
     return 0;
@@ -1925,6 +2032,9 @@ int icar_adv_run(void *handle, float dt, int nsteps, int bc_x, int bc_y)
                        h->o.mpdata_order >= 1;
     if (bc_x < 0 || bc_x > 2 || (bc_y != 0 && bc_y != 2))
         return set_err(h, ICAR_ADV_EINVAL, "bc_x must be 0/1/2 and bc_y 0/2");
+    std::unique_lock<std::mutex> l;
+    rc = lock_work(h, l);
+    if (rc) return rc;
     auto steps = [&]() -> int {
         for (int s = 0; s < nsteps; s++) {
             int r = do_advect(h, dt, s == 0);
@@ -2174,7 +2284,12 @@ int icar_adv_ensemble_create(int n, void *const *handles, void **ens)
                         h->compensated});
     }
     std::string m;
-    e->batch = fast_batch_create(doms.data(), n, e->hs[0]->o.mpdata_order, e->hs[0]->o.mpdata_fct, &m);
+    with_memory(e->hs[0], [&] {
+        int rc;
+        e->batch = fast_batch_create(doms.data(), n, e->hs[0]->o.mpdata_order, e->hs[0]->o.mpdata_fct,
+                                     &m, &rc);
+        return rc;
+    });
     if (!e->batch) {
         ens_free(e);
         return ens_err(nullptr, ICAR_ADV_EINVAL, "%s", m.c_str());

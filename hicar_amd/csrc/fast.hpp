@@ -43,7 +43,10 @@ struct FastDomain {
     int compensated;  // the flux divergence with compensated sums (icar_adv_set_compensation)
 };
 struct FastBatch;
-FastBatch *fast_batch_create(const FastDomain *doms, int n, int order, int fct, std::string *err);
+// nullptr on failure, with the message and the error code (ICAR_ADV_ENOMEM or
+// ICAR_ADV_EINVAL; 0 on success)
+FastBatch *fast_batch_create(const FastDomain *doms, int n, int order, int fct, std::string *err,
+                             int *code);
 void fast_batch_destroy(FastBatch *b);
 // Brings the domain tables to these time steps (one per domain), in order with
 // the work on s; a no-op where they hold them.  fast_batch_advect calls it,

@@ -1931,8 +1931,10 @@ void fast_batch_config(const FastBatch *b, int *corr_cfg, int *ksplit)
     if (ksplit) *ksplit = b ? b->h_desc[0][0].nks : -1;
 }
 
-FastBatch *fast_batch_create(const FastDomain *doms, int n, int order, int fct, std::string *err)
+FastBatch *fast_batch_create(const FastDomain *doms, int n, int order, int fct, std::string *err,
+                             int *code)
 {
+    *code = ICAR_ADV_EINVAL;
     if (n < 1 || order < 1 || order > MAXP) {
         *err = "a batch needs at least one domain and 1 <= mpdata_order <= 16";
         return nullptr;
@@ -1964,11 +1966,12 @@ FastBatch *fast_batch_create(const FastDomain *doms, int n, int order, int fct, 
             delete b;
             return nullptr;
         }
-        if (st->tab_order != order && build_tables(st, order)) {
+        if (st->tab_order != order && (*code = build_tables(st, order))) {
             *err = st->err;
             delete b;
             return nullptr;
         }
+        *code = ICAR_ADV_EINVAL;
         b->gens.push_back(st->gen);
         const Dims &d = st->d;
         const int S = (int)st->sp.size();
@@ -2005,6 +2008,7 @@ FastBatch *fast_batch_create(const FastDomain *doms, int n, int order, int fct, 
     b->total_cb = cb;
     set_first_blocks(b);
     set_ksplit(b, b->nks);
+    *code = ICAR_ADV_ENOMEM;
     if (hipMalloc(&b->d_desc, 2 * (size_t)n * sizeof(DomDesc)) != hipSuccess) {
         *err = "hipMalloc of the domain table failed";
         fast_batch_destroy(b);
@@ -2030,6 +2034,7 @@ FastBatch *fast_batch_create(const FastDomain *doms, int n, int order, int fct, 
             return nullptr;
         }
     }
+    *code = 0;
     return b;
 }
 
@@ -2138,7 +2143,6 @@ struct PlainState {
     SpecPass *d_tab = nullptr;  // [species][pass]
     std::vector<float *> q;     // the species and fields the tables are for
     DomainFields f{};
-    int cap = 0;
 };
 
 PlainState *plain_create(Dims d, int order, int fct)
@@ -2165,9 +2169,12 @@ PlainState *plain_create(Dims d, int order, int fct)
     st->b.tj = tile_rows(st->b.corr_cfg);
     set_ksplit(&st->b, st->b.corr_cfg == 3 ? 1 : (1024 + tiles(8) / 2) / tiles(8));
     set_first_blocks(&st->b);
-    const size_t fb = st->fs.N * sizeof(float);
+    // the tables of as many species as there can be, so that no step allocates
+    const size_t fb = st->fs.N * sizeof(float), ns = ICAR_ADV_MAX_SPECIES;
     if (hipMalloc(&st->a, fb) != hipSuccess ||
         (order > 1 && (hipMalloc(&st->c, fb) != hipSuccess || hipMalloc(&st->coef, NCOEF * fb) != hipSuccess)) ||
+        hipMalloc(&st->d_desc, ns * sizeof(DomDesc)) != hipSuccess ||
+        hipMalloc(&st->d_tab, ns * (size_t)order * sizeof(SpecPass)) != hipSuccess ||
         hipMalloc(&st->d_step, 2 * sizeof(unsigned)) != hipSuccess) {  // [0] unused, [1] set by plain_coef
         (void)hipGetLastError();  // the caller takes the kernels that need less memory
         plain_destroy(st);
@@ -2196,18 +2203,9 @@ int plain_prepare(PlainState *st, hipStream_t s, const std::vector<float *> &q, 
         *err = "a previous step failed";
         return ICAR_ADV_EINVAL;
     }
-    if (n > st->cap) {
-        (void)hipFree(st->d_desc);
-        (void)hipFree(st->d_tab);
-        st->d_desc = nullptr;
-        st->d_tab = nullptr;
-        st->cap = 0;
-        if (hipMalloc(&st->d_desc, n * sizeof(DomDesc)) != hipSuccess ||
-            hipMalloc(&st->d_tab, (size_t)n * P * sizeof(SpecPass)) != hipSuccess) {
-            *err = "hipMalloc of the species pass tables failed";
-            return ICAR_ADV_ENOMEM;
-        }
-        st->cap = n;
+    if (n > ICAR_ADV_MAX_SPECIES) {
+        *err = "more species than the pass tables hold";
+        return ICAR_ADV_ERANGE;
     }
     DomDesc D = st->b.h_desc[0][0];  // the launch sizes
     D.d = st->fs.d;
@@ -2256,7 +2254,7 @@ __global__ void k_clear(unsigned *flag) { *flag = 0u; }
 
 void plain_coef(PlainState *st, hipStream_t s)
 {
-    if (!st->d_desc) return;  // no species was prepared: no table to read
+    if (st->q.empty()) return;  // no species was prepared: no table to read
     hipLaunchKernelGGL(k_clear, dim3(1), dim3(1), 0, s, st->d_step + 1);
     launch_coef(&st->b, s, st->d_desc, 1);
 }

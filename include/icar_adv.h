@@ -55,11 +55,12 @@ typedef struct {
  *                   (advection_driver.f90:112-115); advect returns 0
  *   kernel_variant  no reference counterpart: 0 = one kernel per MPDATA pass
  *                   and species, in place, with 14 fields of work memory
- *                   (1 at order 1; where they do not fit, or with
- *                   ICAR_ADV_PASS_KERNELS=0 in the environment, a kernel per
- *                   subroutine and 7), 1 = fused kernels batched over all
- *                   species of the handle (faster with several species);
- *                   both keep the reference's
+ *                   (1 at order 1).  Where they do not fit, when the handle
+ *                   is created or when a later allocation of any handle on
+ *                   the GPU fails, and with ICAR_ADV_PASS_KERNELS=0 in the
+ *                   environment: a kernel per subroutine and 7 fields.
+ *                   1 = fused kernels batched over all species of the handle
+ *                   (faster with several species).  All keep the reference's
  *                   IEEE FP32 operation order and give bit-identical results
  *                   for FP32 storage.  MPDATA only.
  *   advection       &physics adv (options_obj.f90:470-490): 1 the standard
