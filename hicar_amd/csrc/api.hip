@@ -1361,17 +1361,27 @@ int icar_adv_bind_species(void *handle, int idx, float *host, int storage, int p
         std::lock_guard<std::mutex> l(h->plain_mu);
         drop_graph(h);
     }
+    // a species without its buffers is not bound; the others stay as they were
+    auto failed = [&](int code) {
+        const std::string msg = h->err;
+        s.bound = false;
+        (void)hipFree(s.dev);
+        s.dev = nullptr;
+        if (h->fast) (void)sync_fast_species(h);
+        h->err = msg;
+        return code;
+    };
     if (s.dev && s.storage != storage) {
         (void)hipFree(s.dev);
         s.dev = nullptr;
     }
     if (!s.dev) {
         rc = dalloc(h, &s.dev, h->N * elem + 64);  // the fused kernels read 16-bit data in aligned pairs
-        if (rc) return rc;
+        if (rc) return failed(rc);
     }
     if (storage != ICAR_ADV_STORE_F32 && !h->stage) {
         rc = dalloc(h, (void **)&h->stage, h->N * sizeof(float));
-        if (rc) return rc;
+        if (rc) return failed(rc);
     }
     if (h->is_std) {  // next-state buffer, second RK3 stage, limiter work arrays
         void **per[] = {(void **)&h->std_alt[idx], (void **)&h->std_b[idx],
@@ -1380,7 +1390,7 @@ int icar_adv_bind_species(void *handle, int idx, float *host, int storage, int p
         for (int q = 0; q < 3; q++)
             if (need[q] && !*per[q]) {
                 rc = dalloc(h, per[q], h->N * sizeof(float) + 64);
-                if (rc) return rc;
+                if (rc) return failed(rc);
             }
     }
     s.host = host;
@@ -1388,7 +1398,7 @@ int icar_adv_bind_species(void *handle, int idx, float *host, int storage, int p
     s.pow2 = storage == ICAR_ADV_STORE_F32 ? 0 : pow2_exp;
     s.bound = true;
     if (idx + 1 > h->nspecies) h->nspecies = idx + 1;
-    if (h->fast) return sync_fast_species(h);
+    if (h->fast && (rc = sync_fast_species(h))) return failed(rc);
     return 0;
 }
 

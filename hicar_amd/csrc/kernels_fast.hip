@@ -1966,6 +1966,13 @@ FastBatch *fast_batch_create(const FastDomain *doms, int n, int order, int fct, 
             delete b;
             return nullptr;
         }
+        // (a failed allocation leaves them out)
+        if (std::count(st->alt.begin(), st->alt.end(), nullptr) > 0) {
+            *code = ICAR_ADV_ENOMEM;
+            *err = "a domain of the batch has a species without its second buffer";
+            delete b;
+            return nullptr;
+        }
         if (st->tab_order != order && (*code = build_tables(st, order))) {
             *err = st->err;
             delete b;

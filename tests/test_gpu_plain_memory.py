@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 from hicar_amd import _lib
-from hicar_amd.advection import Advection
+from hicar_amd.advection import Advection, _ptr
 from test_gpu_parity import random_domain
 from test_zz_no_alloc import Hip
 
@@ -173,3 +173,30 @@ def test_what_does_not_fit_with_seven_is_refused(oracle32, filler):
         assert passes_in_place(st)
     finally:
         st.close()
+
+
+# A new FP32 species finds room for its buffer, not for the second one that the
+# fused path keeps; one bound again in 16 bits finds room for its buffer (half a
+# field), not for the field it is converted through.
+@pytest.mark.parametrize("nspec,storage,room", [(1, _lib.STORE_F32, 1.5), (2, _lib.STORE_F16, 0.3)])
+def test_a_species_that_does_not_fit_is_not_bound(oracle32, filler, nspec, storage, room):
+    case = domain(17, nspec)
+    d, o = case.domain, case.options
+    o.kernel_variant = 1
+    late = np.ones_like(d.species["s0"])
+    keep = {n: a.copy() for n, a in d.species.items()}
+    ref = oracle32.run(d, o, 20.0, 2, 1, 2, {"s0": keep["s0"]})
+    st = Advection(d, o)
+    try:
+        filler.leave(room)
+        with pytest.raises(_lib.IcarAdvError) as e:
+            st._check(st.lib.icar_adv_bind_species(st.h, 1, _ptr(late), storage, 0))
+        assert e.value.code == _lib.ENOMEM
+        st.run(20.0, 2, 1, 2)
+        st.download()
+    finally:
+        st.close()
+    assert_bits(d, ref)
+    assert np.all(late == 1)
+    if nspec == 2:
+        np.testing.assert_array_equal(d.species["s1"], keep["s1"])
