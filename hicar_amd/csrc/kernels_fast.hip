@@ -1363,14 +1363,19 @@ __global__ void __launch_bounds__((Tile<TJ, RW>::CNT))
             for (int t = 0; t < RW; t++) {
                 const int gj = gj0 + t;
                 float q = qc[CX * t];
+                // the top flux is the value times a velocity of 0 (:96-97): a zero of
+                // its sign, and NaN for what is not finite.  Selected here for
+                // every level; a branch at the top cost 1.2% of a run of 256 x
+                // 64 x 20, one species (562 -> 569 us), this nothing
+                const float fzt = L2 == nz - 1 ? q * 0.0f : Fzc[t];
                 if (gj > 0 && gj < ny - 1) {  // the ring keeps its values
                     float v;
                     if (D.compensated) {
-                        v = divergence_compensated(q, Fxl[t], Fxr[t], Fy[t], Fy[t + 1], Fzc[t], Fzp[t],
+                        v = divergence_compensated(q, Fxl[t], Fxr[t], Fy[t], Fy[t + 1], fzt, Fzp[t],
                                                    kg[t], kgz[t]);
                     } else {
                         v = q - ((Fxr[t] - Fxl[t]) + (Fy[t + 1] - Fy[t])) / kg[t];
-                        v = v - (Fzc[t] - Fzp[t]) / kgz[t];
+                        v = v - (fzt - Fzp[t]) / kgz[t];
                     }
                     q = at_w || at_e ? q : v;
                 }
