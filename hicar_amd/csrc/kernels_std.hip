@@ -443,8 +443,8 @@ __device__ __forceinline__ float face_under(float w, const float *q, size_t o, u
 // One barrier per level: iteration k reads plane k (x, y) and its own columns
 // of the ring (z), stages level k + LA into the slot of the lowest level only
 // its own columns read, and passes the y faces through a buffer per parity.
-// Measured on 1024 x 1024 x 30, 10 species, h5/v3: mode 0 1.62 ms (6.9 GB,
-// 4.3 TB/s: near the rate of a copy), mode 1 1.94 ms (6.2 GB; waiting for
+// Measured on 1024 x 1024 x 30, 10 species, h5/v3: mode 0 1.62 ms (7.1 GB,
+// 4.4 TB/s: near the rate of a copy), mode 1 1.94 ms (6.4 GB; waiting for
 // memory and barriers half of the time), against 1.93 and 2.29 ms for one-row
 // waves over 7-row tiles whose quotients took the IEEE sequence.  Six waves
 // per SIMD: 80 registers hold mode 1 with a few values in scratch; five waves
@@ -661,7 +661,7 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(6)))
 // rows 0..LROWS-1; the last row supplies its south face only).  Two barriers
 // per level.  Bound by VALU issue and the waits at the barriers, with two
 // blocks of eight waves per CU; what a level carries to the next is kept small
-// (113 registers at h5/v3: the state after the horizontal update instead of
+// (111 registers at h5/v3: the state after the horizontal update instead of
 // its parts, one register for the one halo row a wave stages) because spilling
 // it took 4.7 ms and keeping it in three-row slots 9.3.  1024 x 1024 x 30, 10
 // species, h5/v3: 4.1 ms, against 6.4 ms for two marches that each computed
