@@ -2150,7 +2150,7 @@ struct PlainState {
     FastBatch b;
     int order = 0;
     float *coef = nullptr, *a = nullptr, *c = nullptr;
-    unsigned *d_step = nullptr;
+    unsigned *d_step = nullptr; // the tables' allocation: two flags, then
     DomDesc *d_desc = nullptr;  // one per species
     SpecPass *d_tab = nullptr;  // [species][pass]
     std::vector<float *> q;     // the species and fields the tables are for
@@ -2182,23 +2182,27 @@ PlainState *plain_create(Dims d, int order, int fct)
     set_ksplit(&st->b, st->b.corr_cfg == 3 ? 1 : (1024 + tiles(8) / 2) / tiles(8));
     set_first_blocks(&st->b);
     // the tables of as many species as there can be, so that no step allocates
-    const size_t fb = st->fs.N * sizeof(float), ns = ICAR_ADV_MAX_SPECIES;
+    constexpr size_t NS = ICAR_ADV_MAX_SPECIES, FLAGS = 256;  // [0] unused, [1] set by plain_coef
+    static_assert(NS * sizeof(DomDesc) % alignof(SpecPass) == 0, "the pass table follows");
+    const size_t fb = st->fs.N * sizeof(float);
+    char *tables = nullptr;
     if (hipMalloc(&st->a, fb) != hipSuccess ||
         (order > 1 && (hipMalloc(&st->c, fb) != hipSuccess || hipMalloc(&st->coef, NCOEF * fb) != hipSuccess)) ||
-        hipMalloc(&st->d_desc, ns * sizeof(DomDesc)) != hipSuccess ||
-        hipMalloc(&st->d_tab, ns * (size_t)order * sizeof(SpecPass)) != hipSuccess ||
-        hipMalloc(&st->d_step, 2 * sizeof(unsigned)) != hipSuccess) {  // [0] unused, [1] set by plain_coef
+        hipMalloc(&tables, FLAGS + NS * (sizeof(DomDesc) + (size_t)order * sizeof(SpecPass))) != hipSuccess) {
         (void)hipGetLastError();  // the caller takes the kernels that need less memory
         plain_destroy(st);
         return nullptr;
     }
+    st->d_step = (unsigned *)tables;
+    st->d_desc = (DomDesc *)(tables + FLAGS);
+    st->d_tab = (SpecPass *)(st->d_desc + NS);
     return st;
 }
 
 void plain_destroy(PlainState *st)
 {
     if (!st) return;
-    void *bufs[] = {st->coef, st->a, st->c, st->d_step, st->d_desc, st->d_tab};
+    void *bufs[] = {st->coef, st->a, st->c, st->d_step};
     for (void *p : bufs) (void)hipFree(p);
     delete st;
 }
