@@ -162,7 +162,9 @@ int icar_adv_bind_field(void *handle, int field_id, float *host, const int lb[3]
 /* Registers advected species idx (0-based position in domain%adv_vars,
  * domain_obj.f90:68-89) with its host array (mass-grid bounds of the
  * domain).  storage selects the device format; pow2_exp is the per-species
- * power-of-two scale e: the device holds q * 2^-e (ignored for FP32). */
+ * power-of-two scale e: the device holds q * 2^-e (ignored for FP32).  Where
+ * the buffers cannot be allocated (ICAR_ADV_ENOMEM) the species is not bound,
+ * also if it was; the others keep their values. */
 int icar_adv_bind_species(void *handle, int idx, float *host, int storage, int pow2_exp);
 
 /* Copies the selected host arrays to the device (after CPU physics touched
